@@ -1,0 +1,1103 @@
+// Matrix products over several activation rows (prompts, short turns, the
+// rows of an expert) with quantized weights: out[M, N] = x[M, K] . W[N, K]^T
+// for Q4_0, Q4_0F and Q2_K, M >= 2, on the f16 matrix cores
+// (v_mfma_f32_16x16x32_f16) with fp32 sums.
+//
+// Two launches.  x_split_kernel (with the RMSNorm / LayerNorm prologue, or a
+// row gather, fused in) writes every row once as two f16 parts in matrix-core
+// fragment order; rows_gemm_kernel multiplies.
+//
+// Precision.  A row is scaled by a power of two so that its largest magnitude
+// lies in [2^13, 2^14), then split x = h + l, h = f16(x), l = f16(x - h):
+// 22 significant bits at least (the split drops at most the last of the 24,
+// for one value in four), products with the small weight integers are exact
+// in the matrix core's fp32, sums are fp32.  The row scale comes out again in
+// the epilogue, exactly.  inf and NaN stay themselves in h (l = 0), so Q4 rows
+// that hold them give what fp32 products give; Q2_K rows give NaN (the minima
+// are a second product).  Against 64-bit
+// products the result is as close as with an exact three-part bf16 split and
+// one serial K loop (M 512, K 2048 / 8192: see the launch rules below), since
+// the K dimension is summed in up to eight independent slices.
+//
+// Weights.  Q4: q - 7 is exact in f16, one fp32 fma per output and 32-value
+// block applies the block scale.  Q2_K: sc * q <= 45 is exact in f16; d is
+// applied per 128-value page (per 32-value slice where rows do not start at
+// pages); the minima are a second, 16 times shorter contraction
+// -(dmin m) . X16 over the sums X16 of each 16 values of x: bf16 parts, two
+// of dmin m (exact: 15 bits) and three of X16 (exact).
+//
+// Structure.  A wave owns 16 MI rows x 16 NJ columns (per matrix) over its
+// share of K and reads its operands straight into registers: A fragments as
+// contiguous 1 KiB loads, weights as whole blocks (a lane loads one Q4 block,
+// v_permlane16/32_swap transposes the four blocks of a 128-value step across
+// the wave's four lane rows).  No LDS and no barrier in the K loop, so the
+// waves of a workgroup (NW across columns, KW along K, interleaved by 128
+// values) never wait for each other; the KW partial tiles meet in LDS once
+// at the end.
+#include "rina_common.hpp"
+#include "rows_gemm.hpp"
+
+namespace {
+
+typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
+typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef float f32x16 __attribute__((ext_vector_type(16)));
+
+enum { FMT_Q4_0 = 0, FMT_Q4_0F = 1, FMT_Q2_K = 2, FMT_Q2_S = 3 };   // Q2_S: Q2_K rows that start inside a page
+
+// 16- and 8-byte loads at 4-byte alignment (weight blocks)
+__device__ __forceinline__ u32x4 gld4(const uint8_t* p) {
+    typedef u32x4 __attribute__((aligned(4))) T;
+    return *(const __attribute__((address_space(1))) T*)p;
+}
+__device__ __forceinline__ u32x2 gld2(const uint8_t* p) {
+    typedef u32x2 __attribute__((aligned(4))) T;
+    return *(const __attribute__((address_space(1))) T*)p;
+}
+
+__device__ __forceinline__ float silu_mul(float g, float u) { return g / (1.0f + expf(-g)) * u; }
+
+// ---------------------------------------------------------------------------
+// activation rows -> f16 fragments
+// ---------------------------------------------------------------------------
+// Layout: 16-row tile mt, 32-value step ks, part p (0: h, 1: l), 64 lanes of
+// 16 bytes; lane (r, f) holds row 16 mt + r, values 32 ks + 8 f .. + 7 in the
+// order in which the weight bytes unpack: Q4 dword j = values (j, j + 4);
+// Q2_K dwords = values (0, 2), (1, 3), (4, 6), (5, 7).  Q2_K also gets the
+// sums of 16 values as three bf16 parts: 16-row tile, window of 32 sums,
+// part, lane (r, f) = sums 8 f .. + 7 of row r.  K is padded with zeros to
+// whole 128-value steps (and windows), rows to whole tiles.
+struct SplitXArgs {
+    const float* x;
+    const float* nw;
+    const int* src;        // row gather: packed row r is x row src[r] (< 0: zero row)
+    uint4* xp;
+    float* xs;             // [rows] 2^-e of the row scale 2^e
+    uint16_t* xg;          // Q2_K: group-sum fragments
+    int M, K, nks, ngw;
+    int pro;
+    float eps;
+};
+
+// A workgroup takes 4 rows, 256 threads each: the four rows' 16-byte stores of
+// one fragment make 64 contiguous bytes, and every load of a row is in flight
+// at once.  NU: 8-value units per thread held in registers between the
+// statistics and the split (rows of up to 2048 NU values); 0: longer rows, the
+// units read again.  One wave per row (16 rows per workgroup, the units in a
+// loop) took 12.4 us at 512 x 2048 and 35 us at 512 x 8192.
+constexpr int kSplitRows = 4;
+
+template <bool Q2, int NU>
+__global__ __launch_bounds__(256 * kSplitRows) void x_split_kernel(SplitXArgs a) {
+    __shared__ float s_red[3][kSplitRows][4];
+    const int r = threadIdx.x >> 8, tid = threadIdx.x & 255, wave = tid >> 6, lane = tid & 63;
+    const int row = blockIdx.x * kSplitRows + r, mt = row >> 4;
+    int srow = row < a.M ? row : -1;
+    if (a.src) srow = __builtin_amdgcn_readfirstlane(gld(a.src + row));
+    const int nu = a.K >> 3, nup = a.nks * 4;      // 8-value units, padded
+    const float* xr = a.x + (int64_t)(srow < 0 ? 0 : srow) * a.K;
+    const f32x4 z4{0.f, 0.f, 0.f, 0.f};
+    // 8 values at p: element loads where they are not 16-byte aligned
+    auto load8 = [&](const float* p, f32x4& lo, f32x4& hi) {
+        if (((uintptr_t)p & 15) == 0) {
+            lo = gld((const f32x4*)p);
+            hi = gld((const f32x4*)(p + 4));
+        } else {
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                lo[i] = gld(p + i);
+                hi[i] = gld(p + 4 + i);
+            }
+        }
+    };
+    f32x4 v[NU ? NU : 1][2];
+    if (NU > 0) {
+#pragma unroll
+        for (int i = 0; i < NU; i++) {
+            v[i][0] = v[i][1] = z4;
+            if (srow >= 0 && tid + 256 * i < nu) load8(xr + 8 * (tid + 256 * i), v[i][0], v[i][1]);
+        }
+    }
+    auto each = [&](auto&& f) {                     // f(unit, low half, high half) over the row
+        if (NU > 0) {
+#pragma unroll
+            for (int i = 0; i < (NU ? NU : 1); i++)
+                if (tid + 256 * i < nup) f(tid + 256 * i, v[i][0], v[i][1]);
+        } else {
+            for (int u = tid; u < nup; u += 256) {
+                f32x4 p = z4, q = z4;
+                if (srow >= 0 && u < nu) load8(xr + 8 * u, p, q);
+                f(u, p, q);
+            }
+        }
+    };
+    // a row's sum / maximum over its four waves, each in its own slot
+    auto row_sum = [&](float x, int k) {
+        x = wave_sum(x);
+        if (lane == 0) s_red[k][r][wave] = x;
+        __syncthreads();
+        return (s_red[k][r][0] + s_red[k][r][1]) + (s_red[k][r][2] + s_red[k][r][3]);
+    };
+    // the norm of rina_hip_rms_norm / rina_hip_layer_norm, applied to a unit
+    float mean = 0.f, inv = 1.f;
+    if (a.pro == RINA_PRO_LAYERNORM) {
+        float s = 0.f;
+        each([&](int, const f32x4& p, const f32x4& q) {
+#pragma unroll
+            for (int i = 0; i < 4; i++) s += p[i] + q[i];
+        });
+        mean = row_sum(s, 0) / (float)a.K;
+    }
+    if (a.pro != RINA_PRO_NONE) {
+        float ss = 0.f;
+        each([&](int u, const f32x4& p, const f32x4& q) {
+            if (u >= nu) return;
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                ss = fmaf(p[i] - mean, p[i] - mean, ss);
+                ss = fmaf(q[i] - mean, q[i] - mean, ss);
+            }
+        });
+        inv = 1.0f / sqrtf(row_sum(ss, 1) / (float)a.K + a.eps);
+    }
+    auto normed = [&](int u, f32x4& p, f32x4& q) {
+        if (a.pro == RINA_PRO_NONE) return;
+        f32x4 g, h;
+        load8(a.nw + 8 * (u < nu ? u : 0), g, h);
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            p[i] = u < nu ? (p[i] - mean) * inv * g[i] : 0.f;
+            q[i] = u < nu ? (q[i] - mean) * inv * h[i] : 0.f;
+        }
+    };
+    if (NU > 0) {
+#pragma unroll
+        for (int i = 0; i < NU; i++) normed(tid + 256 * i, v[i][0], v[i][1]);
+    }
+    float mx = 0.f;                                 // largest finite magnitude
+    each([&](int u, const f32x4& p0, const f32x4& q0) {
+        f32x4 p = p0, q = q0;
+        if (NU == 0) normed(u, p, q);
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            mx = fmaxf(mx, fabsf(p[i]) < INFINITY ? fabsf(p[i]) : 0.f);
+            mx = fmaxf(mx, fabsf(q[i]) < INFINITY ? fabsf(q[i]) : 0.f);
+        }
+    });
+    mx = wave_max(mx);
+    if (lane == 0) s_red[2][r][wave] = mx;
+    __syncthreads();
+    mx = fmaxf(fmaxf(s_red[2][r][0], s_red[2][r][1]), fmaxf(s_red[2][r][2], s_red[2][r][3]));
+    // 2^e with mx 2^e in [2^13, 2^14); rows of zeros keep 2^0
+    const int ex = (int)((__float_as_uint(mx) >> 23) & 0xFF) - 127;
+    const int e = mx > 0.f ? min(max(13 - ex, -126), 126) : 0;
+    const float sc = __uint_as_float((uint32_t)(e + 127) << 23);
+    if (tid == 0) gst(a.xs + row, __uint_as_float((uint32_t)(127 - e) << 23));
+    uint4* xp = a.xp + (int64_t)mt * a.nks * 128 + (row & 15);
+    each([&](int u, const f32x4& p0, const f32x4& q0) {
+        f32x4 p = p0, q = q0;
+        if (NU == 0) normed(u, p, q);
+        float w[8];
+        _Float16 h[8], l[8];
+#pragma unroll
+        for (int i = 0; i < 4; i++) { w[i] = p[i] * sc; w[4 + i] = q[i] * sc; }
+#pragma unroll
+        for (int i = 0; i < 8; i++) {
+            h[i] = (_Float16)w[i];
+            l[i] = fabsf(w[i]) < INFINITY ? (_Float16)(w[i] - (float)h[i]) : (_Float16)0.0f;
+        }
+        constexpr int O[2][8] = {{0, 4, 1, 5, 2, 6, 3, 7}, {0, 2, 1, 3, 4, 6, 5, 7}};
+        f16x8 hv, lv;
+#pragma unroll
+        for (int i = 0; i < 8; i++) { hv[i] = h[O[Q2][i]]; lv[i] = l[O[Q2][i]]; }
+        uint4* d = xp + (int64_t)(u >> 2) * 128 + (u & 3) * 16;
+        gst((f16x8*)d, hv);
+        gst((f16x8*)(d + 64), lv);
+        if (Q2) {
+            // sums of 16 values: threads 2 i, 2 i + 1 hold the two units
+            float s = ((w[0] + w[1]) + (w[2] + w[3])) + ((w[4] + w[5]) + (w[6] + w[7]));
+            s += dpp_f<0xB1>(s);
+            if (!(u & 1)) {
+                const int g = u >> 1;
+                const uint32_t b0 = __float_as_uint(s) & 0xFFFF0000u;
+                const float s1 = s - __uint_as_float(b0);
+                const uint32_t b1 = __float_as_uint(s1) & 0xFFFF0000u;
+                const float s2 = s1 - __uint_as_float(b1);
+                uint16_t* o = a.xg + (((int64_t)mt * a.ngw + (g >> 5)) * 3 * 64 + ((g >> 3) & 3) * 16 + (row & 15)) * 8 + (g & 7);
+                gst(o, (uint16_t)(b0 >> 16));
+                gst(o + 64 * 8, (uint16_t)(b1 >> 16));
+                gst(o + 2 * 64 * 8, (uint16_t)(__float_as_uint(s2) >> 16));
+            }
+        }
+    });
+    if (Q2) {
+        // zero the sums past the padded row (whole windows are read)
+        for (int g = nup / 2 + tid; g < 32 * a.ngw; g += 256) {
+            uint16_t* o = a.xg + (((int64_t)mt * a.ngw + (g >> 5)) * 3 * 64 + ((g >> 3) & 3) * 16 + (row & 15)) * 8 + (g & 7);
+#pragma unroll
+            for (int p = 0; p < 3; p++) gst(o + p * 64 * 8, (uint16_t)0);
+        }
+    }
+}
+
+// ---------------------------------------------------------------------------
+// the product
+// ---------------------------------------------------------------------------
+struct RowsArgs {
+    const uint4* xp;
+    const float* xs;
+    const uint4* xg;
+    const uint8_t* w[3];
+    const uint8_t* w2;
+    float* y[3];
+    int N[3];
+    int t0[3];             // first column tile of each segment
+    int nseg;
+    int M, K, nks, ngw, epi;
+    int mt, nt;            // row tiles of 16 MI, column tiles of 16 NJ NW
+    int xb, mpp, npp;      // XCD split: weight parts, row / column tiles per part
+    int NW, KW;
+    // grouped rows (experts): plan[0] = row tiles in use, plan[1 + i] = group of row tile i
+    const int* plan;
+    int64_t stride;
+};
+
+// x[j] of lane row g -> x[g] of lane row j (lane rows: 16 lanes each)
+__device__ __forceinline__ void transpose4(uint32_t (&x)[4]) {
+    const auto a = __builtin_amdgcn_permlane16_swap(x[0], x[1], false, false);
+    const auto b = __builtin_amdgcn_permlane16_swap(x[2], x[3], false, false);
+    const auto c = __builtin_amdgcn_permlane32_swap(a[0], b[0], false, false);
+    const auto d = __builtin_amdgcn_permlane32_swap(a[1], b[1], false, false);
+    x[0] = c[0]; x[2] = c[1]; x[1] = d[0]; x[3] = d[1];
+}
+
+// o[g] in every lane = v of lane row g (same lane % 16)
+__device__ __forceinline__ void spread4(uint32_t v, uint32_t (&o)[4]) {
+    const auto a = __builtin_amdgcn_permlane16_swap(v, v, false, false);      // [0 0 2 2], [1 1 3 3]
+    const auto b = __builtin_amdgcn_permlane32_swap(a[0], a[0], false, false);
+    const auto c = __builtin_amdgcn_permlane32_swap(a[1], a[1], false, false);
+    o[0] = b[0]; o[2] = b[1]; o[1] = c[0]; o[3] = c[1];
+}
+
+// One column tile's weights for a 128-value step, as loaded
+template <int FMT>
+struct WRaw;
+template <>
+struct WRaw<FMT_Q4_0F> { u32x4 n; uint32_t s; };
+template <>
+struct WRaw<FMT_Q4_0> { u32x4 n; uint32_t s; };
+template <>
+struct WRaw<FMT_Q2_K> { u32x2 q, s; uint32_t d; };
+template <>
+struct WRaw<FMT_Q2_S> { u32x2 q[4]; uint32_t s[4], d[4]; };
+
+// Column n, 128-value step ss, lane row f.  Steps past the row's blocks read
+// its last block; x is zero there.  Columns past N read column 0.
+template <int FMT>
+__device__ __forceinline__ void w_load(const uint8_t* w, int n, int K, int ss, int f, WRaw<FMT>& r) {
+    if constexpr (FMT == FMT_Q4_0F) {
+        const int nb = K >> 5;
+        const uint8_t* p = w + ((int64_t)n * nb + min(4 * ss + f, nb - 1)) * 20;
+        r.s = gld((const uint32_t*)p);
+        r.n = gld4(p + 4);
+    } else if constexpr (FMT == FMT_Q4_0) {
+        // 18-byte blocks: an odd block's 16 nibble bytes are 4-byte aligned
+        // behind its scale, an even block's first 16 bytes are; the other
+        // two bytes are the scale or the last four nibbles
+        const int nb = K >> 5;
+        const int64_t u = (int64_t)n * nb + min(4 * ss + f, nb - 1);
+        const uint8_t* p = w + u * 18;
+        const int odd = (int)(u & 1);
+        r.n = gld4(p + 2 * odd);
+        r.s = (uint32_t)gld((const uint16_t*)(p + (odd ? 0 : 16))) | ((uint32_t)odd << 31);
+    } else if constexpr (FMT == FMT_Q2_K) {
+        const int64_t pg = (int64_t)n * (K >> 7) + ss;
+        const uint8_t* b = w + (pg >> 1) * 84;
+        const int o = (int)(pg & 1);
+        r.s = gld2(b + 8 * o);
+        r.q = gld2(b + 16 + 32 * o + 8 * f);
+        r.d = gld((const uint16_t*)(b + 80));
+    } else {
+        const int nb = K >> 5;
+#pragma unroll
+        for (int s = 0; s < 4; s++) {
+            const int64_t sl = (int64_t)n * nb + min(4 * ss + s, nb - 1);   // 32-value slice in flat order
+            const uint8_t* b = w + (sl >> 3) * 84;
+            const int j = (int)(sl & 7);
+            r.q[s] = gld2(b + 16 + 32 * (j >> 2) + 8 * f);
+            r.s[s] = (uint32_t)gld(b + 2 * j + (f >> 1)) | ((uint32_t)(2 * (j & 3)) << 8);
+            r.d[s] = gld((const uint16_t*)(b + 80));
+        }
+    }
+}
+
+// (v & mask) | 0x64006400: bit fields of both halves as f16 1024 + field (one
+// v_and_or_b32; written out because the compiler splits it into two literals)
+__device__ __forceinline__ f16x2 f16_field(uint32_t v, uint32_t mask) {
+    uint32_t r;
+    asm("v_and_or_b32 %0, %1, %2, %3" : "=v"(r) : "v"(v), "s"(mask), "v"(0x64006400u));
+    return __builtin_bit_cast(f16x2, r);
+}
+__device__ __forceinline__ f16x2 f16_both(float v) { return f16x2{(_Float16)v, (_Float16)v}; }
+__device__ __forceinline__ uint32_t f16_fma(f16x2 a, f16x2 b, f16x2 c) {
+    return __builtin_bit_cast(uint32_t, __builtin_elementwise_fma(a, b, c));
+}
+// the eight nibbles of a dword -> q - 7 as f16, dword j = nibbles (j, j + 4);
+// a field at bit 4 of its half is 1024 + 16 q: the scale by 1/16 is exact
+__device__ __forceinline__ u32x4 q4_unpack(uint32_t x) {
+    const uint32_t y = x >> 8;
+    const f16x2 one = f16_both(1.0f), m7 = f16_both(-1031.0f), sx = f16_both(0.0625f), m71 = f16_both(-71.0f);
+    return u32x4{f16_fma(f16_field(x, 0x000F000Fu), one, m7), f16_fma(f16_field(x, 0x00F000F0u), sx, m71),
+                 f16_fma(f16_field(y, 0x000F000Fu), one, m7), f16_fma(f16_field(y, 0x00F000F0u), sx, m71)};
+}
+// sc * q as f16 for the 2-bit fields at bit 2 st of eight bytes, dwords =
+// bytes (0, 2), (1, 3), (4, 6), (5, 7); a field there is 1024 + 4^st q, so the
+// factor is sc 4^-st and every step is exact (sc <= 15); by: the scale byte
+__device__ __forceinline__ u32x4 q2_unpack(u32x2 b, uint32_t by, int st) {
+    const float f = st == 0 ? 1.0f : st == 1 ? 0.25f : st == 2 ? 0.0625f : 0.015625f;
+    const uint32_t mask = 0x00030003u << (2 * st);
+    const f16x2 t = f16_field(__builtin_amdgcn_perm(by, by, 0x0C000C00u), 0x000F000Fu);
+    const f16x2 sc = __builtin_bit_cast(f16x2, f16_fma(t, f16_both(f), f16_both(-1024.0f * f)));
+    const f16x2 m = sc * f16_both(-1024.0f);
+    return u32x4{f16_fma(f16_field(b.x, mask), sc, m), f16_fma(f16_field(b.x >> 8, mask), sc, m),
+                 f16_fma(f16_field(b.y, mask), sc, m), f16_fma(f16_field(b.y >> 8, mask), sc, m)};
+}
+
+// nibble dwords and fp32 scale of one loaded Q4 block
+template <int FMT>
+__device__ __forceinline__ void q4_block(const WRaw<FMT>& r, uint32_t (&n)[4], uint32_t& s) {
+    if constexpr (FMT == FMT_Q4_0F) {
+        s = r.s;
+        n[0] = r.n.x; n[1] = r.n.y; n[2] = r.n.z; n[3] = r.n.w;
+    } else {
+        const bool odd = (int)r.s < 0;
+        const uint32_t x = r.s & 0xFFFFu;
+        const uint32_t e0 = __builtin_amdgcn_alignbyte(r.n.y, r.n.x, 2), e1 = __builtin_amdgcn_alignbyte(r.n.z, r.n.y, 2);
+        const uint32_t e2 = __builtin_amdgcn_alignbyte(r.n.w, r.n.z, 2), e3 = __builtin_amdgcn_alignbyte(x, r.n.w, 2);
+        n[0] = odd ? r.n.x : e0; n[1] = odd ? r.n.y : e1; n[2] = odd ? r.n.z : e2; n[3] = odd ? r.n.w : e3;
+        s = __float_as_uint(f16_to_f32(odd ? x : r.n.x & 0xFFFFu));
+    }
+}
+
+// Weights of a 128-value step ready to use: the four steps' B fragments are
+// formed one at a time by step()
+template <int FMT>
+struct WStep {
+    uint32_t n[4];       // Q4: this lane's nibble dword of each 32-value block
+    float sc[4];         // Q4 / Q2_S: the column's scale per block; Q2_K: sc[0]
+    u32x2 q[FMT == FMT_Q2_S ? 4 : 1];
+    uint32_t s[4];
+    __device__ __forceinline__ void take(const WRaw<FMT>& r, int f) {
+        if constexpr (FMT == FMT_Q4_0F || FMT == FMT_Q4_0) {
+            uint32_t s1, s4[4];
+            q4_block<FMT>(r, n, s1);
+            transpose4(n);
+            spread4(s1, s4);
+#pragma unroll
+            for (int i = 0; i < 4; i++) sc[i] = __uint_as_float(s4[i]);
+        } else if constexpr (FMT == FMT_Q2_K) {
+            q[0] = r.q;
+            // scale byte of group 2 g + half: byte 2 g + (f >> 1) of the page's eight
+            const uint32_t sh = 8 * (f >> 1);
+            s[0] = r.s.x >> sh; s[1] = r.s.x >> (sh + 16); s[2] = r.s.y >> sh; s[3] = r.s.y >> (sh + 16);
+            sc[0] = f16_to_f32(r.d);
+        } else {
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                q[i] = r.q[i];
+                s[i] = r.s[i];
+                sc[i] = f16_to_f32(r.d[i]);
+            }
+        }
+    }
+    __device__ __forceinline__ f16x8 frag(int st) const {
+        if constexpr (FMT == FMT_Q4_0F || FMT == FMT_Q4_0) return __builtin_bit_cast(f16x8, q4_unpack(n[st]));
+        else if constexpr (FMT == FMT_Q2_K) return __builtin_bit_cast(f16x8, q2_unpack(q[0], s[st], st));
+        else return __builtin_bit_cast(f16x8, q2_unpack(u32x2{q[st].x >> (s[st] >> 8), q[st].y >> (s[st] >> 8)}, s[st], 0));
+    }
+};
+
+// -(dmin m) of the eight 16-value groups g0 .. g0 + 7 of column n as two bf16 parts
+template <int FMT>
+__device__ __forceinline__ void min_frag(const uint8_t* w, int n, int K, int g0, bf16x8& hi, bf16x8& lo) {
+    const int ng = K >> 4;
+    uint32_t ph[4], pl[4];
+    u32x2 pb{0, 0};
+    float pd = 0.f;
+    if constexpr (FMT == FMT_Q2_K) {                // a page of the row: eight groups of one block
+        const int64_t pg = (int64_t)n * (K >> 7) + min(g0 >> 3, (K >> 7) - 1);
+        const uint8_t* b = w + (pg >> 1) * 84;
+        pb = gld2(b + 8 * (pg & 1));
+        pd = -f16_to_f32(gld((const uint16_t*)(b + 82)));
+    }
+#pragma unroll
+    for (int i = 0; i < 4; i++) {                   // a 32-value slice: two groups of one block
+        uint32_t by;
+        float d;
+        if constexpr (FMT == FMT_Q2_K) {
+            by = ((i & 2) ? pb.y : pb.x) >> (16 * (i & 1));
+            d = pd;
+        } else {
+            const int64_t sl = (int64_t)n * (K >> 5) + (min(g0 + 2 * i, ng - 2) >> 1);
+            const uint8_t* b = w + (sl >> 3) * 84;
+            by = gld((const uint16_t*)(b + 2 * (sl & 7)));
+            d = -f16_to_f32(gld((const uint16_t*)(b + 82)));
+        }
+        const float v0 = d * (float)((by >> 4) & 15u), v1 = d * (float)((by >> 12) & 15u);
+        const uint32_t h0 = __float_as_uint(v0) & 0xFFFF0000u, h1 = __float_as_uint(v1) & 0xFFFF0000u;
+        ph[i] = (h0 >> 16) | h1;
+        pl[i] = (__float_as_uint(v0 - __uint_as_float(h0)) >> 16) | (__float_as_uint(v1 - __uint_as_float(h1)) & 0xFFFF0000u);
+    }
+    hi = __builtin_bit_cast(bf16x8, u32x4{ph[0], ph[1], ph[2], ph[3]});
+    lo = __builtin_bit_cast(bf16x8, u32x4{pl[0], pl[1], pl[2], pl[3]});
+}
+
+// This workgroup's tile.  Workgroups go to the 8 XCDs round-robin in linear
+// order: id % 8 owns row part (id % 8) / xb and column part (id % 8) % xb.
+struct Tile {
+    const uint8_t* w;
+    const uint8_t* w2;
+    float* y;
+    int N, by, bx;         // bx: column tile inside the segment
+    __device__ __forceinline__ bool find(const RowsArgs& a) {
+        const int xcd = blockIdx.x & 7, kb = blockIdx.x >> 3;
+        const int mm = kb / a.npp, nn = kb - mm * a.npp;
+        int mpp = a.mpp, mt = a.mt;
+        if (a.plan) {                               // row tiles in use: known on the device only
+            mt = min(mt, __builtin_amdgcn_readfirstlane(gld(a.plan)));
+            mpp = (mt + 8 / a.xb - 1) / (8 / a.xb);
+        }
+        by = (xcd / a.xb) * mpp + mm;
+        bx = (xcd % a.xb) * a.npp + nn;
+        if (mm >= mpp || by >= mt || bx >= a.nt) return false;
+        const int sg = (a.nseg > 1 && bx >= a.t0[1]) + (a.nseg > 2 && bx >= a.t0[2]);
+        w = sg == 0 ? a.w[0] : sg == 1 ? a.w[1] : a.w[2];
+        w2 = a.w2;
+        y = sg == 0 ? a.y[0] : sg == 1 ? a.y[1] : a.y[2];
+        N = sg == 0 ? a.N[0] : sg == 1 ? a.N[1] : a.N[2];
+        bx -= sg == 0 ? a.t0[0] : sg == 1 ? a.t0[1] : a.t0[2];
+        if (a.plan) {
+            const int64_t g = __builtin_amdgcn_readfirstlane(gld(a.plan + 1 + by));
+            w += g * a.stride;
+            w2 += g * a.stride;
+        }
+        return true;
+    }
+};
+
+template <int NMAT>
+__device__ __forceinline__ void finish(const RowsArgs& a, const Tile& t, int r, int c, float v, float u) {
+    if (r >= a.M || c >= t.N) return;
+    float* o = t.y + (int64_t)r * t.N + c;
+    if (NMAT == 2) gst(o, silu_mul(v, u));
+    else if (a.epi == RINA_EPI_ADD) gst(o, gld(o) + v);
+    else gst(o, v);
+}
+
+// The same for 32-column tiles (two lane rows of 32 columns): a lane holds
+// blocks 4 ss + f and 4 ss + 2 + f of its column, or its half of a page
+template <int FMT>
+struct WRaw32;
+template <>
+struct WRaw32<FMT_Q4_0F> { WRaw<FMT_Q4_0F> b[2]; };
+template <>
+struct WRaw32<FMT_Q4_0> { WRaw<FMT_Q4_0> b[2]; };
+template <>
+struct WRaw32<FMT_Q2_K> { u32x2 q[2], s; uint32_t d; };
+template <>
+struct WRaw32<FMT_Q2_S> { u32x2 q[4][2]; uint32_t s[4], d[4]; };
+
+template <int FMT>
+__device__ __forceinline__ void w_load32(const uint8_t* w, int n, int K, int ss, int f, WRaw32<FMT>& r) {
+    if constexpr (FMT == FMT_Q4_0F || FMT == FMT_Q4_0) {
+        w_load<FMT>(w, n, K, ss, f, r.b[0]);
+        w_load<FMT>(w, n, K, ss, f + 2, r.b[1]);
+    } else if constexpr (FMT == FMT_Q2_K) {
+        const int64_t pg = (int64_t)n * (K >> 7) + ss;
+        const uint8_t* b = w + (pg >> 1) * 84;
+        const int o = (int)(pg & 1);
+        r.s = gld2(b + 8 * o);
+        r.q[0] = gld2(b + 16 + 32 * o + 8 * f);
+        r.q[1] = gld2(b + 32 + 32 * o + 8 * f);
+        r.d = gld((const uint16_t*)(b + 80));
+    } else {
+        const int nb = K >> 5;
+#pragma unroll
+        for (int s = 0; s < 4; s++) {
+            const int64_t sl = (int64_t)n * nb + min(4 * ss + s, nb - 1);   // 32-value slice in flat order
+            const uint8_t* b = w + (sl >> 3) * 84;
+            const int j = (int)(sl & 7);
+            r.q[s][0] = gld2(b + 16 + 32 * (j >> 2) + 8 * f);
+            r.q[s][1] = gld2(b + 32 + 32 * (j >> 2) + 8 * f);
+            r.s[s] = (uint32_t)gld((const uint16_t*)(b + 2 * j)) | ((uint32_t)(2 * (j & 3)) << 16);
+            r.d[s] = gld((const uint16_t*)(b + 80));
+        }
+    }
+}
+
+template <int FMT>
+struct WStep32 {
+    uint32_t n[4][2];    // Q4: this lane's nibble dwords (halves 0, 1) of each 32-value block
+    float sc[4];
+    u32x2 q[FMT == FMT_Q2_S ? 4 : 1][2];
+    uint32_t s[4];
+    __device__ __forceinline__ void take(const WRaw32<FMT>& r) {
+        if constexpr (FMT == FMT_Q4_0F || FMT == FMT_Q4_0) {
+#pragma unroll
+            for (int b = 0; b < 2; b++) {           // lane row 0 holds block 2 b, lane row 1 block 2 b + 1
+                uint32_t x[4], s1;
+                q4_block<FMT>(r.b[b], x, s1);
+                // [own d0, d1 of the lower row | d0, d1 of the upper row]: lane row f gets dword f (and 2 + f)
+                const auto lo = __builtin_amdgcn_permlane32_swap(x[0], x[1], false, false);
+                const auto hi = __builtin_amdgcn_permlane32_swap(x[2], x[3], false, false);
+                const auto sp = __builtin_amdgcn_permlane32_swap(s1, s1, false, false);
+                n[2 * b][0] = lo[0]; n[2 * b + 1][0] = lo[1];
+                n[2 * b][1] = hi[0]; n[2 * b + 1][1] = hi[1];
+                sc[2 * b] = __uint_as_float(sp[0]);
+                sc[2 * b + 1] = __uint_as_float(sp[1]);
+            }
+        } else if constexpr (FMT == FMT_Q2_K) {
+            q[0][0] = r.q[0]; q[0][1] = r.q[1];
+            s[0] = r.s.x; s[1] = r.s.x >> 16; s[2] = r.s.y; s[3] = r.s.y >> 16;
+            sc[0] = f16_to_f32(r.d);
+        } else {
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                q[i][0] = r.q[i][0]; q[i][1] = r.q[i][1];
+                s[i] = r.s[i];
+                sc[i] = f16_to_f32(r.d[i]);
+            }
+        }
+    }
+    // weights of 16-value half h of 32-value step st
+    __device__ __forceinline__ f16x8 frag(int st, int h) const {
+        if constexpr (FMT == FMT_Q4_0F || FMT == FMT_Q4_0) return __builtin_bit_cast(f16x8, q4_unpack(n[st][h]));
+        else if constexpr (FMT == FMT_Q2_K) return __builtin_bit_cast(f16x8, q2_unpack(q[0][h], s[st] >> (8 * h), st));
+        else {
+            const uint32_t sh = s[st] >> 16;
+            return __builtin_bit_cast(f16x8, q2_unpack(u32x2{q[st][h].x >> sh, q[st][h].y >> sh}, s[st] >> (8 * h), 0));
+        }
+    }
+};
+
+// 128-value steps whose weights a wave loads together, one batch ahead: with
+// few rows the launch is the weight stream, and a wave that asks for one step
+// at a time waits a memory round trip per step (8 x 2048 x 8192: 23.6 us with
+// one step ahead).  Bounded by the registers.
+template <int FMT, int NMAT, int MI>
+struct Batch16 { static constexpr int BT = FMT == FMT_Q2_S ? 1 : NMAT * MI >= 4 ? 2 : 4; };
+
+// ---- M <= 32: v_mfma_f32_16x16x32_f16 tiles ----
+// MI 16-row tiles (all the rows of a group), 16 columns (per matrix) per wave.
+template <int FMT, int NMAT, int MI>
+__global__ __launch_bounds__(512, 2) void rows16_kernel(RowsArgs a) {
+    extern __shared__ __align__(16) float s_part[];
+    constexpr int BT = Batch16<FMT, NMAT, MI>::BT;
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int fr = lane & 15, f = lane >> 4;
+    Tile t;
+    if (!t.find(a)) return;
+    const int wn = wave % a.NW, wk = wave / a.NW;
+    const int c0 = (t.bx * a.NW + wn) * 16 + fr, N = t.N;
+    const int K = a.K, nss = a.nks >> 2, col = c0 < N ? c0 : 0;
+    const int mtiles = (a.M + 15) >> 4;
+    const f16x8* ap[MI];
+#pragma unroll
+    for (int i = 0; i < MI; i++) ap[i] = (const f16x8*)a.xp + (int64_t)min(t.by * MI + i, mtiles - 1) * a.nks * 128 + lane;
+    f32x4 acc[NMAT][MI];
+#pragma unroll
+    for (int m = 0; m < NMAT; m++)
+#pragma unroll
+        for (int i = 0; i < MI; i++) acc[m][i] = f32x4{0.f, 0.f, 0.f, 0.f};
+    WRaw<FMT> raw[BT][NMAT];
+    f16x8 af[MI][8];
+    // batch b: steps BT b .. + BT - 1 (past the end: the last step again, not multiplied)
+    auto load_w = [&](int b) {
+#pragma unroll
+        for (int s = 0; s < BT; s++)
+#pragma unroll
+            for (int m = 0; m < NMAT; m++) w_load<FMT>(m ? t.w2 : t.w, col, K, min(BT * b + s, nss - 1), f, raw[s][m]);
+    };
+    auto load_a = [&](int ss) {
+#pragma unroll
+        for (int i = 0; i < MI; i++)
+#pragma unroll
+            for (int c = 0; c < 8; c++) af[i][c] = gld(ap[i] + (int64_t)min(ss, nss - 1) * 512 + 64 * c);
+    };
+    constexpr bool PAGE = FMT == FMT_Q2_K;          // one scale per 128-value step
+    const int nb = (nss + BT - 1) / BT;
+    if (wk < nb) {
+        load_w(wk);
+        load_a(BT * wk);
+    }
+    for (int b = wk; b < nb; b += a.KW) {
+        WStep<FMT> ws[BT][NMAT];
+#pragma unroll
+        for (int s = 0; s < BT; s++)
+#pragma unroll
+            for (int m = 0; m < NMAT; m++) ws[s][m].take(raw[s][m], f);
+        const int bn = b + a.KW < nb ? b + a.KW : b;   // the last batch loads itself again
+#pragma unroll
+        for (int s = 0; s < BT; s++) {
+            f16x8 at[MI][8];
+#pragma unroll
+            for (int i = 0; i < MI; i++)
+#pragma unroll
+                for (int c = 0; c < 8; c++) at[i][c] = af[i][c];
+            load_a(s + 1 < BT ? BT * b + s + 1 : BT * bn);
+            if (s == 0) load_w(bn);
+            __builtin_amdgcn_sched_barrier(0);      // issued before this step's products
+            if (BT > 1 && BT * b + s >= nss) continue;
+#pragma unroll
+            for (int m = 0; m < NMAT; m++) {
+                f32x4 d[MI];
+#pragma unroll
+                for (int st = 0; st < 4; st++) {
+                    const f16x8 w = ws[s][m].frag(st);
+#pragma unroll
+                    for (int i = 0; i < MI; i++) {
+                        if (!PAGE || st == 0) d[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+                        d[i] = __builtin_amdgcn_mfma_f32_16x16x32_f16(at[i][2 * st + 1], w, d[i], 0, 0, 0);
+                    }
+#pragma unroll
+                    for (int i = 0; i < MI; i++) {
+                        d[i] = __builtin_amdgcn_mfma_f32_16x16x32_f16(at[i][2 * st], w, d[i], 0, 0, 0);
+                        if (!PAGE || st == 3) {
+#pragma unroll
+                            for (int e = 0; e < 4; e++) acc[m][i][e] = fmaf(ws[s][m].sc[PAGE ? 0 : st], d[i][e], acc[m][i][e]);
+                        }
+                    }
+                }
+            }
+        }
+    }
+    if constexpr (FMT == FMT_Q2_K || FMT == FMT_Q2_S) {
+        for (int gw = wk; gw < a.ngw; gw += a.KW) {
+            bf16x8 xg[MI][3];
+#pragma unroll
+            for (int i = 0; i < MI; i++) {
+                const bf16x8* gp = (const bf16x8*)a.xg + ((int64_t)min(t.by * MI + i, mtiles - 1) * a.ngw + gw) * 192 + lane;
+#pragma unroll
+                for (int p = 0; p < 3; p++) xg[i][p] = gld(gp + 64 * p);
+            }
+#pragma unroll
+            for (int m = 0; m < NMAT; m++) {
+                bf16x8 hi, lo;
+                min_frag<FMT>(m ? t.w2 : t.w, col, K, 32 * gw + 8 * f, hi, lo);
+#pragma unroll
+                for (int i = 0; i < MI; i++) {
+                    f32x4 d = acc[m][i];
+                    d = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xg[i][2], hi, d, 0, 0, 0);
+                    d = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xg[i][1], lo, d, 0, 0, 0);
+                    d = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xg[i][1], hi, d, 0, 0, 0);
+                    d = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xg[i][0], lo, d, 0, 0, 0);
+                    acc[m][i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xg[i][0], hi, d, 0, 0, 0);
+                }
+            }
+        }
+    }
+    // the KW partial tiles, halved per round: waves h .. 2 h - 1 leave theirs
+    // in LDS, waves 0 .. h - 1 add
+    f32x4* sp = (f32x4*)s_part;
+    for (int h = a.KW >> 1; h >= 1; h >>= 1) {
+        f32x4* d = sp + (int64_t)((wk >= h ? wk - h : wk) * a.NW + wn) * NMAT * MI * 64 + lane;
+        if (wk >= h && wk < 2 * h) {
+#pragma unroll
+            for (int m = 0; m < NMAT; m++)
+#pragma unroll
+                for (int i = 0; i < MI; i++) d[(m * MI + i) * 64] = acc[m][i];
+        }
+        __syncthreads();
+        if (wk < h) {
+#pragma unroll
+            for (int m = 0; m < NMAT; m++)
+#pragma unroll
+                for (int i = 0; i < MI; i++) acc[m][i] += d[(m * MI + i) * 64];
+        }
+        __syncthreads();
+    }
+    if (wk > 0) return;
+#pragma unroll
+    for (int i = 0; i < MI; i++) {
+        const int r0 = (t.by * MI + i) * 16 + 4 * f;
+        if (r0 >= a.M) continue;
+        const f32x4 sc = gld((const f32x4*)(a.xs + r0));
+#pragma unroll
+        for (int e = 0; e < 4; e++) finish<NMAT>(a, t, r0 + e, c0, acc[0][i][e] * sc[e], acc[NMAT - 1][i][e] * sc[e]);
+    }
+}
+
+// ---- M > 32: v_mfma_f32_32x32x16_f16 tiles ----
+// A wave owns 32 R rows x 32 C columns (per matrix).  SH: the 4 waves of a
+// workgroup take neighbouring columns over the whole of K and share the rows'
+// fragments through LDS (two buffers of a 128-value step); else every wave
+// reads its rows' fragments itself and KW waves split K.
+template <int FMT, int NMAT, int R, int C, bool SH>
+__global__ __launch_bounds__(SH ? 256 : 512, 2) void rows32_kernel(RowsArgs a) {
+    extern __shared__ __align__(16) float s_part[];
+    __shared__ __align__(16) f16x8 s_a[SH ? 2 : 1][SH ? 2 * R : 1][SH ? 8 : 1][64];
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int fr = lane & 31, f = lane >> 5;
+    Tile t;
+    if (!t.find(a)) return;
+    const int wn = wave % a.NW, wk = wave / a.NW;
+    const int n0 = (t.bx * a.NW + wn) * 32 * C, N = t.N;
+    const int K = a.K, nss = a.nks >> 2, mtiles = (a.M + 15) >> 4;
+    int col[C];
+#pragma unroll
+    for (int j = 0; j < C; j++) col[j] = n0 + 32 * j + fr < N ? n0 + 32 * j + fr : 0;
+    f32x16 acc[NMAT][R][C];
+#pragma unroll
+    for (int m = 0; m < NMAT; m++)
+#pragma unroll
+        for (int i = 0; i < R; i++)
+#pragma unroll
+            for (int j = 0; j < C; j++)
+#pragma unroll
+                for (int e = 0; e < 16; e++) acc[m][i][j][e] = 0.f;
+    WRaw32<FMT> raw[NMAT][C];
+    auto load_w = [&](int ss) {
+#pragma unroll
+        for (int m = 0; m < NMAT; m++)
+#pragma unroll
+            for (int j = 0; j < C; j++) w_load32<FMT>(m ? t.w2 : t.w, col[j], K, ss, f, raw[m][j]);
+    };
+    // fragment of 32-row tile i, 16-value half h, part p of a 32-value step:
+    // 16-row tile 2 i + (row / 16), lane row 2 h + f of its 64-unit chunk
+    const int lu = (fr & 15) + 16 * f;
+    constexpr bool PAGE = FMT == FMT_Q2_K;          // one scale per 128-value step
+    f32x16 pd[PAGE ? NMAT : 1][PAGE ? R : 1][PAGE ? C : 1];
+    // the products of step st (32 values) of a 128-value step; at[i][h][p]
+    auto mul = [&](const WStep32<FMT> (&ws)[NMAT][C], const f16x8 (&at)[R][2][2], int st) {
+#pragma unroll
+        for (int m = 0; m < NMAT; m++)
+#pragma unroll
+            for (int j = 0; j < C; j++) {
+                f32x16 d[R];
+#pragma unroll
+                for (int h = 0; h < 2; h++) {
+                    const f16x8 b = ws[m][j].frag(st, h);
+#pragma unroll
+                    for (int p = 1; p >= 0; p--)
+#pragma unroll
+                        for (int i = 0; i < R; i++) {
+                            f32x16 c;
+                            if (h == 0 && p == 1) {
+                                if (PAGE && st > 0) c = pd[PAGE ? m : 0][PAGE ? i : 0][PAGE ? j : 0];
+                                else {
+#pragma unroll
+                                    for (int e = 0; e < 16; e++) c[e] = 0.f;
+                                }
+                            } else {
+                                c = d[i];
+                            }
+                            d[i] = __builtin_amdgcn_mfma_f32_32x32x16_f16(at[i][h][p], b, c, 0, 0, 0);
+                        }
+                }
+#pragma unroll
+                for (int i = 0; i < R; i++) {
+                    if constexpr (PAGE) pd[m][i][j] = d[i];
+                    if (!PAGE || st == 3) {
+                        const float sc = ws[m][j].sc[PAGE ? 0 : st];
+#pragma unroll
+                        for (int e = 0; e < 16; e++) acc[m][i][j][e] = fmaf(sc, d[i][e], acc[m][i][j][e]);
+                    }
+                    // consumed here: left alone, the compiler defers the scale
+                    // products of a whole step and spills
+                    if constexpr (PAGE) asm volatile("" : "+v"(pd[m][i][j]));
+                    else asm volatile("" : "+v"(acc[m][i][j]));
+                }
+            }
+    };
+    auto take = [&](WStep32<FMT> (&ws)[NMAT][C]) {
+#pragma unroll
+        for (int m = 0; m < NMAT; m++)
+#pragma unroll
+            for (int j = 0; j < C; j++) ws[m][j].take(raw[m][j]);
+    };
+    if constexpr (SH) {
+        // wave wn moves a quarter of a step: two of the eight (step, part)
+        // chunks of every 16-row tile
+        const f16x8* ap[2 * R];
+#pragma unroll
+        for (int i = 0; i < 2 * R; i++) ap[i] = (const f16x8*)a.xp + (int64_t)min(t.by * 2 * R + i, mtiles - 1) * a.nks * 128 + lane;
+        f16x8 sr[2 * R][2];
+        auto load_s = [&](int ss) {
+#pragma unroll
+            for (int i = 0; i < 2 * R; i++)
+#pragma unroll
+                for (int c = 0; c < 2; c++) sr[i][c] = gld(ap[i] + (int64_t)ss * 512 + (2 * wn + c) * 64);
+        };
+        auto store_s = [&](int buf) {
+#pragma unroll
+            for (int i = 0; i < 2 * R; i++)
+#pragma unroll
+                for (int c = 0; c < 2; c++) s_a[buf][i][2 * wn + c][lane] = sr[i][c];
+        };
+        load_s(0);
+        load_w(0);
+        store_s(0);
+        __syncthreads();
+        for (int ss = 0; ss < nss; ss++) {
+            const int sn = ss + 1 < nss ? ss + 1 : ss;     // the last step loads itself again
+            load_s(sn);
+            WStep32<FMT> ws[NMAT][C];
+            take(ws);
+            load_w(sn);
+            __builtin_amdgcn_sched_barrier(0);      // issued before this step's products
+#pragma unroll
+            for (int st = 0; st < 4; st++) {
+                f16x8 at[R][2][2];
+#pragma unroll
+                for (int i = 0; i < R; i++)
+#pragma unroll
+                    for (int h = 0; h < 2; h++)
+#pragma unroll
+                        for (int p = 0; p < 2; p++) at[i][h][p] = s_a[ss & 1][2 * i + (fr >> 4)][2 * st + p][lu + 32 * h];
+                mul(ws, at, st);
+            }
+            store_s((ss & 1) ^ 1);                  // that buffer's readers are past the last barrier
+            __syncthreads();
+        }
+    } else {
+        const f16x8* ap[R];
+#pragma unroll
+        for (int i = 0; i < R; i++) ap[i] = (const f16x8*)a.xp + (int64_t)min((t.by * R + i) * 2 + (fr >> 4), mtiles - 1) * a.nks * 128 + lu;
+        f16x8 af[2][R][2][2];
+        auto load_a = [&](f16x8 (&x)[R][2][2], int ks) {
+#pragma unroll
+            for (int i = 0; i < R; i++)
+#pragma unroll
+                for (int h = 0; h < 2; h++)
+#pragma unroll
+                    for (int p = 0; p < 2; p++) x[i][h][p] = gld(ap[i] + (int64_t)ks * 128 + 64 * p + 32 * h);
+        };
+        if (wk < nss) {
+            load_w(wk);
+            load_a(af[0], 4 * wk);
+        }
+        for (int ss = wk; ss < nss; ss += a.KW) {
+            const int sn = ss + a.KW < nss ? ss + a.KW : ss;   // the last step loads itself again
+            WStep32<FMT> ws[NMAT][C];
+            take(ws);
+#pragma unroll
+            for (int st = 0; st < 4; st++) {
+                load_a(af[(st & 1) ^ 1], st < 3 ? 4 * ss + st + 1 : 4 * sn);
+                if (st == 0) load_w(sn);
+                __builtin_amdgcn_sched_barrier(0);  // issued before this step's products
+                mul(ws, af[st & 1], st);
+            }
+        }
+    }
+    if constexpr (FMT == FMT_Q2_K || FMT == FMT_Q2_S) {
+        for (int g2 = wk; g2 < 2 * a.ngw; g2 += a.KW) {   // 16 groups: half a window
+            bf16x8 xg[R][3];
+#pragma unroll
+            for (int i = 0; i < R; i++) {
+                const bf16x8* gp = (const bf16x8*)a.xg + ((int64_t)min((t.by * R + i) * 2 + (fr >> 4), mtiles - 1) * a.ngw + (g2 >> 1)) * 192 +
+                                   lu + 32 * (g2 & 1);
+#pragma unroll
+                for (int p = 0; p < 3; p++) xg[i][p] = gld(gp + 64 * p);
+            }
+#pragma unroll
+            for (int m = 0; m < NMAT; m++)
+#pragma unroll
+                for (int j = 0; j < C; j++) {
+                    bf16x8 hi, lo;
+                    min_frag<FMT>(m ? t.w2 : t.w, col[j], K, 16 * g2 + 8 * f, hi, lo);
+#pragma unroll
+                    for (int i = 0; i < R; i++) {
+                        f32x16 d = acc[m][i][j];
+                        d = __builtin_amdgcn_mfma_f32_32x32x16_bf16(xg[i][2], hi, d, 0, 0, 0);
+                        d = __builtin_amdgcn_mfma_f32_32x32x16_bf16(xg[i][1], lo, d, 0, 0, 0);
+                        d = __builtin_amdgcn_mfma_f32_32x32x16_bf16(xg[i][1], hi, d, 0, 0, 0);
+                        d = __builtin_amdgcn_mfma_f32_32x32x16_bf16(xg[i][0], lo, d, 0, 0, 0);
+                        acc[m][i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(xg[i][0], hi, d, 0, 0, 0);
+                    }
+                }
+        }
+    }
+    if constexpr (!SH) {
+        // the KW partial tiles, halved per round (as rows16_kernel)
+        f32x4* sp = (f32x4*)s_part;
+        constexpr int NR = NMAT * R * C * 4;
+        for (int h = a.KW >> 1; h >= 1; h >>= 1) {
+            f32x4* d = sp + (int64_t)((wk >= h ? wk - h : wk) * a.NW + wn) * NR * 64 + lane;
+            if (wk >= h && wk < 2 * h) {
+#pragma unroll
+                for (int m = 0; m < NMAT; m++)
+#pragma unroll
+                    for (int i = 0; i < R; i++)
+#pragma unroll
+                        for (int j = 0; j < C; j++)
+#pragma unroll
+                            for (int q = 0; q < 4; q++)
+                                d[(((m * R + i) * C + j) * 4 + q) * 64] = f32x4{acc[m][i][j][4 * q], acc[m][i][j][4 * q + 1], acc[m][i][j][4 * q + 2], acc[m][i][j][4 * q + 3]};
+            }
+            __syncthreads();
+            if (wk < h) {
+#pragma unroll
+                for (int m = 0; m < NMAT; m++)
+#pragma unroll
+                    for (int i = 0; i < R; i++)
+#pragma unroll
+                        for (int j = 0; j < C; j++)
+#pragma unroll
+                            for (int q = 0; q < 4; q++) {
+                                const f32x4 v = d[(((m * R + i) * C + j) * 4 + q) * 64];
+#pragma unroll
+                                for (int e = 0; e < 4; e++) acc[m][i][j][4 * q + e] += v[e];
+                            }
+            }
+            __syncthreads();
+        }
+        if (wk > 0) return;
+    }
+    // result element e of lane l: row 8 (e / 4) + 4 f + e % 4, column l % 32
+#pragma unroll
+    for (int i = 0; i < R; i++)
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+            const int r0 = (t.by * R + i) * 32 + 8 * q + 4 * f;
+            if (r0 >= a.M) continue;
+            const f32x4 sc = gld((const f32x4*)(a.xs + r0));
+#pragma unroll
+            for (int j = 0; j < C; j++)
+#pragma unroll
+                for (int e = 0; e < 4; e++)
+                    finish<NMAT>(a, t, r0 + e, n0 + 32 * j + fr, acc[0][i][j][4 * q + e] * sc[e], acc[NMAT - 1][i][j][4 * q + e] * sc[e]);
+        }
+}
+
+template <int FMT, int NMAT, int MI>
+int launch16(const RowsArgs& a, hipStream_t st) {
+    const size_t lds = a.KW > 1 ? (size_t)(a.KW / 2) * a.NW * NMAT * MI * 1024 : 0;
+    hipLaunchKernelGGL((rows16_kernel<FMT, NMAT, MI>), dim3(8 * a.mpp * a.npp), dim3(64 * a.NW * a.KW), lds, st, a);
+    return hipGetLastError() == hipSuccess ? RINA_OK : RINA_ERR_HIP;
+}
+
+template <int FMT, int NMAT, int R, int C>
+int launch32(const RowsArgs& a, hipStream_t st) {
+    const dim3 grid(8 * a.mpp * a.npp);
+    if (a.NW == 4) {
+        hipLaunchKernelGGL((rows32_kernel<FMT, NMAT, R, C, true>), grid, dim3(256), 0, st, a);
+    } else {
+        const size_t lds = a.KW > 1 ? (size_t)(a.KW / 2) * a.NW * NMAT * R * C * 4096 : 0;
+        hipLaunchKernelGGL((rows32_kernel<FMT, NMAT, R, C, false>), grid, dim3(64 * a.NW * a.KW), lds, st, a);
+    }
+    return hipGetLastError() == hipSuccess ? RINA_OK : RINA_ERR_HIP;
+}
+
+// rt: 0 / 1: one or two 16-row tiles (rows16_kernel), 2: 64 rows (rows32_kernel)
+template <int FMT>
+int launch_fmt(const RowsArgs& a, int nmat, int rt, int ct, hipStream_t st) {
+    if (nmat == 2) return rt == 0 ? launch16<FMT, 2, 1>(a, st) : rt == 1 ? launch16<FMT, 2, 2>(a, st) : launch32<FMT, 2, 2, 1>(a, st);
+    if (rt < 2) return rt == 0 ? launch16<FMT, 1, 1>(a, st) : launch16<FMT, 1, 2>(a, st);
+    return ct == 1 ? launch32<FMT, 1, 2, 1>(a, st) : launch32<FMT, 1, 2, 2>(a, st);
+}
+
+size_t up256(size_t n) { return (n + 255) & ~(size_t)255; }
+
+}  // namespace
+
+bool rows_gemm_ok(int qt, int K) {
+    return (qt == RINA_QT_Q4_0 || qt == RINA_QT_Q4_0F || qt == RINA_QT_GGML_Q2_K) && K % 32 == 0;
+}
+
+size_t rows_split_bytes(int qt, int rows, int K) {
+    const size_t mt = (rows + 15) / 16, nks = (size_t)(K + 127) / 128 * 4, ngw = (K + 511) / 512;
+    return up256(mt * nks * 2048) + up256(mt * 64) + (qt == RINA_QT_GGML_Q2_K ? mt * ngw * 3072 : 0);
+}
+
+int rows_split(int qt, const float* x, const int* src, int rows, int K, int pro, const float* nw, float eps, void* buf,
+               RowsX* out, hipStream_t st) {
+    const int mt = (rows + 15) / 16;
+    SplitXArgs a{};
+    a.x = x; a.nw = nw; a.src = src; a.M = rows; a.K = K; a.pro = pro; a.eps = eps;
+    a.nks = (K + 127) / 128 * 4;
+    a.ngw = (K + 511) / 512;
+    a.xp = (uint4*)buf;
+    a.xs = (float*)((char*)buf + up256((size_t)mt * a.nks * 2048));
+    a.xg = (uint16_t*)((char*)a.xs + up256((size_t)mt * 64));
+    const dim3 grid(mt * 16 / kSplitRows), blk(256 * kSplitRows);
+    const int nu = (K + 2047) / 2048;
+#define X_SPLIT(Q) \
+    do { if (nu <= 1) hipLaunchKernelGGL((x_split_kernel<Q, 1>), grid, blk, 0, st, a); \
+         else if (nu <= 2) hipLaunchKernelGGL((x_split_kernel<Q, 2>), grid, blk, 0, st, a); \
+         else if (nu <= 4) hipLaunchKernelGGL((x_split_kernel<Q, 4>), grid, blk, 0, st, a); \
+         else if (nu <= 6) hipLaunchKernelGGL((x_split_kernel<Q, 6>), grid, blk, 0, st, a); \
+         else hipLaunchKernelGGL((x_split_kernel<Q, 0>), grid, blk, 0, st, a); } while (0)
+    if (qt == RINA_QT_GGML_Q2_K) X_SPLIT(true);
+    else X_SPLIT(false);
+#undef X_SPLIT
+    out->xp = a.xp;
+    out->xs = a.xs;
+    out->xg = a.xg;
+    out->rows = rows;
+    out->K = K;
+    return hipGetLastError() == hipSuccess ? RINA_OK : RINA_ERR_HIP;
+}
+
+int rows_gemm(const rina_linear_seg* segs, int nseg, int qt, const RowsX& x, int epi, const int* plan, int64_t stride,
+              int rt_plan, hipStream_t st) {
+    const bool two = epi == RINA_EPI_SWIGLU;
+    const int nmat = two ? 2 : 1;
+    RowsArgs a{};
+    a.xp = (const uint4*)x.xp; a.xs = x.xs; a.xg = (const uint4*)x.xg;
+    a.M = x.rows; a.K = x.K; a.epi = epi; a.nseg = nseg;
+    a.nks = (x.K + 127) / 128 * 4;
+    a.ngw = (x.K + 511) / 512;
+    a.w2 = two ? (const uint8_t*)segs[0].weight2 : nullptr;
+    a.plan = plan;
+    a.stride = stride;
+    const int nss = a.nks / 4;
+    // row tiles of 16, 32 or 64 rows (rt 0, 1, 2); columns per wave: 16, or 32 ct at 64 rows
+    const int rt = plan ? rt_plan : x.rows <= 16 ? 0 : x.rows <= 32 ? 1 : 2;
+    const int tr = 16 << rt, tc = rt < 2 ? 16 : 32;
+    const int64_t mts = (x.rows + tr - 1) / tr;
+    auto tiles = [&](int ct) {
+        int64_t t = 0;
+        for (int s = 0; s < nseg; s++) t += (segs[s].N + tc * ct - 1) / (tc * ct);
+        return t * mts;
+    };
+    // K slices until there are two waves per SIMD; 64 columns per wave only
+    // where that leaves every SIMD a wave without splitting K
+    const int64_t simds = 4LL * rina_num_cus();
+    const int nj = nmat == 1 && rt == 2 && tiles(2) >= simds ? 2 : 1;
+    int kw = 1;
+    while (kw < 8 && tiles(nj) * kw < 2 * simds && nss >= 2 * kw) kw *= 2;
+    a.KW = kw;
+    a.NW = kw >= 4 ? 1 : 4 / kw;
+    const int BN = tc * nj * a.NW;
+    int t = 0;
+    for (int s = 0; s < 3; s++) {
+        const int ss = s < nseg ? s : 0;
+        a.w[s] = (const uint8_t*)segs[ss].weight;
+        a.y[s] = segs[ss].out;
+        a.N[s] = segs[ss].N;
+        a.t0[s] = s < nseg ? t : 1 << 30;
+        if (s < nseg) t += (segs[s].N + BN - 1) / BN;
+    }
+    a.mt = (int)mts;
+    a.nt = t;
+    // XCD split with the fewest bytes fetched by the 8 L2s: xb x + (8 / xb) W
+    // (grouped rows: every group's weights on one XCD)
+    const double xbytes = 4.0 * x.rows * x.K;
+    const double wbytes = (double)nmat * BN * t * x.K * (qt == RINA_QT_Q4_0F ? 0.625 : qt == RINA_QT_GGML_Q2_K ? 84.0 / 256 : 0.5625);
+    int best = 1;
+    if (!plan)
+        for (int xb = 2; xb <= 8; xb *= 2)
+            if (xb * xbytes + (8 / xb) * wbytes < best * xbytes + (8 / best) * wbytes) best = xb;
+    a.xb = best;
+    a.mpp = (a.mt + 8 / best - 1) / (8 / best);
+    a.npp = (t + best - 1) / best;
+    if (qt == RINA_QT_Q4_0) return launch_fmt<FMT_Q4_0>(a, nmat, rt, nj, st);
+    if (qt == RINA_QT_Q4_0F) return launch_fmt<FMT_Q4_0F>(a, nmat, rt, nj, st);
+    return x.K % 128 == 0 ? launch_fmt<FMT_Q2_K>(a, nmat, rt, nj, st) : launch_fmt<FMT_Q2_S>(a, nmat, rt, nj, st);
+}

@@ -18,6 +18,7 @@
 #include <type_traits>
 #include "rina_common.hpp"
 #include "q2k_col.hpp"
+#include "rows_gemm.hpp"
 
 namespace {
 
@@ -1030,426 +1031,6 @@ __global__ __launch_bounds__(256) void gemm_tile_kernel(GemmArgs a) {
 }
 
 // ---------------------------------------------------------------------------
-// M >= 16 with Q4 weights on the matrix cores (prompt phase):
-// v_mfma_f32_16x16x4f32 over BM x 64 output tiles (BM 64, or 32 when 64-row
-// tiles would leave fewer than two workgroups per CU), K stepped by one
-// 32-value block.  The x tile and the dequantized weight tile ((q - 7) * scale, the
-// reference dequant's per-element value) sit in LDS as fp32, K-major with a
-// row stride of 80 floats (a 64-lane fragment read touches every bank
-// twice), so each product is the reference's fp32 product and the matrix
-// cores accumulate in fp32 (the sums in another order).  Wave w owns the
-// (BM / 2) x 32 quarter (w / 2, w % 2) as (BM / 32) x 2 MFMA tiles per
-// matrix; the next
-// block's x values and weight bytes are loaded into registers while the
-// current block is multiplied.
-// MFMA operand layout (16x16x4 f32): lane l supplies A[l % 16][l / 16] and
-// B[l / 16][l % 16]; result element e of lane l is D[4 (l / 16) + e][l % 16].
-// ---------------------------------------------------------------------------
-typedef float f32x4m __attribute__((ext_vector_type(4)));
-
-constexpr int kMfmaLd = 80;
-
-// Up to 3 weight segments sharing x (q / k / v) in one launch: column
-// tiles t0[s] .. of segment s, in order.
-// XCD-aware tile order: workgroups go to the 8 XCDs round-robin in linear
-// order, so workgroup id serves XCD id % 8.  The x rows are split into xa
-// parts and the weight columns into xb parts (xa * xb = 8); XCD x takes
-// m-tiles of part x / xb and n-tiles of part x % xb, so each L2 fetches
-// 1/xa of the activation tiles and 1/xb of the weight tiles (the host
-// picks the split with the fewest bytes fetched).
-struct MfmaArgs {
-    GemmArgs g;                  // g.w / g.w2 / g.y / g.N: segment 0
-    const uint8_t* w[3];
-    float* y[3];
-    int N[3];
-    int t0[3];
-    int nseg;
-    int mt, nt;                  // m-tiles, n-tiles
-    int xb;                      // weight parts (8 / xb activation parts)
-    int mpp, npp;                // m-tiles, n-tiles per part
-};
-
-template <int FMT, int NMAT, int BM>
-__global__ __launch_bounds__(256) void gemm_mfma_kernel(MfmaArgs ma) {
-    constexpr int BB = FMT == FMT_Q4_0F ? 20 : 18;
-    constexpr int MI = BM / 32;                    // MFMA tiles per wave along M
-    __shared__ float xs[32][kMfmaLd];
-    __shared__ float ws[NMAT][32][kMfmaLd];
-    const int tid = threadIdx.x, lane = tid & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    // this workgroup's tile: XCD id % 8 owns activation part (id % 8) / xb
-    // and weight part (id % 8) % xb
-    const int xcd = blockIdx.x & 7, k = blockIdx.x >> 3;
-    const int mm = k / ma.npp, nn = k - mm * ma.npp;
-    const int by = (xcd / ma.xb) * ma.mpp + mm, bx = (xcd % ma.xb) * ma.npp + nn;
-    if (mm >= ma.mpp || by >= ma.mt || bx >= ma.nt) return;   // padding of the split
-    // this workgroup's segment (wave-uniform selects, no indexed argument reads)
-    GemmArgs a = ma.g;
-    const int sg = (ma.nseg > 1 && bx >= ma.t0[1]) + (ma.nseg > 2 && bx >= ma.t0[2]);
-    a.w = sg == 0 ? ma.w[0] : sg == 1 ? ma.w[1] : ma.w[2];
-    a.y = sg == 0 ? ma.y[0] : sg == 1 ? ma.y[1] : ma.y[2];
-    a.N = sg == 0 ? ma.N[0] : sg == 1 ? ma.N[1] : ma.N[2];
-    const int tb = sg == 0 ? ma.t0[0] : sg == 1 ? ma.t0[1] : ma.t0[2];
-    const int m0 = by * BM, n0 = (bx - tb) * 64;
-    const int nb = a.K / 32;
-    // staging: thread t takes row t / 4 of the x tile (rows < BM) and of
-    // each weight tile, values 8 (t % 4) .. 8 (t % 4) + 7 of the block
-    const int sr = tid >> 2, sq = tid & 3;
-    const bool xok = sr < BM && m0 + sr < a.M, wok = n0 + sr < a.N;
-    const float* xrow = a.x + (int64_t)(xok ? m0 + sr : 0) * a.K + 8 * sq;
-    const int64_t wrow = (int64_t)(wok ? n0 + sr : 0) * nb * BB;
-    // Q2_K (flat element order): values 8 sq .. 8 sq + 7 of the row's block b
-    // are elements e = row K + 32 b + 8 sq, inside one 256-value block and
-    // one shift group g of one 128-value page (row starts and b are
-    // multiples of 32): qs bytes 16 + 32 page + 8 sq .. + 7, scale byte
-    // 8 page + sq / 2 + 2 g, fp16 d / dmin at 80 / 82
-    const int64_t erow = (int64_t)(wok ? n0 + sr : 0) * a.K + 8 * sq;
-    f32x4 xr0, xr1;
-    uint32_t wsc[NMAT], wnb[NMAT], wq1[NMAT], wdd[NMAT];
-    auto load_blk = [&](int b) {
-        const f32x4* xp = (const f32x4*)(xrow + 32 * b);
-        xr0 = gld(xp);
-        xr1 = gld(xp + 1);
-#pragma unroll
-        for (int m = 0; m < NMAT; m++) {
-            if constexpr (FMT == FMT_Q2_K) {
-                const int64_t e = erow + 32 * b;
-                const uint8_t* bd = (m ? a.w2 : a.w) + (e >> 8) * 84;
-                const int inb = (int)(e & 255), page = inb >> 7, g = (inb & 127) >> 5;
-                const int is = 8 * page + (sq >> 1) + 2 * g;
-                wnb[m] = gld((const uint32_t*)(bd + 16 + 32 * page + 8 * sq));
-                wq1[m] = gld((const uint32_t*)(bd + 20 + 32 * page + 8 * sq));
-                wsc[m] = ((gld((const uint32_t*)(bd + (is & ~3))) >> (8 * (is & 3))) & 0xFF) | ((uint32_t)(2 * g) << 8);
-                wdd[m] = gld((const uint32_t*)(bd + 80));
-            } else {
-                const uint8_t* bp = (m ? a.w2 : a.w) + wrow + (int64_t)b * BB;
-                if constexpr (FMT == FMT_Q4_0F) {
-                    wsc[m] = gld((const uint32_t*)bp);
-                    wnb[m] = gld((const uint32_t*)(bp + 4 + 4 * sq));
-                } else {
-                    wsc[m] = gld((const uint16_t*)bp);
-                    wnb[m] = (uint32_t)gld((const uint16_t*)(bp + 2 + 4 * sq)) |
-                             ((uint32_t)gld((const uint16_t*)(bp + 4 + 4 * sq)) << 16);
-                }
-            }
-        }
-    };
-    // value 8 sq + t of the block is nibble t of wnb (byte t / 2, low nibble for even t)
-    auto store_blk = [&]() {
-        const float xv[8] = {xr0.x, xr0.y, xr0.z, xr0.w, xr1.x, xr1.y, xr1.z, xr1.w};
-        if (sr < BM) {
-#pragma unroll
-            for (int t = 0; t < 8; t++) xs[8 * sq + t][sr] = xok ? xv[t] : 0.f;
-        }
-#pragma unroll
-        for (int m = 0; m < NMAT; m++) {
-            if constexpr (FMT == FMT_Q2_K) {
-                // ops/linear.cu:413-431: d * (sc & 15) * q - dmin * (sc >> 4)
-                const uint32_t sc = wsc[m] & 0xFF, sh = wsc[m] >> 8;
-                const float dv = f16_to_f32((uint16_t)(wdd[m] & 0xFFFF)), mv = f16_to_f32((uint16_t)(wdd[m] >> 16));
-                const float scale = dv * (float)(sc & 0xF), mn = mv * (float)(sc >> 4);
-#pragma unroll
-                for (int t = 0; t < 8; t++) {
-                    const uint32_t qb = ((t < 4 ? wnb[m] : wq1[m]) >> (8 * (t & 3))) & 0xFF;
-                    ws[m][8 * sq + t][sr] = wok ? fmaf(scale, (float)((qb >> sh) & 3), -mn) : 0.f;
-                }
-            } else {
-                const float sc = FMT == FMT_Q4_0F ? __uint_as_float(wsc[m]) : f16_to_f32((uint16_t)wsc[m]);
-#pragma unroll
-                for (int t = 0; t < 8; t++)
-                    ws[m][8 * sq + t][sr] = wok ? (float)((int)((wnb[m] >> (4 * t)) & 0xF) - 7) * sc : 0.f;
-            }
-        }
-    };
-    const int wm = (wave >> 1) * 16 * MI, wn = (wave & 1) * 32;
-    const int fr = lane & 15, fk = lane >> 4;
-    f32x4m acc[NMAT][MI][2];
-#pragma unroll
-    for (int m = 0; m < NMAT; m++)
-#pragma unroll
-        for (int i = 0; i < MI; i++)
-#pragma unroll
-            for (int j = 0; j < 2; j++) acc[m][i][j] = f32x4m{0.f, 0.f, 0.f, 0.f};
-    load_blk(0);
-    for (int b = 0; b < nb; b++) {
-        __syncthreads();                           // the previous block's fragments are read
-        store_blk();
-        __syncthreads();
-        load_blk(b + 1 < nb ? b + 1 : b);          // unconditional: the last block reloads itself
-#pragma unroll
-        for (int kk = 0; kk < 8; kk++) {
-            const int k = 4 * kk + fk;
-            float av[MI];
-#pragma unroll
-            for (int i = 0; i < MI; i++) av[i] = xs[k][wm + 16 * i + fr];
-#pragma unroll
-            for (int m = 0; m < NMAT; m++) {
-                const float b0 = ws[m][k][wn + fr], b1 = ws[m][k][wn + 16 + fr];
-#pragma unroll
-                for (int i = 0; i < MI; i++) {
-                    acc[m][i][0] = __builtin_amdgcn_mfma_f32_16x16x4f32(av[i], b0, acc[m][i][0], 0, 0, 0);
-                    acc[m][i][1] = __builtin_amdgcn_mfma_f32_16x16x4f32(av[i], b1, acc[m][i][1], 0, 0, 0);
-                }
-            }
-        }
-    }
-#pragma unroll
-    for (int i = 0; i < MI; i++)
-#pragma unroll
-        for (int j = 0; j < 2; j++)
-#pragma unroll
-            for (int e = 0; e < 4; e++) {
-                const int row = m0 + wm + 16 * i + 4 * fk + e, col = n0 + wn + 16 * j + fr;
-                if (row >= a.M || col >= a.N) continue;
-                float* y = a.y + (int64_t)row * a.N + col;
-                const float v0 = acc[0][i][j][e];
-                if (NMAT == 2) *y = silu_mul(v0, acc[NMAT - 1][i][j][e]);
-                else if (a.epi == RINA_EPI_ADD) *y = *y + v0;
-                else *y = v0;
-            }
-}
-
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-
-// the high halves of two fp32 bit patterns as one dword of two bf16 (a's in
-// the low half)
-__device__ __forceinline__ uint32_t hi16_pair(uint32_t a, uint32_t b) { return __builtin_amdgcn_perm(b, a, 0x07060302u); }
-
-// x0, x1 split into three bf16 parts each, x = h + m + l: h is x cut to its
-// top 8 significant bits, m the remainder cut the same way, l the rest (at
-// most 8 significant bits); packed as two-value dwords.  Exact for finite
-// |x| >= 2^-103 and for 0, where both remainders are normal fp32 values; an
-// infinite x gives NaN parts (inf - inf), and a smaller x loses low bits of
-// l (the matrix cores may also flush bf16 denormals)
-__device__ __forceinline__ void split3_pair(float x0, float x1, uint32_t& ph, uint32_t& pm, uint32_t& pl) {
-    const uint32_t u0 = __float_as_uint(x0), u1 = __float_as_uint(x1);
-    ph = hi16_pair(u0, u1);
-    const float r0 = x0 - __uint_as_float(u0 & 0xFFFF0000u), r1 = x1 - __uint_as_float(u1 & 0xFFFF0000u);
-    const uint32_t v0 = __float_as_uint(r0), v1 = __float_as_uint(r1);
-    pm = hi16_pair(v0, v1);
-    const float s0 = r0 - __uint_as_float(v0 & 0xFFFF0000u), s1 = r1 - __uint_as_float(v1 & 0xFFFF0000u);
-    pl = hi16_pair(__float_as_uint(s0), __float_as_uint(s1));
-}
-
-// Prompt matmul for Q4_0 / Q4_0F weights on the bf16 matrix cores, with fp32
-// products and sums.  Every x value is split exactly into three bf16 parts,
-// x = h + m + l (8 significant bits each: the two remainders are exact in
-// fp32), and a weight value q - 7 is a small integer, exact in bf16, so
-// v_mfma_f32_16x16x32_bf16 forms the exact products of the fp32 x with the
-// integer weights and sums them in fp32.  Per 32-value block and 16x16 tile
-// three MFMAs (l, m, h into one accumulator), then one fp32 fma with the
-// block scale of the tile column.  XCD order, segments and epilogues as
-// gemm_mfma_kernel; tiles are BM x 32 WN with 2 WN waves (two down the rows,
-// WN across, each wave 16 MI rows x 32 columns), so one split of an x tile
-// serves 32 WN columns.  LDS rows of (32 * KB + 8) bf16 keep the 16-byte
-// fragment reads of 16 rows on distinct banks.  Fragment layout (16x16x32): lane l holds
-// A[l % 16][8 (l / 16) .. + 7], B[8 (l / 16) .. + 7][l % 16] and
-// D[4 (l / 16) + e][l % 16].
-template <int FMT, int NMAT, int BM, int WN>
-__global__ __launch_bounds__(128 * WN) void gemm_bf3_kernel(MfmaArgs ma) {
-    constexpr int BB = FMT == FMT_Q4_0F ? 20 : 18;
-    constexpr int MI = BM / 32;                    // MFMA tiles per wave along M
-    // 32-value blocks per LDS stage: four cut the barriers of the one-matrix
-    // launches (two at 64 rows, whose LDS would otherwise hold one
-    // workgroup per CU); the paired SwiGLU tile keeps one (its registers
-    // would cut occupancy to 3 waves per SIMD)
-    constexpr int KB = NMAT == 2 ? 1 : BM == 64 ? 2 : 4;
-    constexpr int LD = 32 * KB + 8;
-    // WN waves across the tile's columns (32 each) and two down its rows
-    constexpr int BN = 32 * WN, NT = 128 * WN;
-    __shared__ __align__(16) uint16_t xs[3][BM][LD];
-    __shared__ __align__(16) uint16_t ws[NMAT][BN][LD];
-    __shared__ float wsc_s[NMAT][KB][BN];
-    const int tid = threadIdx.x, lane = tid & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int xcd = blockIdx.x & 7, k = blockIdx.x >> 3;
-    const int mm = k / ma.npp, nn = k - mm * ma.npp;
-    const int by = (xcd / ma.xb) * ma.mpp + mm, bx = (xcd % ma.xb) * ma.npp + nn;
-    if (mm >= ma.mpp || by >= ma.mt || bx >= ma.nt) return;   // padding of the split
-    GemmArgs a = ma.g;
-    const int sg = (ma.nseg > 1 && bx >= ma.t0[1]) + (ma.nseg > 2 && bx >= ma.t0[2]);
-    a.w = sg == 0 ? ma.w[0] : sg == 1 ? ma.w[1] : ma.w[2];
-    a.y = sg == 0 ? ma.y[0] : sg == 1 ? ma.y[1] : ma.y[2];
-    a.N = sg == 0 ? ma.N[0] : sg == 1 ? ma.N[1] : ma.N[2];
-    const int tb = sg == 0 ? ma.t0[0] : sg == 1 ? ma.t0[1] : ma.t0[2];
-    const int m0 = by * BM, n0 = (bx - tb) * BN;
-    const int nb = a.K / 32, nst = (nb + KB - 1) / KB;
-    // x staging: every thread splits XV values of one row per block (XT
-    // threads per row), so the split work is spread over all the waves;
-    // weight staging: thread tid takes values 8 sq .. 8 sq + 7 of column sr
-    constexpr int XV = BM * 32 / NT, XT = 32 / XV;
-    const int xsr = tid / XT, xsq = tid % XT;
-    const int sr = tid >> 2, sq = tid & 3;
-    const bool xok = m0 + xsr < a.M, wok = n0 + sr < a.N;
-    const float* xrow = a.x + (int64_t)(xok ? m0 + xsr : 0) * a.K + XV * xsq;
-    const int64_t wrow = (int64_t)(wok ? n0 + sr : 0) * nb * BB;
-    // register sets holding one stage's loads each; with two, a stage's loads
-    // are issued two stages before they are stored to LDS
-    struct Stage {
-        float xr[KB][XV];
-        uint32_t wsc[KB][NMAT], wnb[KB][NMAT];
-    };
-    Stage r0, r1;
-    // stage st: blocks KB st .. KB st + KB - 1 (past nb: block nb - 1 again,
-    // stored as zeros)
-    auto load_stage = [&](Stage& r, int st) {
-#pragma unroll
-        for (int kb = 0; kb < KB; kb++) {
-            const int b = min(KB * st + kb, nb - 1);
-            if constexpr (XV >= 4) {
-                const f32x4* xp = (const f32x4*)(xrow + 32 * b);
-#pragma unroll
-                for (int v = 0; v < XV / 4; v++) {
-                    const f32x4 t = gld(xp + v);
-                    r.xr[kb][4 * v] = t.x; r.xr[kb][4 * v + 1] = t.y; r.xr[kb][4 * v + 2] = t.z; r.xr[kb][4 * v + 3] = t.w;
-                }
-            } else {
-                const f32x2 t = gld((const f32x2*)(xrow + 32 * b));
-                r.xr[kb][0] = t.x; r.xr[kb][1] = t.y;
-            }
-#pragma unroll
-            for (int m = 0; m < NMAT; m++) {
-                const uint8_t* bp = (m ? a.w2 : a.w) + wrow + (int64_t)b * BB;
-                if constexpr (FMT == FMT_Q4_0F) {
-                    r.wsc[kb][m] = gld((const uint32_t*)bp);
-                    r.wnb[kb][m] = gld((const uint32_t*)(bp + 4 + 4 * sq));
-                } else {
-                    r.wsc[kb][m] = gld((const uint16_t*)bp);
-                    r.wnb[kb][m] = (uint32_t)gld((const uint16_t*)(bp + 2 + 4 * sq)) |
-                                 ((uint32_t)gld((const uint16_t*)(bp + 4 + 4 * sq)) << 16);
-                }
-            }
-        }
-    };
-    // value 8 sq + t of a block is nibble t of wnb (byte t / 2, low nibble for even t)
-    auto store_stage = [&](const Stage& r, int st) {
-#pragma unroll
-        for (int kb = 0; kb < KB; kb++) {
-            const bool bok = KB * st + kb < nb;
-            {
-                float xv[XV];
-#pragma unroll
-                for (int v = 0; v < XV; v++) xv[v] = r.xr[kb][v];
-                const bool on = xok && bok;
-                uint32_t ph[XV / 2], pm[XV / 2], pl[XV / 2];
-#pragma unroll
-                for (int t = 0; t < XV; t += 2)
-                    split3_pair(on ? xv[t] : 0.f, on ? xv[t + 1] : 0.f, ph[t >> 1], pm[t >> 1], pl[t >> 1]);
-                uint16_t* d0 = &xs[0][xsr][32 * kb + XV * xsq];
-                uint16_t* d1 = &xs[1][xsr][32 * kb + XV * xsq];
-                uint16_t* d2 = &xs[2][xsr][32 * kb + XV * xsq];
-                if constexpr (XV == 8) {
-                    *(u32x4*)d0 = u32x4{ph[0], ph[1], ph[2], ph[3]};
-                    *(u32x4*)d1 = u32x4{pm[0], pm[1], pm[2], pm[3]};
-                    *(u32x4*)d2 = u32x4{pl[0], pl[1], pl[2], pl[3]};
-                } else if constexpr (XV == 2) {
-                    *(uint32_t*)d0 = ph[0];
-                    *(uint32_t*)d1 = pm[0];
-                    *(uint32_t*)d2 = pl[0];
-                } else {
-                    *(u32x2*)d0 = u32x2{ph[0], ph[1]};
-                    *(u32x2*)d1 = u32x2{pm[0], pm[1]};
-                    *(u32x2*)d2 = u32x2{pl[0], pl[1]};
-                }
-            }
-#pragma unroll
-            for (int m = 0; m < NMAT; m++) {
-                // q - 7 as bf16, a small integer (exact): nibble t of wnb is
-                // byte t / 2 of lo (even t) or hi (odd t)
-                const uint32_t lo = and_opaque(r.wnb[kb][m], 0x0F0F0F0Fu), hi = and_opaque(r.wnb[kb][m] >> 4, 0x0F0F0F0Fu);
-                uint32_t pw[4];
-#pragma unroll
-                for (int j = 0; j < 4; j++) {
-                    const float f0 = (float)((lo >> (8 * j)) & 0xFF) - 7.0f, f1 = (float)((hi >> (8 * j)) & 0xFF) - 7.0f;
-                    pw[j] = wok && bok ? hi16_pair(__float_as_uint(f0), __float_as_uint(f1)) : 0u;
-                }
-                *(u32x4*)&ws[m][sr][32 * kb + 8 * sq] = u32x4{pw[0], pw[1], pw[2], pw[3]};
-                if (sq == 0) {
-                    const float sc = FMT == FMT_Q4_0F ? __uint_as_float(r.wsc[kb][m]) : f16_to_f32((uint16_t)r.wsc[kb][m]);
-                    wsc_s[m][kb][sr] = wok && bok ? sc : 0.f;
-                }
-            }
-        }
-    };
-    const int wm = (wave / WN) * 16 * MI, wn = (wave % WN) * 32;
-    const int fr = lane & 15, fk = lane >> 4;
-    f32x4m acc[NMAT][MI][2];
-#pragma unroll
-    for (int m = 0; m < NMAT; m++)
-#pragma unroll
-        for (int i = 0; i < MI; i++)
-#pragma unroll
-            for (int j = 0; j < 2; j++) acc[m][i][j] = f32x4m{0.f, 0.f, 0.f, 0.f};
-    auto compute_stage = [&]() {
-#pragma unroll
-        for (int kb = 0; kb < KB; kb++) {
-            bf16x8 af[3][MI];
-#pragma unroll
-            for (int p = 0; p < 3; p++)
-#pragma unroll
-                for (int i = 0; i < MI; i++) af[p][i] = *(const bf16x8*)&xs[p][wm + 16 * i + fr][32 * kb + 8 * fk];
-#pragma unroll
-            for (int m = 0; m < NMAT; m++)
-#pragma unroll
-                for (int j = 0; j < 2; j++) {
-                    const bf16x8 bf = *(const bf16x8*)&ws[m][wn + 16 * j + fr][32 * kb + 8 * fk];
-                    const float sc = wsc_s[m][kb][wn + 16 * j + fr];
-#pragma unroll
-                    for (int i = 0; i < MI; i++) {
-                        f32x4m d = __builtin_amdgcn_mfma_f32_16x16x32_bf16(af[2][i], bf, f32x4m{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
-                        d = __builtin_amdgcn_mfma_f32_16x16x32_bf16(af[1][i], bf, d, 0, 0, 0);
-                        d = __builtin_amdgcn_mfma_f32_16x16x32_bf16(af[0][i], bf, d, 0, 0, 0);
-#pragma unroll
-                        for (int e = 0; e < 4; e++) acc[m][i][j][e] = fmaf(sc, d[e], acc[m][i][j][e]);
-                    }
-                }
-        }
-    };
-    load_stage(r0, 0);
-    if constexpr (NMAT == 1) {
-        // stages in pairs, unconditionally: with nst odd the last pair's
-        // second stage lies past nb, is stored as zeros and adds sc 0 times d 0
-        load_stage(r1, 1);
-        for (int st = 0; st < nst; st += 2) {
-            __syncthreads();                       // the previous stage's fragments are read
-            store_stage(r0, st);
-            __syncthreads();
-            load_stage(r0, st + 2);
-            compute_stage();
-            __syncthreads();
-            store_stage(r1, st + 1);
-            __syncthreads();
-            load_stage(r1, st + 3);
-            compute_stage();
-        }
-    } else {
-        // the paired SwiGLU tile keeps one register set (a second would cut
-        // occupancy from 5 to 3 waves per SIMD, which costs it more)
-        for (int st = 0; st < nst; st++) {
-            __syncthreads();
-            store_stage(r0, st);
-            __syncthreads();
-            load_stage(r0, st + 1);                // past the end: block nb - 1, not stored
-            compute_stage();
-        }
-    }
-#pragma unroll
-    for (int i = 0; i < MI; i++)
-#pragma unroll
-        for (int j = 0; j < 2; j++)
-#pragma unroll
-            for (int e = 0; e < 4; e++) {
-                const int row = m0 + wm + 16 * i + 4 * fk + e, col = n0 + wn + 16 * j + fr;
-                if (row >= a.M || col >= a.N) continue;
-                float* y = a.y + (int64_t)row * a.N + col;
-                const float v0 = acc[0][i][j][e];
-                if (NMAT == 2) *y = silu_mul(v0, acc[NMAT - 1][i][j][e]);
-                else if (a.epi == RINA_EPI_ADD) *y = *y + v0;
-                else *y = v0;
-            }
-}
-
-// ---------------------------------------------------------------------------
 // host side
 // ---------------------------------------------------------------------------
 
@@ -1789,85 +1370,7 @@ int gemv_f32(const rina_linear_seg* segs, int nseg, const float* x, int K, int e
     return hipGetLastError() == hipSuccess ? RINA_OK : RINA_ERR_HIP;
 }
 
-bool mfma_ok(int qt, const float* x, int M, int K) {
-    return M >= 16 && (qt == RINA_QT_Q4_0 || qt == RINA_QT_Q4_0F || qt == RINA_QT_GGML_Q2_K) && K % 32 == 0 &&
-           (uintptr_t)x % 16 == 0;
-}
-
-// Matrix-core prompt matmul over up to 3 segments sharing x (one launch).
-int gemm_mfma(const rina_linear_seg* segs, int nseg, int qt, const float* x, int M, int K, int epi, hipStream_t st) {
-    MfmaArgs ma{};
-    ma.g = GemmArgs{(const uint8_t*)segs[0].weight, epi == RINA_EPI_SWIGLU ? (const uint8_t*)segs[0].weight2 : nullptr,
-                    x, segs[0].out, M, segs[0].N, K, qt, epi};
-    ma.nseg = nseg;
-    const bool two = epi == RINA_EPI_SWIGLU;
-    // Q4 launches take 128-column tiles of eight waves (the x tile's split
-    // and staging then serve twice the columns) when those tiles fill the
-    // CUs in whole rounds, else 64-column tiles of four waves (q/k/v at M
-    // 512: 384 wide tiles would leave half the CUs a second one); Q2_K
-    // 64-column tiles
-    auto count = [&](int bn) {
-        int t = 0;
-        for (int s = 0; s < nseg; s++) t += (segs[s].N + bn - 1) / bn;
-        return t;
-    };
-    const bool half = (int64_t)count(64) * ((M + 63) / 64) < 2LL * rina_num_cus();   // 32-row tiles: more workgroups in flight
-    const int64_t mtiles = half ? (M + 31) / 32 : (M + 63) / 64;
-    const bool wide = qt != RINA_QT_GGML_Q2_K && mtiles * count(128) % rina_num_cus() == 0;
-    const int BN = wide ? 128 : 64;
-    int tiles = 0;
-    for (int s = 0; s < 3; s++) {
-        const int ss = s < nseg ? s : 0;
-        ma.w[s] = (const uint8_t*)segs[ss].weight;
-        ma.y[s] = segs[ss].out;
-        ma.N[s] = segs[ss].N;
-        ma.t0[s] = s < nseg ? tiles : 1 << 30;
-        if (s < nseg) tiles += (segs[s].N + BN - 1) / BN;
-    }
-    ma.mt = half ? (M + 31) / 32 : (M + 63) / 64;
-    ma.nt = tiles;
-    // bytes the 8 L2s fetch for a split of x into 8 / xb parts and the
-    // weights into xb parts: xb * (x bytes) + (8 / xb) * (weight bytes)
-    const double xbytes = 4.0 * M * K;
-    const double wbytes = (two ? 2.0 : 1.0) * BN * (double)tiles * K *
-                          (qt == RINA_QT_Q4_0F ? 20.0 / 32 : qt == RINA_QT_GGML_Q2_K ? 84.0 / 256 : 18.0 / 32);
-    int best = 1;
-    for (int xb = 2; xb <= 8; xb *= 2)
-        if (xb * xbytes + (8 / xb) * wbytes < best * xbytes + (8 / best) * wbytes) best = xb;
-    ma.xb = best;
-    ma.mpp = (ma.mt + 8 / best - 1) / (8 / best);
-    ma.npp = (tiles + best - 1) / best;
-    const dim3 g(8 * ma.mpp * ma.npp);
-#define MFMA_LAUNCH(KN, F, NM) \
-    do { if (half) hipLaunchKernelGGL((KN<F, NM, 32>), g, dim3(256), 0, st, ma); \
-         else hipLaunchKernelGGL((KN<F, NM, 64>), g, dim3(256), 0, st, ma); } while (0)
-    // Q4 weights: bf16 matrix cores on exact three-part splits of x; Q2_K
-    // (weights d sc q - dmin m, not small integers): fp32 matrix cores
-#define BF3_WN(F, NM, WN) \
-    do { if (half) hipLaunchKernelGGL((gemm_bf3_kernel<F, NM, 32, WN>), g, dim3(128 * WN), 0, st, ma); \
-         else hipLaunchKernelGGL((gemm_bf3_kernel<F, NM, 64, WN>), g, dim3(128 * WN), 0, st, ma); } while (0)
-#define BF3_LAUNCH(F, NM) \
-    do { if (wide) BF3_WN(F, NM, 4); else BF3_WN(F, NM, 2); } while (0)
-    if (qt == RINA_QT_GGML_Q2_K) {
-        if (two) MFMA_LAUNCH(gemm_mfma_kernel, FMT_Q2_K, 2);
-        else MFMA_LAUNCH(gemm_mfma_kernel, FMT_Q2_K, 1);
-    } else if (qt == RINA_QT_Q4_0F) {
-        if (two) BF3_LAUNCH(FMT_Q4_0F, 2);
-        else BF3_LAUNCH(FMT_Q4_0F, 1);
-    } else {
-        if (two) BF3_LAUNCH(FMT_Q4_0, 2);
-        else BF3_LAUNCH(FMT_Q4_0, 1);
-    }
-#undef BF3_LAUNCH
-#undef BF3_WN
-#undef MFMA_LAUNCH
-    return hipGetLastError() == hipSuccess ? RINA_OK : RINA_ERR_HIP;
-}
-
 int gemm_tiled(const rina_linear_seg& seg, int qt, const float* x, int M, int K, int epi, hipStream_t st) {
-    // matrix cores for prompt-sized M and Q4 / Q2_K weights (K % 32 == 0, x
-    // rows 16-byte aligned; weights 4-byte aligned)
-    if (mfma_ok(qt, x, M, K)) return gemm_mfma(&seg, 1, qt, x, M, K, epi, st);
     GemmArgs a{(const uint8_t*)seg.weight, epi == RINA_EPI_SWIGLU ? (const uint8_t*)seg.weight2 : nullptr,
                x, seg.out, M, seg.N, K, qt, epi};
     dim3 grid((seg.N + 63) / 64, (M + 31) / 32);
@@ -1897,6 +1400,16 @@ extern "C" int rina_hip_linear_fused_ex(const rina_linear_seg* segs, int nseg, i
         if ((uintptr_t)segs[s].weight % 4 || (segs[s].weight2 && (uintptr_t)segs[s].weight2 % 4)) return RINA_ERR_ARG;
     }
     hipStream_t st = as_stream(stream);
+    if (M > 1 && rows_gemm_ok(qt, K)) {
+        // several rows: split once (with the prologue), then 3 segments per launch
+        void* buf = rina_scratch(rows_split_bytes(qt, M, K), st, kScratchRows);
+        if (!buf) return RINA_ERR_HIP;
+        RowsX xr;
+        int rc = rows_split(qt, input, nullptr, M, K, pro, nw, eps, buf, &xr, st);
+        for (int s0 = 0; s0 < nseg && rc == RINA_OK; s0 += 3)
+            rc = rows_gemm(segs + s0, nseg - s0 < 3 ? nseg - s0 : 3, qt, xr, epi, nullptr, 0, 0, st);
+        return rc;
+    }
     int unit = qt == RINA_QT_GGML_Q2_K ? 16 : 32;
     int wpr = 1, cpl = 1;
     if (qt != RINA_QT_FP32 && K % unit == 0) split_row(K / unit, wpr, cpl);
@@ -1910,7 +1423,7 @@ extern "C" int rina_hip_linear_fused_ex(const rina_linear_seg* segs, int nseg, i
     if (pro != RINA_PRO_NONE && (!fused_pro || (norm_out && !direct))) {
         // normalize first (into norm_out when given, else library scratch):
         // prompt rows, unusual shapes
-        float* tmp = norm_out ? norm_out : (float*)rina_scratch((size_t)M * K * 4, as_stream(stream));
+        float* tmp = norm_out ? norm_out : (float*)rina_scratch((size_t)M * K * 4, as_stream(stream), kScratchNorm);
         if (!tmp) return RINA_ERR_HIP;
         int rc = pro == RINA_PRO_RMSNORM ? rina_hip_rms_norm(input, tmp, nw, M, K, eps, stream)
                                          : rina_hip_layer_norm(input, tmp, nw, M, K, eps, stream);
@@ -1928,7 +1441,6 @@ extern "C" int rina_hip_linear_fused_ex(const rina_linear_seg* segs, int nseg, i
         return RINA_OK;
     }
     if (M > 1) {
-        if (mfma_ok(qt, input, M, K)) return gemm_mfma(segs, nseg, qt, input, M, K, epi, st);   // nseg <= 3 here
         for (int s = 0; s < nseg; s++) {
             int rc = gemm_tiled(segs[s], qt, input, M, K, epi, st);
             if (rc) return rc;
@@ -1977,7 +1489,7 @@ extern "C" int rina_hip_linear(const void* weight, int qt, const float* input, f
     bool alias = ib < oe && ob < ie;
     float* dst = output;
     if (alias) {
-        dst = (float*)rina_scratch((size_t)M * N * 4, st);
+        dst = (float*)rina_scratch((size_t)M * N * 4, st, kScratchOut);
         if (!dst) return RINA_ERR_HIP;
     }
     rina_linear_seg seg{weight, nullptr, dst, N};

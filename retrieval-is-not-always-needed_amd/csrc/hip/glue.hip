@@ -256,7 +256,7 @@ std::mutex g_mu;
 // one may still be read by queued work, so it is kept (retired) until the
 // process ends: at most log2 of the largest request buffers per stream.
 struct ScratchSlot {
-    int dev;
+    int dev, use;
     hipStream_t st;
     void* p;
     size_t bytes;
@@ -277,24 +277,35 @@ int rina_num_cus() {
     return g_dev[dev].cus;
 }
 
-void* rina_scratch(size_t bytes, hipStream_t st) {
+// hipMalloc that a stream capture of the calling thread does not forbid (the
+// buffer outlives the graph: it is never freed)
+static void* alloc_scratch(size_t bytes) {
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+    const bool swapped = hipThreadExchangeStreamCaptureMode(&mode) == hipSuccess;
+    void* p = nullptr;
+    if (hipMalloc(&p, bytes) != hipSuccess) p = nullptr;
+    if (swapped) (void)hipThreadExchangeStreamCaptureMode(&mode);
+    return p;
+}
+
+void* rina_scratch(size_t bytes, hipStream_t st, int use) {
     int dev = 0;
     if (hipGetDevice(&dev) != hipSuccess || dev < 0) return nullptr;
     std::lock_guard<std::mutex> lk(g_mu);
     for (ScratchSlot& s : g_scratch) {
-        if (s.dev != dev || s.st != st) continue;
+        if (s.dev != dev || s.st != st || s.use != use) continue;
         if (s.bytes >= bytes) return s.p;
         size_t nb = bytes > 2 * s.bytes ? bytes : 2 * s.bytes;
-        void* p = nullptr;
-        if (hipMalloc(&p, nb) != hipSuccess) return nullptr;
+        void* p = alloc_scratch(nb);
+        if (!p) return nullptr;
         g_retired.push_back(s.p);
         s.p = p;
         s.bytes = nb;
         return p;
     }
-    void* p = nullptr;
-    if (hipMalloc(&p, bytes) != hipSuccess) return nullptr;
-    g_scratch.push_back({dev, st, p, bytes});
+    void* p = alloc_scratch(bytes);
+    if (!p) return nullptr;
+    g_scratch.push_back({dev, use, st, p, bytes});
     return p;
 }
 

@@ -180,10 +180,14 @@ static inline hipStream_t as_stream(void* s) { return (hipStream_t)s; }
 // Number of compute units of the current device (cached per device).
 int rina_num_cus();
 
-// Scratch owned by the library, one buffer per (device, stream), grown on
-// demand and never shrunk.  Used only where a caller aliases input and
-// output, and for a norm that runs before a matvec as its own launch.
-void* rina_scratch(size_t bytes, hipStream_t stream);
+// Scratch owned by the library, one buffer per (device, stream, use), grown
+// on demand and never shrunk: the output of a call that aliases input and
+// output, the row of a norm that runs before a matvec as its own launch, the
+// split activation rows of a product over several rows.  The uses of one call
+// nest, so each has a buffer of its own; calls on one stream run in order and
+// share them.
+enum { kScratchOut = 0, kScratchNorm = 1, kScratchRows = 2 };
+void* rina_scratch(size_t bytes, hipStream_t stream, int use);
 
 __device__ __forceinline__ int read_pos(int start_pos, const int* d_pos) {
     return start_pos + (d_pos ? *d_pos : 0);

@@ -1,0 +1,26 @@
+// Products over several activation rows (gemm.hip): split the rows once,
+// multiply them by one or more weight matrices.
+#pragma once
+#include "rina_common.hpp"
+
+// split rows in matrix-core fragment order, inside a caller's buffer
+struct RowsX {
+    const void* xp;
+    const float* xs;
+    const void* xg;
+    int rows, K;
+};
+
+// quant types and row lengths the products take (M >= 2 rows)
+bool rows_gemm_ok(int qt, int K);
+size_t rows_split_bytes(int qt, int rows, int K);
+// x [.., K] -> fragments in buf (rows_split_bytes, 256-byte aligned), with the
+// norm prologue; src != NULL: packed row r is x row src[r], a zero row where
+// src[r] < 0 (src holds whole 16-row tiles)
+int rows_split(int qt, const float* x, const int* src, int rows, int K, int pro, const float* nw, float eps, void* buf,
+               RowsX* out, hipStream_t st);
+// up to 3 segments of one quant type; plan != NULL: grouped rows, plan[0] row
+// tiles (16, 32 or 64 rows: rt_plan 0, 1, 2) in use, plan[1 + i] the group of tile i, whose
+// weights start group * stride bytes into the segment
+int rows_gemm(const rina_linear_seg* segs, int nseg, int qt, const RowsX& x, int epi, const int* plan, int64_t stride,
+              int rt_plan, hipStream_t st);
