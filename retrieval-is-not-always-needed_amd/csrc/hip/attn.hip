@@ -27,6 +27,7 @@
 // (the workgroup holding that position), replacing the separate append launch.
 #include "rina_common.hpp"
 #include "kv_formats.hpp"
+#include "attn_rows.hpp"
 #include <mutex>
 
 namespace {
@@ -831,7 +832,6 @@ struct DqArgs {
     uint8_t* ckq;                       // q2k_q1v: key content, q2_1 blocks [max_seq][Hkv][da/32]
     float* ckr;                         // q2k_q1v: key RoPE part, fp32 [max_seq][Hkv][db]
     uint8_t* cvq;                       // q2k_q1v: values, q1_0 records [max_seq][Hkv][dv/32]
-    float* out;                         // dq_prompt_kv_kernel: [T][H][dv]
     int H, Hkv, da, db, dv, start_pos, max_seq;
     const int* d_pos;
     float scale;
@@ -854,26 +854,6 @@ __device__ __forceinline__ float q1_0_dim(const uint8_t* row, int lane) {
 }
 
 constexpr int kDqChunk = 32;
-
-// grid H + Hkv: workgroup h < H builds query h; the rest append KV head h - H
-// Dim i (< da + db) of the row [xa | RoPE_hf(xb)] at position pos (tables
-// [max_seq][db/2], NULL: no rotation), the rotation in the reference's
-// fused-multiply form.  Every load is issued unconditionally (clamped
-// indices) so the caller's load counters stay exact.
-__device__ __forceinline__ float dq_dim(const float* xa, const float* xb, const float* tc, const float* ts, int da,
-                                        int db, int pos, int i) {
-    const int hb = db / 2;
-    const int j = i - da, pi = j < 0 ? 0 : (j >> 1 < hb ? j >> 1 : hb - 1);
-    const float va = gld(xa + (i < da ? i : da - 1));
-    const float* xbb = db > 0 ? xb : xa;
-    const float x0 = gld(xbb + (db > 0 ? 2 * pi : 0)), x1 = gld(xbb + (db > 0 ? 2 * pi + 1 : 0));
-    const bool rot = tc != nullptr && db > 0;
-    const float c = gld((rot ? tc : xbb) + (rot ? (int64_t)pos * hb + pi : 0));
-    const float sn = gld((rot ? ts : xbb) + (rot ? (int64_t)pos * hb + pi : 0));
-    const float cc = rot ? c : 1.0f, ss = rot ? sn : 0.0f;
-    const float vb = (j & 1) ? fmaf(x0, ss, x1 * cc) : fmaf(x0, cc, -(x1 * ss));
-    return i < da ? va : vb;
-}
 
 // A prompt's rows for the RINA-MLA attention over fp32 caches: grid
 // (T, H + Hkv), one workgroup per (row, head).  Query heads: [qa | HF-RoPE(qb)]
@@ -1012,13 +992,9 @@ __global__ __launch_bounds__(256) void dq_split_kernel(DqArgs a, SplitArgs p) {
 // (QKV 0) or the q2k_q1v cache (QKV 1).  dq_pack_rows_kernel, grid (T, Hkv),
 // one wave per (row, KV head): the row's key and value as
 // dq_split_kernel<QKV> appends them at its position (the same dims, lanes
-// and, packed, block codec).  dq_prompt_kv_kernel, grid (T, H), four waves
-// per (row, query head), after it: row t reads the positions before it from
-// the cache (as dq_split_kernel<QKV> reads them) and its own position from
-// its fp32 rows, as the decode step of that row would; each wave takes every
-// fourth position of each 32-position chunk with the running softmax (the
-// next chunk's loads issued before the current chunk is scored), then the
-// four waves merge and the row is normalized.
+// and, packed, block codec).  attn_rows (ROWS_DQ) then reads, for row t, the
+// positions before it from the cache and its own position from its fp32 rows,
+// as the decode step of that row would.
 template <int QKV>
 __global__ __launch_bounds__(64) void dq_pack_rows_kernel(DqArgs a) {
     const int lane = threadIdx.x, t = blockIdx.x, kvh = blockIdx.y;
@@ -1043,357 +1019,15 @@ __global__ __launch_bounds__(64) void dq_pack_rows_kernel(DqArgs a) {
     }
 }
 
-template <int QKV>
-__global__ __launch_bounds__(256) void dq_prompt_kv_kernel(DqArgs a) {
-    constexpr int PW = kDqChunk / 4;
-    __shared__ float s_o[4][64];
-    __shared__ float s_m[4], s_l[4];
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int t = blockIdx.x, h = blockIdx.y;
-    const int pos0 = a.start_pos + t, L = pos0 + 1;
-    const int dq = a.da + a.db, kvh = h / (a.H / a.Hkv);
-    const int i1 = lane + 64 < dq ? lane + 64 : dq - 1;
-    const bool hi = lane + 64 < dq;
-    const float* qa = a.qa + ((int64_t)t * a.H + h) * a.da;
-    const float* qb = a.qb + ((int64_t)t * a.H + h) * a.db;
-    const float* ka = a.ka + ((int64_t)t * a.Hkv + kvh) * a.da;
-    const float* kb = a.kb + ((int64_t)t * a.Hkv + kvh) * a.db;
-    const float q0 = dq_dim(qa, qb, a.qc, a.qs, a.da, a.db, pos0, lane);
-    const float q1v = dq_dim(qa, qb, a.qc, a.qs, a.da, a.db, pos0, i1);
-    const float kc0 = dq_dim(ka, kb, a.kc, a.ks, a.da, a.db, pos0, lane);
-    const float kc1v = dq_dim(ka, kb, a.kc, a.ks, a.da, a.db, pos0, i1);
-    const float vc = gld(a.v + ((int64_t)t * a.Hkv + kvh) * a.dv + lane);
-    const float q1 = hi ? q1v : 0.f, kc1 = hi ? kc1v : 0.f;
-    // the wave's positions j0 + wave + 4 i of a chunk; positions at or past
-    // pos0 read position 0's record (in the cache, never used)
-    auto load = [&](int j0, float (&x0)[PW], float (&x1)[PW], float (&xv)[PW]) {
-#pragma unroll
-        for (int i = 0; i < PW; i++) {
-            const int p = j0 + wave + 4 * i;
-            const int64_t r = (int64_t)(p < pos0 ? p : 0) * a.Hkv + kvh;
-            if (QKV == 0) {
-                x0[i] = gld(a.ck + r * dq + lane);
-                x1[i] = lane + 64 < dq ? gld(a.ck + r * dq + lane + 64) : 0.f;
-                xv[i] = gld(a.cv + r * a.dv + lane);
-            } else {
-                x0[i] = q2_1_dim(a.ckq + r * 20, lane);
-                x1[i] = lane < a.db ? gld(a.ckr + r * a.db + lane) : 0.f;
-                xv[i] = q1_0_dim(a.cvq + r * 12, lane);
-            }
-        }
-    };
-    const float sc2 = a.scale * 1.44269504088896341f;   // scores in base-2 units
-    float m = -INFINITY, l = 0.f, o = 0.f;
-    auto consume = [&](int j0, const float (&x0)[PW], const float (&x1)[PW], const float (&xv)[PW]) {
-#pragma unroll
-        for (int i = 0; i < PW; i++) {
-            const int p = j0 + wave + 4 * i;
-            const bool cur = p == pos0;                  // wave-uniform
-            const float kk0 = cur ? kc0 : x0[i], kk1 = cur ? kc1 : x1[i], vx = cur ? vc : xv[i];
-            const float sc = wave_sum(fmaf(q0, kk0, q1 * kk1)) * sc2;
-            if (p < L) {
-                const float mn = fmaxf(m, sc);
-                const float al = __builtin_amdgcn_exp2f(m - mn), pe = __builtin_amdgcn_exp2f(sc - mn);
-                l = fmaf(l, al, pe);
-                o = fmaf(o, al, pe * vx);
-                m = mn;
-            }
-        }
-    };
-    float kA[PW], rA[PW], vA[PW], kB[PW], rB[PW], vB[PW];
-    load(0, kA, rA, vA);
-    for (int j0 = 0;;) {
-        if (j0 + kDqChunk < L) {
-            load(j0 + kDqChunk, kB, rB, vB);
-            consume(j0, kA, rA, vA);
-        } else {
-            consume(j0, kA, rA, vA);
-            break;
-        }
-        j0 += kDqChunk;
-        if (j0 + kDqChunk < L) {
-            load(j0 + kDqChunk, kA, rA, vA);
-            consume(j0, kB, rB, vB);
-        } else {
-            consume(j0, kB, rB, vB);
-            break;
-        }
-        j0 += kDqChunk;
-    }
-    s_o[wave][lane] = o;
-    if (lane == 0) { s_m[wave] = m; s_l[wave] = l; }
-    __syncthreads();
-    if (wave == 0) {
-        float M = -INFINITY;
-#pragma unroll
-        for (int w = 0; w < 4; w++) M = fmaxf(M, s_m[w]);
-        float ot = 0.f, lt = 0.f;
-#pragma unroll
-        for (int w = 0; w < 4; w++) {
-            const float aw = s_m[w] == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(s_m[w] - M);
-            ot = fmaf(s_o[w][lane], aw, ot);
-            lt = fmaf(s_l[w], aw, lt);
-        }
-        gst(a.out + ((int64_t)t * a.H + h) * 64 + lane, ot / lt);   // pos0 itself is always counted: lt > 0
-    }
-}
-
 // ---------------------------------------------------------------------------
-// Generic causal kernel: any T, dh <= 256, pre-RoPE caches.  One wave per
+// Generic causal kernel: head widths other than 64 up to 256, and rows whose
+// alignment attn_rows does not take.  One wave per
 // (query head, query row); keys in order with the online normalized update
 // of flash_fp32.cu:55-81, parallel over dims.
 // ---------------------------------------------------------------------------
 __device__ __forceinline__ float cache_val(int fmt, const uint8_t* c, int64_t idx) {
     if (fmt == 0) return ((const float*)c)[idx];
     return kvq::dequant_one(fmt, c + (idx >> 5) * kvq::block_bytes(fmt), (int)(idx & 31));
-}
-
-// Prompt attention from position 0 (every key and value is a current row,
-// dh == 64): one wave per (query head, 16 query rows).  Keys and values
-// come in blocks of 64 positions: lane j holds key j of the block (64
-// floats) and lane d holds dim d of the block's 64 values, so a query's 64
-// scores are one FMA chain per lane (the query from LDS, broadcast) and its
-// output update is one FMA chain per lane (the weights from LDS, broadcast).
-// Softmax per block in base-2 units (scale and log2 e folded into the
-// query): one maximum and one rescale per query and block.  Causal: query
-// row t sees positions 0..t.
-constexpr int kPromptRows = 16;
-
-__global__ __launch_bounds__(64) void attn_prompt_kernel(AttnArgs a) {
-    constexpr int DH = 64;
-    __shared__ __align__(16) float s_q[kPromptRows][DH];
-    __shared__ __align__(16) float s_o[kPromptRows][DH];
-    __shared__ float s_m[kPromptRows], s_l[kPromptRows];
-    __shared__ __align__(16) float s_p[DH];
-    const int h = blockIdx.x, lane = threadIdx.x;
-    const int t0 = blockIdx.y * kPromptRows;
-    const int nq = min(kPromptRows, a.T - t0);
-    const int kvd = a.Hkv * DH, kvh = h / (a.H / a.Hkv);
-    const float qsc = a.scale * 1.44269504088896341f;
-    for (int i = 0; i < nq; i++) {
-        s_q[i][lane] = a.q[((int64_t)(t0 + i) * a.H + h) * DH + lane] * qsc;
-        s_o[i][lane] = 0.f;
-    }
-    if (lane < kPromptRows) {
-        s_m[lane] = -INFINITY;
-        s_l[lane] = 0.f;
-    }
-    const int tmax = t0 + nq - 1;
-    for (int j0 = 0; j0 <= tmax; j0 += 64) {
-        // key j0 + lane (clamped past tmax: masked below) and value dim lane
-        const int jk = min(j0 + lane, tmax);
-        const f32x4* kp = (const f32x4*)(a.kcur + (int64_t)jk * kvd + kvh * DH);
-        float kr[DH];
-#pragma unroll
-        for (int i = 0; i < DH / 4; i++) {
-            const f32x4 v = gld(kp + i);
-            kr[4 * i] = v.x; kr[4 * i + 1] = v.y; kr[4 * i + 2] = v.z; kr[4 * i + 3] = v.w;
-        }
-        float vr[64];
-#pragma unroll
-        for (int j = 0; j < 64; j++) vr[j] = gld(a.vcur + (int64_t)min(j0 + j, tmax) * kvd + kvh * DH + lane);
-        const int i0 = j0 > t0 ? j0 - t0 : 0;                  // rows before j0 see nothing of this block
-#pragma unroll 1
-        for (int i = i0; i < nq; i++) {
-            const int t = t0 + i;
-            float sc = 0.f;
-#pragma unroll
-            for (int d = 0; d < DH; d += 4) {
-                const f32x4 qv = *(const f32x4*)&s_q[i][d];
-                sc = fmaf(qv.x, kr[d], sc);
-                sc = fmaf(qv.y, kr[d + 1], sc);
-                sc = fmaf(qv.z, kr[d + 2], sc);
-                sc = fmaf(qv.w, kr[d + 3], sc);
-            }
-            if (j0 + lane > t) sc = -INFINITY;
-            const float mo = s_m[i];
-            const float mn = fmaxf(mo, wave_max(sc));           // finite: position j0 <= t is in the block
-            const float al = __builtin_amdgcn_exp2f(mo - mn);
-            const float p = __builtin_amdgcn_exp2f(sc - mn);
-            const float ls = wave_sum(p);
-            s_p[lane] = p;
-            float acc = 0.f;
-#pragma unroll
-            for (int j = 0; j < 64; j += 4) {
-                const f32x4 pv = *(const f32x4*)&s_p[j];
-                acc = fmaf(pv.x, vr[j], acc);
-                acc = fmaf(pv.y, vr[j + 1], acc);
-                acc = fmaf(pv.z, vr[j + 2], acc);
-                acc = fmaf(pv.w, vr[j + 3], acc);
-            }
-            s_o[i][lane] = fmaf(s_o[i][lane], al, acc);
-            if (lane == 0) {
-                s_m[i] = mn;
-                s_l[i] = fmaf(s_l[i], al, ls);
-            }
-        }
-    }
-    for (int i = 0; i < nq; i++) a.out[((int64_t)(t0 + i) * a.H + h) * DH + lane] = s_o[i][lane] / s_l[i];
-}
-
-// The same prompt attention on the matrix cores (v_mfma_f32_16x16x4f32: fp32
-// products, fp32 sums), for query heads in groups of 4 that share a KV head
-// (H / Hkv a multiple of 4).  A workgroup takes one group and 16 query rows
-// with NSET sets of 4 waves, wave w of a set query head 4 blockIdx.x + w:
-// set k takes the 64-position K/V blocks k, k + NSET, ..., each with its
-// own online softmax, merged at the end through LDS (so the longest row
-// tiles take 1 / NSET as many steps; launched with two sets, four measured
-// slower).  A set stages its block once in LDS (the
-// next block's loads in registers while the current one is multiplied).
-// Per block a wave forms S^T = K Q^T (4 tiles of 16 keys x 16 rows, 16 steps
-// of 4 dims each: lane l's A value is key l % 16 of the tile at dim
-// 16 (l / 16) + step, its B value the query row l % 16 at that dim), so a
-// lane holds 16 scores of one query row (keys 16 kt + 4 (l / 16) + e), the
-// row maximum and sum take two cross-lane steps, and those scores are
-// directly the B operand of O^T += V^T P^T (step 4 kt + e uses key
-// 16 kt + 4 (l / 16) + e; A value: dim 4 (l % 16) + dt of that key for
-// output tile dt).  A lane ends with dims 16 (l / 16) .. + 15 of its row.
-// Base-2 softmax units and the per-block rescale as in attn_prompt_kernel.
-template <int NSET>
-__global__ __launch_bounds__(256 * NSET) void attn_prompt_mfma_kernel(AttnArgs a) {
-    constexpr int DH = 64, LDK = DH + 4;
-    __shared__ __align__(16) float s_k[NSET][64][LDK];
-    __shared__ __align__(16) float s_v[NSET][64][LDK];
-    const int tid = threadIdx.x, lane = tid & 63;
-    const int ws = __builtin_amdgcn_readfirstlane(tid >> 8);     // wave set: even / odd blocks
-    const int ts = tid & 255;
-    const int w = __builtin_amdgcn_readfirstlane((tid >> 6) & 3);
-    const int ntile = (a.T + kPromptRows - 1) / kPromptRows;
-    const int t0 = (ntile - 1 - (int)blockIdx.y) * kPromptRows;   // longest row tiles first
-    const int h = 4 * (int)blockIdx.x + w;
-    const int kvh = 4 * (int)blockIdx.x / (a.H / a.Hkv);
-    const int kvd = a.Hkv * DH;
-    const int tmax = min(t0 + kPromptRows, a.T) - 1;
-    const int nblk = tmax / 64 + 1, npair = (nblk + NSET - 1) / NSET;
-    const int fr = lane & 15, g = lane >> 4;
-    const int row = t0 + fr;
-    const float qsc = a.scale * 1.44269504088896341f;
-    float qv[16];                                   // row fr (clamped), dims 16 g .. 16 g + 15
-    {
-        const f32x4* qp = (const f32x4*)(a.q + ((int64_t)min(row, a.T - 1) * a.H + h) * DH + 16 * g);
-#pragma unroll
-        for (int i = 0; i < 4; i++) {
-            const f32x4 v = gld(qp + i);
-            qv[4 * i] = v.x * qsc; qv[4 * i + 1] = v.y * qsc; qv[4 * i + 2] = v.z * qsc; qv[4 * i + 3] = v.w * qsc;
-        }
-    }
-    // staging: thread ts of a set moves dims 16 (ts % 4) .. + 15 of key
-    // j0 + ts / 4 (clamped to tmax: such keys are masked)
-    const int sk = ts >> 2, sq = ts & 3;
-    f32x4 kr[4], vr[4];
-    auto load_blk = [&](int j0) {
-        const int64_t off = (int64_t)min(j0 + sk, tmax) * kvd + kvh * DH + 16 * sq;
-        const f32x4* kp = (const f32x4*)(a.kcur + off);
-        const f32x4* vp = (const f32x4*)(a.vcur + off);
-#pragma unroll
-        for (int i = 0; i < 4; i++) {
-            kr[i] = gld(kp + i);
-            vr[i] = gld(vp + i);
-        }
-    };
-    f32x4 o[4];                                     // O^T tile dt: dims 16 g + 4 e + dt of row fr
-#pragma unroll
-    for (int dt = 0; dt < 4; dt++) o[dt] = f32x4{0.f, 0.f, 0.f, 0.f};
-    float m = -INFINITY, l = 0.f;
-    load_blk(64 * ws);
-    for (int ip = 0; ip < npair; ip++) {
-        const int j0 = 64 * (NSET * ip + ws);       // this set's block; past tmax: none (same for the set)
-        __syncthreads();                            // the previous block's operands are read
-#pragma unroll
-        for (int i = 0; i < 4; i++) {
-            *(f32x4*)&s_k[ws][sk][16 * sq + 4 * i] = kr[i];
-            *(f32x4*)&s_v[ws][sk][16 * sq + 4 * i] = vr[i];
-        }
-        __syncthreads();
-        load_blk(j0 + 64 * NSET <= tmax ? j0 + 64 * NSET : j0);   // unconditional: the last block reloads itself
-        if (j0 > tmax) continue;
-        f32x4 s[4];
-#pragma unroll
-        for (int kt = 0; kt < 4; kt++) s[kt] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int q4 = 0; q4 < 4; q4++) {
-            f32x4 kv[4];
-#pragma unroll
-            for (int kt = 0; kt < 4; kt++) kv[kt] = *(const f32x4*)&s_k[ws][16 * kt + fr][16 * g + 4 * q4];
-#pragma unroll
-            for (int c = 0; c < 4; c++)
-#pragma unroll
-                for (int kt = 0; kt < 4; kt++)
-                    s[kt] = __builtin_amdgcn_mfma_f32_16x16x4f32(kv[kt][c], qv[4 * q4 + c], s[kt], 0, 0, 0);
-        }
-        // causal mask, then the row's maximum over the lanes l % 16 == fr
-        float mx = -INFINITY;
-#pragma unroll
-        for (int kt = 0; kt < 4; kt++)
-#pragma unroll
-            for (int e = 0; e < 4; e++) {
-                if (j0 + 16 * kt + 4 * g + e > row) s[kt][e] = -INFINITY;
-                mx = fmaxf(mx, s[kt][e]);
-            }
-        mx = fmaxf(mx, __shfl_xor(mx, 16));
-        mx = fmaxf(mx, __shfl_xor(mx, 32));
-        const float mn = fmaxf(m, mx);              // finite: key j0 <= every row of the tile
-        const float al = __builtin_amdgcn_exp2f(m - mn);
-        float ps = 0.f;
-#pragma unroll
-        for (int kt = 0; kt < 4; kt++)
-#pragma unroll
-            for (int e = 0; e < 4; e++) {
-                s[kt][e] = __builtin_amdgcn_exp2f(s[kt][e] - mn);
-                ps += s[kt][e];
-            }
-        ps += __shfl_xor(ps, 16);
-        ps += __shfl_xor(ps, 32);
-        l = fmaf(l, al, ps);
-        m = mn;
-#pragma unroll
-        for (int dt = 0; dt < 4; dt++) o[dt] *= al;
-#pragma unroll
-        for (int kt = 0; kt < 4; kt++)
-#pragma unroll
-            for (int e = 0; e < 4; e++) {
-                const f32x4 vv = *(const f32x4*)&s_v[ws][16 * kt + 4 * g + e][4 * fr];
-#pragma unroll
-                for (int dt = 0; dt < 4; dt++) o[dt] = __builtin_amdgcn_mfma_f32_16x16x4f32(vv[dt], s[kt][e], o[dt], 0, 0, 0);
-            }
-    }
-    // merge: set 1 leaves (m, l, O) in LDS, set 0 combines (set 0 always
-    // holds block 0, so its maximum is finite; set 1's may be -inf: weight 0)
-    __syncthreads();
-    float* xch = &s_k[0][0][0];                     // 18 floats per thread of sets 1 ..
-    if (ws > 0) {
-        float* d = xch + 18 * (256 * (ws - 1) + ts);
-        d[0] = m;
-        d[1] = l;
-#pragma unroll
-        for (int dt = 0; dt < 4; dt++) *(f32x4*)&d[2 + 4 * dt] = o[dt];
-    }
-    __syncthreads();
-    if (ws == 0 && row < a.T) {
-        float mm = m;
-#pragma unroll
-        for (int k = 1; k < NSET; k++) mm = fmaxf(mm, xch[18 * (256 * (k - 1) + ts)]);
-        const float a0 = __builtin_amdgcn_exp2f(m - mm);
-        float lt = l * a0;
-        f32x4 ot[4];
-#pragma unroll
-        for (int dt = 0; dt < 4; dt++) ot[dt] = o[dt] * a0;
-#pragma unroll
-        for (int k = 1; k < NSET; k++) {
-            const float* d = xch + 18 * (256 * (k - 1) + ts);
-            const float a1 = d[0] == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(d[0] - mm);
-            lt = fmaf(d[1], a1, lt);
-#pragma unroll
-            for (int dt = 0; dt < 4; dt++) {
-                const f32x4 o1 = *(const f32x4*)&d[2 + 4 * dt];
-#pragma unroll
-                for (int e = 0; e < 4; e++) ot[dt][e] = fmaf(o1[e], a1, ot[dt][e]);
-            }
-        }
-        f32x4* op = (f32x4*)(a.out + ((int64_t)row * a.H + h) * DH + 16 * g);
-#pragma unroll
-        for (int e = 0; e < 4; e++) gst(op + e, f32x4{ot[0][e] / lt, ot[1][e] / lt, ot[2][e] / lt, ot[3][e] / lt});
-    }
 }
 
 __global__ __launch_bounds__(64) void attn_generic_kernel(AttnArgs a, int kf, int vf) {
@@ -1571,6 +1205,17 @@ extern "C" int rina_hip_gqa_attention(const float* q, const float* kcur, const f
         sa.scale = 1.0f / sqrtf((float)dh);
         return launch_split_mode<false>(sa, rep, ws_bytes, workspace, st);
     }
+    if (dh == 64) {
+        RowsAttnArgs r{};
+        r.q = q; r.k = kcur; r.v = vcur;
+        r.ck = (const uint8_t*)cache_k; r.cv = (const uint8_t*)cache_v;
+        r.rkc = rkc; r.rks = rks; r.out = out;
+        r.mode = mode; r.pre_rope = pre_rope; r.T = T; r.H = H; r.Hkv = Hkv;
+        r.start_pos = start_pos; r.max_seq = max_seq; r.d_pos = d_pos;
+        r.scale = 1.0f / sqrtf((float)dh);
+        const int rc = attn_rows(ROWS_GQA, r, 64, 64, st);
+        if (rc != RINA_ERR_SHAPE) return rc;         // alignment it does not take: the generic kernel
+    }
     AttnArgs a{};
     a.q = q; a.kcur = kcur; a.vcur = vcur;
     a.ck = (const uint8_t*)cache_k; a.cv = (const uint8_t*)cache_v;
@@ -1578,16 +1223,6 @@ extern "C" int rina_hip_gqa_attention(const float* q, const float* kcur, const f
     a.mode = mode; a.pre_rope = pre_rope; a.T = T; a.H = H; a.Hkv = Hkv; a.dh = dh;
     a.start_pos = start_pos; a.max_seq = max_seq; a.d_pos = d_pos;
     a.scale = 1.0f / sqrtf((float)dh);
-    // a prompt from position 0 reads only the current rows
-    if (T > 1 && !d_pos && start_pos == 0 && dh == 64 && ((uintptr_t)kcur % 16 == 0)) {
-        const int ntile = (T + kPromptRows - 1) / kPromptRows;
-        if (rep % 4 == 0 && ((uintptr_t)q | (uintptr_t)vcur | (uintptr_t)out) % 16 == 0)
-            hipLaunchKernelGGL(attn_prompt_mfma_kernel<2>, dim3(H / 4, ntile), dim3(512), 0, st, a);
-        else
-            hipLaunchKernelGGL(attn_prompt_kernel, dim3(H, ntile), dim3(64), 0, st, a);
-        RINA_LAUNCH_CHECK();
-        return RINA_OK;
-    }
     hipLaunchKernelGGL(attn_generic_kernel, dim3(H, T), dim3(64), 0, st, a, kf, vf);
     RINA_LAUNCH_CHECK();
     return RINA_OK;
@@ -1820,15 +1455,17 @@ extern "C" int rina_hip_dq_prompt_attention_kv(const float* qa, const float* qb,
     a.qc = rope_q_cos; a.qs = rope_q_sin; a.kc = rope_k_cos; a.ks = rope_k_sin;
     if (packed) { a.ckq = (uint8_t*)cache_k; a.ckr = cache_kr; a.cvq = (uint8_t*)cache_v; }
     else { a.ck = (float*)cache_k; a.cv = (float*)cache_v; }
-    a.out = out;
     a.H = H; a.Hkv = Hkv; a.da = da; a.db = db; a.dv = dv; a.start_pos = start_pos; a.max_seq = max_seq;
     a.scale = 1.0f / sqrtf((float)(da + db));
     hipStream_t st = as_stream(stream);
     if (packed) hipLaunchKernelGGL(dq_pack_rows_kernel<1>, dim3(T, Hkv), dim3(64), 0, st, a);
     else hipLaunchKernelGGL(dq_pack_rows_kernel<0>, dim3(T, Hkv), dim3(64), 0, st, a);
     RINA_LAUNCH_CHECK();
-    if (packed) hipLaunchKernelGGL(dq_prompt_kv_kernel<1>, dim3(T, H), dim3(256), 0, st, a);
-    else hipLaunchKernelGGL(dq_prompt_kv_kernel<0>, dim3(T, H), dim3(256), 0, st, a);
-    RINA_LAUNCH_CHECK();
-    return RINA_OK;
+    RowsAttnArgs r{};
+    r.qa = qa; r.qb = qb; r.ka = ka; r.kb = kb; r.v = v;
+    r.qc = rope_q_cos; r.qs = rope_q_sin; r.kc = rope_k_cos; r.ks = rope_k_sin;
+    r.ck = (const uint8_t*)cache_k; r.cv = (const uint8_t*)cache_v; r.ckr = cache_kr;
+    r.out = out; r.mode = kv_mode; r.T = T; r.H = H; r.Hkv = Hkv; r.da = da; r.db = db;
+    r.start_pos = start_pos; r.max_seq = max_seq; r.scale = a.scale;
+    return attn_rows(ROWS_DQ, r, da + db, dv, st);
 }

@@ -25,6 +25,7 @@
 #include <algorithm>
 #include <vector>
 #include "rina_common.hpp"
+#include "attn_rows.hpp"
 
 namespace {
 
@@ -1015,6 +1016,8 @@ __global__ __launch_bounds__(256) void mla_combine_kernel(MlaArgs a) {
 //                      normalized c into a contiguous matrix and its query
 //                      [q_nope | RoPE(q_rope)] per head;
 //   one T-row product of the two halves of w_kv_b (K_nope, V);
+//   at the DeepSeek-V2 head shape (128 + 64, 128) attn_rows on those rows and
+//   the records; at other shapes
 //   mla_expand_kernel: per row and head, K = [K_nope | RoPE(k_pe)] and V
 //                      padded with zeros to the key width;
 //   causal attention over the T rows (rina_hip_gqa_attention with H KV
@@ -1406,6 +1409,16 @@ extern "C" int rina_hip_mla_prompt_attention(const float* q, const float* kva, c
                                {(const uint8_t*)w_kv_b + vb_off, nullptr, v_rows, H * v_dim}};
     int rc = rina_hip_linear_fused(segs, 2, qt_kv_b, c_rows, T, dc, RINA_EPI_STORE, RINA_PRO_NONE, nullptr, 0.f, stream);
     if (rc) return rc;
+    // the DeepSeek-V2 head shape: straight from K_nope, V and the records
+    if (nope == 128 && rope == 64 && v_dim == 128) {
+        RowsAttnArgs r{};
+        r.q = q_full; r.k = k_nope; r.v = v_rows; r.ck = (const uint8_t*)cache;
+        r.da = dc; r.db = dc + rope;
+        r.out = out; r.T = T; r.H = H; r.Hkv = H; r.max_seq = max_seq;
+        r.scale = 1.0f / sqrtf((float)D);
+        rc = attn_rows(ROWS_MLA, r, D, v_dim, st);
+        if (rc != RINA_ERR_SHAPE) return rc;         // alignment it does not take: the general form
+    }
     hipLaunchKernelGGL(mla_expand_kernel, dim3(T, H), dim3(256), 0, st, a, k_nope, v_rows, k_full, v_full);
     RINA_LAUNCH_CHECK();
     rc = rina_hip_gqa_attention(q_full, k_full, v_full, k_full, v_full, RINA_KV_FP32, 0, nullptr, nullptr, T, H, H, D,
