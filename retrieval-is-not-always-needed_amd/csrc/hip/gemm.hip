@@ -1002,6 +1002,177 @@ int launch_fmt(const RowsArgs& a, int nmat, int rt, int ct, hipStream_t st) {
     return ct == 1 ? launch32<FMT, 1, 2, 1>(a, st) : launch32<FMT, 1, 2, 2>(a, st);
 }
 
+// ---- fp32 weights: v_mfma_f32_16x16x4f32 tiles ----
+// A wave owns MI 16-row tiles x NJ 16-column tiles (per matrix) of its K
+// slice (32-value chunks, interleaved over the KW waves); rows and weights
+// come straight from memory, a lane holding 8 consecutive values of its row
+// and column per chunk (any order of K does, as long as both agree).  Sums are
+// kept per 256 values and added up: the error of one 2048-long chain, as a
+// serial product has it, halves.  NT: the weights are read once (one row
+// tile), streamed past the caches.
+// LM head 128256 x 2048: bound by the weight stream up to 32 rows (1.05 GB),
+// beyond by the fp32 matrix cores.
+template <int NMAT, int MI, int NJ, bool NT>
+__global__ __launch_bounds__(512, 2) void rows_f32_kernel(RowsArgs a) {
+    extern __shared__ __align__(16) float s_part[];
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int fr = lane & 15, g = lane >> 4;
+    Tile t;
+    if (!t.find(a)) return;
+    const int wn = wave % a.NW, wk = wave / a.NW;
+    const int n0 = (t.bx * a.NW + wn) * 16 * NJ, N = t.N, K = a.K, nch = (K + 31) >> 5;
+    const float* xr[MI];
+    const float* wr[NMAT][NJ];
+#pragma unroll
+    for (int i = 0; i < MI; i++) xr[i] = (const float*)a.xp + (int64_t)min((t.by * MI + i) * 16 + fr, a.M - 1) * K;
+#pragma unroll
+    for (int m = 0; m < NMAT; m++)
+#pragma unroll
+        for (int j = 0; j < NJ; j++) wr[m][j] = (const float*)(m ? t.w2 : t.w) + (int64_t)min(n0 + 16 * j + fr, N - 1) * K;
+    f32x4 tot[NMAT][MI][NJ], acc[NMAT][MI][NJ];
+    const f32x4 z4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int m = 0; m < NMAT; m++)
+#pragma unroll
+        for (int i = 0; i < MI; i++)
+#pragma unroll
+            for (int j = 0; j < NJ; j++) tot[m][i][j] = acc[m][i][j] = z4;
+    struct Chunk {
+        f32x4 x[MI][2], w[NMAT][NJ][2];
+    };
+    // chunk c: values 32 c + 8 g .. + 7 (K % 4 == 0; past K: zeros)
+    auto load = [&](int c, Chunk& r) {
+        const int k = 32 * c + 8 * g;
+#pragma unroll
+        for (int u = 0; u < 2; u++) {
+            const bool on = k + 4 * u < K;
+            const int kk = on ? k + 4 * u : 0;
+#pragma unroll
+            for (int i = 0; i < MI; i++) {
+                r.x[i][u] = gld((const f32x4*)(xr[i] + kk));
+                if (!on) r.x[i][u] = z4;
+            }
+#pragma unroll
+            for (int m = 0; m < NMAT; m++)
+#pragma unroll
+                for (int j = 0; j < NJ; j++) {
+                    r.w[m][j][u] = NT ? gld_nt((const f32x4*)(wr[m][j] + kk)) : gld((const f32x4*)(wr[m][j] + kk));
+                    if (!on) r.w[m][j][u] = z4;
+                }
+        }
+    };
+    auto mul = [&](const Chunk& r) {
+#pragma unroll
+        for (int u = 0; u < 2; u++)
+#pragma unroll
+            for (int e = 0; e < 4; e++)
+#pragma unroll
+                for (int m = 0; m < NMAT; m++)
+#pragma unroll
+                    for (int j = 0; j < NJ; j++)
+#pragma unroll
+                        for (int i = 0; i < MI; i++)
+                            acc[m][i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(r.x[i][u][e], r.w[m][j][u][e], acc[m][i][j], 0, 0, 0);
+    };
+    auto flush = [&]() {
+#pragma unroll
+        for (int m = 0; m < NMAT; m++)
+#pragma unroll
+            for (int i = 0; i < MI; i++)
+#pragma unroll
+                for (int j = 0; j < NJ; j++) {
+                    tot[m][i][j] += acc[m][i][j];
+                    acc[m][i][j] = z4;
+                }
+    };
+    // two chunks in flight ahead of the one that is multiplied
+    Chunk c0, c1;
+    const int last = wk < nch ? wk + (nch - 1 - wk) / a.KW * a.KW : 0;   // past the end: the last chunk again, not multiplied
+    load(min(wk, last), c0);
+    load(min(wk + a.KW, last), c1);
+    int n = 0;
+    for (int c = wk; c < nch; c += 2 * a.KW) {
+        mul(c0);
+        load(min(c + 2 * a.KW, last), c0);
+        __builtin_amdgcn_sched_barrier(0);
+        if (c + a.KW < nch) mul(c1);
+        load(min(c + 3 * a.KW, last), c1);
+        __builtin_amdgcn_sched_barrier(0);
+        n += 2;
+        if ((n & 7) == 0) flush();
+    }
+    flush();
+    f32x4* sp = (f32x4*)s_part;
+    constexpr int NR = NMAT * MI * NJ;
+    for (int h = a.KW >> 1; h >= 1; h >>= 1) {
+        f32x4* d = sp + (int64_t)((wk >= h ? wk - h : wk) * a.NW + wn) * NR * 64 + lane;
+        if (wk >= h && wk < 2 * h) {
+#pragma unroll
+            for (int m = 0; m < NMAT; m++)
+#pragma unroll
+                for (int i = 0; i < MI; i++)
+#pragma unroll
+                    for (int j = 0; j < NJ; j++) d[((m * MI + i) * NJ + j) * 64] = tot[m][i][j];
+        }
+        __syncthreads();
+        if (wk < h) {
+#pragma unroll
+            for (int m = 0; m < NMAT; m++)
+#pragma unroll
+                for (int i = 0; i < MI; i++)
+#pragma unroll
+                    for (int j = 0; j < NJ; j++) tot[m][i][j] += d[((m * MI + i) * NJ + j) * 64];
+        }
+        __syncthreads();
+    }
+    if (wk > 0) return;
+#pragma unroll
+    for (int i = 0; i < MI; i++)
+#pragma unroll
+        for (int j = 0; j < NJ; j++)
+#pragma unroll
+            for (int e = 0; e < 4; e++)
+                finish<NMAT>(a, t, (t.by * MI + i) * 16 + 4 * g + e, n0 + 16 * j + fr, tot[0][i][j][e], tot[NMAT - 1][i][j][e]);
+}
+
+template <int NMAT, int MI, int NJ>
+int launch_f32(const RowsArgs& a, hipStream_t st) {
+    const size_t lds = a.KW > 1 ? (size_t)(a.KW / 2) * a.NW * NMAT * MI * NJ * 1024 : 0;
+    const dim3 grid(8 * a.mpp * a.npp), blk(64 * a.NW * a.KW);
+    if (a.mt == 1) hipLaunchKernelGGL((rows_f32_kernel<NMAT, MI, NJ, true>), grid, blk, lds, st, a);
+    else hipLaunchKernelGGL((rows_f32_kernel<NMAT, MI, NJ, false>), grid, blk, lds, st, a);
+    return hipGetLastError() == hipSuccess ? RINA_OK : RINA_ERR_HIP;
+}
+
+// segments, tile counts and the XCD split of a launch: row tiles of tr rows,
+// column tiles of bn, weight bytes per value
+void plan_tiles(RowsArgs& a, const rina_linear_seg* segs, int nseg, int nmat, int tr, int bn, double wb, bool grouped) {
+    int t = 0;
+    for (int s = 0; s < 3; s++) {
+        const int ss = s < nseg ? s : 0;
+        a.w[s] = (const uint8_t*)segs[ss].weight;
+        a.y[s] = segs[ss].out;
+        a.N[s] = segs[ss].N;
+        a.t0[s] = s < nseg ? t : 1 << 30;
+        if (s < nseg) t += (segs[s].N + bn - 1) / bn;
+    }
+    a.nseg = nseg;
+    a.w2 = nmat == 2 ? (const uint8_t*)segs[0].weight2 : nullptr;
+    a.mt = (a.M + tr - 1) / tr;
+    a.nt = t;
+    // the split with the fewest bytes fetched by the 8 L2s: xb x + (8 / xb) W
+    // (grouped rows: every group's weights on one XCD)
+    const double xbytes = 4.0 * a.M * a.K, wbytes = (double)nmat * bn * t * a.K * wb;
+    int best = 1;
+    if (!grouped)
+        for (int xb = 2; xb <= 8; xb *= 2)
+            if (xb * xbytes + (8 / xb) * wbytes < best * xbytes + (8 / best) * wbytes) best = xb;
+    a.xb = best;
+    a.mpp = (a.mt + 8 / best - 1) / (8 / best);
+    a.npp = (t + best - 1) / best;
+}
+
 size_t up256(size_t n) { return (n + 255) & ~(size_t)255; }
 
 }  // namespace
@@ -1050,10 +1221,9 @@ int rows_gemm(const rina_linear_seg* segs, int nseg, int qt, const RowsX& x, int
     const int nmat = two ? 2 : 1;
     RowsArgs a{};
     a.xp = (const uint4*)x.xp; a.xs = x.xs; a.xg = (const uint4*)x.xg;
-    a.M = x.rows; a.K = x.K; a.epi = epi; a.nseg = nseg;
+    a.M = x.rows; a.K = x.K; a.epi = epi;
     a.nks = (x.K + 127) / 128 * 4;
     a.ngw = (x.K + 511) / 512;
-    a.w2 = two ? (const uint8_t*)segs[0].weight2 : nullptr;
     a.plan = plan;
     a.stride = stride;
     const int nss = a.nks / 4;
@@ -1075,29 +1245,45 @@ int rows_gemm(const rina_linear_seg* segs, int nseg, int qt, const RowsX& x, int
     a.KW = kw;
     a.NW = kw >= 4 ? 1 : 4 / kw;
     const int BN = tc * nj * a.NW;
-    int t = 0;
-    for (int s = 0; s < 3; s++) {
-        const int ss = s < nseg ? s : 0;
-        a.w[s] = (const uint8_t*)segs[ss].weight;
-        a.y[s] = segs[ss].out;
-        a.N[s] = segs[ss].N;
-        a.t0[s] = s < nseg ? t : 1 << 30;
-        if (s < nseg) t += (segs[s].N + BN - 1) / BN;
-    }
-    a.mt = (int)mts;
-    a.nt = t;
-    // XCD split with the fewest bytes fetched by the 8 L2s: xb x + (8 / xb) W
-    // (grouped rows: every group's weights on one XCD)
-    const double xbytes = 4.0 * x.rows * x.K;
-    const double wbytes = (double)nmat * BN * t * x.K * (qt == RINA_QT_Q4_0F ? 0.625 : qt == RINA_QT_GGML_Q2_K ? 84.0 / 256 : 0.5625);
-    int best = 1;
-    if (!plan)
-        for (int xb = 2; xb <= 8; xb *= 2)
-            if (xb * xbytes + (8 / xb) * wbytes < best * xbytes + (8 / best) * wbytes) best = xb;
-    a.xb = best;
-    a.mpp = (a.mt + 8 / best - 1) / (8 / best);
-    a.npp = (t + best - 1) / best;
+    plan_tiles(a, segs, nseg, nmat, tr, BN, qt == RINA_QT_Q4_0F ? 0.625 : qt == RINA_QT_GGML_Q2_K ? 84.0 / 256 : 0.5625, plan);
     if (qt == RINA_QT_Q4_0) return launch_fmt<FMT_Q4_0>(a, nmat, rt, nj, st);
     if (qt == RINA_QT_Q4_0F) return launch_fmt<FMT_Q4_0F>(a, nmat, rt, nj, st);
     return x.K % 128 == 0 ? launch_fmt<FMT_Q2_K>(a, nmat, rt, nj, st) : launch_fmt<FMT_Q2_S>(a, nmat, rt, nj, st);
+}
+
+bool rows_f32_ok(const rina_linear_seg* segs, int nseg, const float* x, int K) {
+    bool ok = K % 4 == 0 && (uintptr_t)x % 16 == 0;
+    for (int s = 0; s < nseg; s++) ok = ok && (uintptr_t)segs[s].weight % 16 == 0 && (uintptr_t)segs[s].weight2 % 16 == 0;
+    return ok;
+}
+
+int rows_f32(const rina_linear_seg* segs, int nseg, const float* x, int M, int K, int epi, hipStream_t st) {
+    const int nmat = epi == RINA_EPI_SWIGLU ? 2 : 1;
+    RowsArgs a{};
+    a.xp = (const uint4*)x;
+    a.M = M; a.K = K; a.epi = epi;
+    // (row tiles, column tiles) per wave: 4 x 2, 2 x 4 or 1 x 4 by the row
+    // count, smaller where that leaves SIMDs idle with K split over 8
+    const int64_t simds = 4LL * rina_num_cus();
+    int mi = M > 32 ? 4 : M > 16 ? 2 : 1, nj = (mi == 4 ? 2 : 4) / nmat;
+    auto tiles = [&]() {
+        int64_t t = 0;
+        for (int s = 0; s < nseg; s++) t += (segs[s].N + 16 * nj - 1) / (16 * nj);
+        return t * ((M + 16 * mi - 1) / (16 * mi));
+    };
+    if (tiles() * 8 < simds) { nj = 1; if (mi == 4) mi = 2; }
+    if (mi == 2 && tiles() * 8 < simds) mi = 1;
+    int kw = 1;
+    while (kw < 8 && tiles() * kw < 2 * simds && K >= 256 * kw) kw *= 2;
+    a.KW = kw;
+    a.NW = kw >= 4 ? 1 : 4 / kw;
+    plan_tiles(a, segs, nseg, nmat, 16 * mi, 16 * nj * a.NW, 4.0, false);
+    if (nmat == 2) {
+        if (mi == 4) return launch_f32<2, 4, 1>(a, st);
+        if (mi == 2) return nj == 1 ? launch_f32<2, 2, 1>(a, st) : launch_f32<2, 2, 2>(a, st);
+        return nj == 1 ? launch_f32<2, 1, 1>(a, st) : launch_f32<2, 1, 2>(a, st);
+    }
+    if (mi == 4) return launch_f32<1, 4, 2>(a, st);
+    if (mi == 2) return nj == 1 ? launch_f32<1, 2, 1>(a, st) : launch_f32<1, 2, 4>(a, st);
+    return nj == 1 ? launch_f32<1, 1, 1>(a, st) : launch_f32<1, 1, 4>(a, st);
 }

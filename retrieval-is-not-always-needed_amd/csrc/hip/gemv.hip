@@ -1441,6 +1441,7 @@ extern "C" int rina_hip_linear_fused_ex(const rina_linear_seg* segs, int nseg, i
         return RINA_OK;
     }
     if (M > 1) {
+        if (qt == RINA_QT_FP32 && rows_f32_ok(segs, nseg, input, K)) return rows_f32(segs, nseg, input, M, K, epi, st);
         for (int s = 0; s < nseg; s++) {
             int rc = gemm_tiled(segs[s], qt, input, M, K, epi, st);
             if (rc) return rc;

@@ -24,3 +24,7 @@ int rows_split(int qt, const float* x, const int* src, int rows, int K, int pro,
 // weights start group * stride bytes into the segment
 int rows_gemm(const rina_linear_seg* segs, int nseg, int qt, const RowsX& x, int epi, const int* plan, int64_t stride,
               int rt_plan, hipStream_t st);
+
+// fp32 weights: rows and weights 16-byte aligned, K % 4 == 0; M >= 2, up to 3 segments
+bool rows_f32_ok(const rina_linear_seg* segs, int nseg, const float* x, int K);
+int rows_f32(const rina_linear_seg* segs, int nseg, const float* x, int M, int K, int epi, hipStream_t st);
