@@ -318,9 +318,10 @@ int rina_hip_moe_ffn(const float* x, const void* gate_exps, const void* up_exps,
  * deepseek_mla_layer.cu:291-350, for every row): h[T, d] += shared experts
  * + sum over each row's top-k of p_j * expert_j(RMSNorm(h_row, ln2)).  The
  * norm, the fp32 router logits and the shared experts run as T-row
- * products; the rows are then grouped by selected expert (the selection is
- * read back to the host once: the call synchronizes the stream) and each
- * expert runs as one product over its rows.  gate_sh / up_sh / down_sh may
+ * products; the rows are then grouped by selected expert and each expert
+ * runs over its rows: on the device for Q4_0 / Q4_0F / Q2_K experts with d
+ * and ffn multiples of 32, else one expert after the other (the selection is
+ * then read back to the host once: the call synchronizes the stream).  gate_sh / up_sh / down_sh may
  * be NULL with S == 0.  Any quant type rina_hip_linear_fused takes; the
  * workspace (16-byte aligned) holds rina_hip_moe_rows_workspace() bytes. */
 size_t rina_hip_moe_rows_workspace(int T, int d, int n_experts, int k, int ffn, int shared_ffn);

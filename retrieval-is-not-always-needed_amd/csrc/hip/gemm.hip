@@ -78,6 +78,7 @@ struct SplitXArgs {
     uint4* xp;
     float* xs;             // [rows] 2^-e of the row scale 2^e
     uint16_t* xg;          // Q2_K: group-sum fragments
+    const int* used;       // grouped rows: 16-row tiles in use (NULL: all)
     int M, K, nks, ngw;
     int pro;
     float eps;
@@ -96,6 +97,7 @@ __global__ __launch_bounds__(256 * kSplitRows) void x_split_kernel(SplitXArgs a)
     __shared__ float s_red[3][kSplitRows][4];
     const int r = threadIdx.x >> 8, tid = threadIdx.x & 255, wave = tid >> 6, lane = tid & 63;
     const int row = blockIdx.x * kSplitRows + r, mt = row >> 4;
+    if (a.used && mt >= __builtin_amdgcn_readfirstlane(gld(a.used))) return;   // the whole workgroup: 4 rows of one tile
     int srow = row < a.M ? row : -1;
     if (a.src) srow = __builtin_amdgcn_readfirstlane(gld(a.src + row));
     const int nu = a.K >> 3, nup = a.nks * 4;      // 8-value units, padded
@@ -261,7 +263,8 @@ struct RowsArgs {
     int mt, nt;            // row tiles of 16 MI, column tiles of 16 NJ NW
     int xb, mpp, npp;      // XCD split: weight parts, row / column tiles per part
     int NW, KW;
-    // grouped rows (experts): plan[0] = row tiles in use, plan[1 + i] = group of row tile i
+    // grouped rows (experts): plan[0] row tiles in use, plan[1] 16-row tiles in
+    // use, then per row tile its group, first 16-row tile and row limit
     const int* plan;
     int64_t stride;
 };
@@ -462,8 +465,9 @@ struct Tile {
     const uint8_t* w;
     const uint8_t* w2;
     float* y;
-    int N, by, bx;         // bx: column tile inside the segment
-    __device__ __forceinline__ bool find(const RowsArgs& a) {
+    int N, bx;             // bx: column tile inside the segment
+    int r16, mend;         // first 16-row tile, row limit
+    __device__ __forceinline__ bool find(const RowsArgs& a, int n16) {   // n16: 16-row tiles per row tile
         const int xcd = blockIdx.x & 7, kb = blockIdx.x >> 3;
         const int mm = kb / a.npp, nn = kb - mm * a.npp;
         int mpp = a.mpp, mt = a.mt;
@@ -471,7 +475,7 @@ struct Tile {
             mt = min(mt, __builtin_amdgcn_readfirstlane(gld(a.plan)));
             mpp = (mt + 8 / a.xb - 1) / (8 / a.xb);
         }
-        by = (xcd / a.xb) * mpp + mm;
+        const int by = (xcd / a.xb) * mpp + mm;
         bx = (xcd % a.xb) * a.npp + nn;
         if (mm >= mpp || by >= mt || bx >= a.nt) return false;
         const int sg = (a.nseg > 1 && bx >= a.t0[1]) + (a.nseg > 2 && bx >= a.t0[2]);
@@ -480,8 +484,13 @@ struct Tile {
         y = sg == 0 ? a.y[0] : sg == 1 ? a.y[1] : a.y[2];
         N = sg == 0 ? a.N[0] : sg == 1 ? a.N[1] : a.N[2];
         bx -= sg == 0 ? a.t0[0] : sg == 1 ? a.t0[1] : a.t0[2];
+        r16 = by * n16;
+        mend = a.M;
         if (a.plan) {
-            const int64_t g = __builtin_amdgcn_readfirstlane(gld(a.plan + 1 + by));
+            const int* p = a.plan + 2 + 3 * by;
+            const int64_t g = __builtin_amdgcn_readfirstlane(gld(p));
+            r16 = __builtin_amdgcn_readfirstlane(gld(p + 1));
+            mend = __builtin_amdgcn_readfirstlane(gld(p + 2));
             w += g * a.stride;
             w2 += g * a.stride;
         }
@@ -491,7 +500,7 @@ struct Tile {
 
 template <int NMAT>
 __device__ __forceinline__ void finish(const RowsArgs& a, const Tile& t, int r, int c, float v, float u) {
-    if (r >= a.M || c >= t.N) return;
+    if (r >= t.mend || c >= t.N) return;
     float* o = t.y + (int64_t)r * t.N + c;
     if (NMAT == 2) gst(o, silu_mul(v, u));
     else if (a.epi == RINA_EPI_ADD) gst(o, gld(o) + v);
@@ -601,14 +610,14 @@ __global__ __launch_bounds__(512, 2) void rows16_kernel(RowsArgs a) {
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int fr = lane & 15, f = lane >> 4;
     Tile t;
-    if (!t.find(a)) return;
+    if (!t.find(a, MI)) return;
     const int wn = wave % a.NW, wk = wave / a.NW;
     const int c0 = (t.bx * a.NW + wn) * 16 + fr, N = t.N;
     const int K = a.K, nss = a.nks >> 2, col = c0 < N ? c0 : 0;
     const int mtiles = (a.M + 15) >> 4;
     const f16x8* ap[MI];
 #pragma unroll
-    for (int i = 0; i < MI; i++) ap[i] = (const f16x8*)a.xp + (int64_t)min(t.by * MI + i, mtiles - 1) * a.nks * 128 + lane;
+    for (int i = 0; i < MI; i++) ap[i] = (const f16x8*)a.xp + (int64_t)min(t.r16 + i, mtiles - 1) * a.nks * 128 + lane;
     f32x4 acc[NMAT][MI];
 #pragma unroll
     for (int m = 0; m < NMAT; m++)
@@ -681,7 +690,7 @@ __global__ __launch_bounds__(512, 2) void rows16_kernel(RowsArgs a) {
             bf16x8 xg[MI][3];
 #pragma unroll
             for (int i = 0; i < MI; i++) {
-                const bf16x8* gp = (const bf16x8*)a.xg + ((int64_t)min(t.by * MI + i, mtiles - 1) * a.ngw + gw) * 192 + lane;
+                const bf16x8* gp = (const bf16x8*)a.xg + ((int64_t)min(t.r16 + i, mtiles - 1) * a.ngw + gw) * 192 + lane;
 #pragma unroll
                 for (int p = 0; p < 3; p++) xg[i][p] = gld(gp + 64 * p);
             }
@@ -724,8 +733,8 @@ __global__ __launch_bounds__(512, 2) void rows16_kernel(RowsArgs a) {
     if (wk > 0) return;
 #pragma unroll
     for (int i = 0; i < MI; i++) {
-        const int r0 = (t.by * MI + i) * 16 + 4 * f;
-        if (r0 >= a.M) continue;
+        const int r0 = (t.r16 + i) * 16 + 4 * f;
+        if (r0 >= t.mend) continue;
         const f32x4 sc = gld((const f32x4*)(a.xs + r0));
 #pragma unroll
         for (int e = 0; e < 4; e++) finish<NMAT>(a, t, r0 + e, c0, acc[0][i][e] * sc[e], acc[NMAT - 1][i][e] * sc[e]);
@@ -745,7 +754,7 @@ __global__ __launch_bounds__(SH ? 256 : 512, 2) void rows32_kernel(RowsArgs a) {
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int fr = lane & 31, f = lane >> 5;
     Tile t;
-    if (!t.find(a)) return;
+    if (!t.find(a, 2 * R)) return;
     const int wn = wave % a.NW, wk = wave / a.NW;
     const int n0 = (t.bx * a.NW + wn) * 32 * C, N = t.N;
     const int K = a.K, nss = a.nks >> 2, mtiles = (a.M + 15) >> 4;
@@ -826,7 +835,7 @@ __global__ __launch_bounds__(SH ? 256 : 512, 2) void rows32_kernel(RowsArgs a) {
         // chunks of every 16-row tile
         const f16x8* ap[2 * R];
 #pragma unroll
-        for (int i = 0; i < 2 * R; i++) ap[i] = (const f16x8*)a.xp + (int64_t)min(t.by * 2 * R + i, mtiles - 1) * a.nks * 128 + lane;
+        for (int i = 0; i < 2 * R; i++) ap[i] = (const f16x8*)a.xp + (int64_t)min(t.r16 + i, mtiles - 1) * a.nks * 128 + lane;
         f16x8 sr[2 * R][2];
         auto load_s = [&](int ss) {
 #pragma unroll
@@ -868,7 +877,7 @@ __global__ __launch_bounds__(SH ? 256 : 512, 2) void rows32_kernel(RowsArgs a) {
     } else {
         const f16x8* ap[R];
 #pragma unroll
-        for (int i = 0; i < R; i++) ap[i] = (const f16x8*)a.xp + (int64_t)min((t.by * R + i) * 2 + (fr >> 4), mtiles - 1) * a.nks * 128 + lu;
+        for (int i = 0; i < R; i++) ap[i] = (const f16x8*)a.xp + (int64_t)min(t.r16 + 2 * i + (fr >> 4), mtiles - 1) * a.nks * 128 + lu;
         f16x8 af[2][R][2][2];
         auto load_a = [&](f16x8 (&x)[R][2][2], int ks) {
 #pragma unroll
@@ -900,7 +909,7 @@ __global__ __launch_bounds__(SH ? 256 : 512, 2) void rows32_kernel(RowsArgs a) {
             bf16x8 xg[R][3];
 #pragma unroll
             for (int i = 0; i < R; i++) {
-                const bf16x8* gp = (const bf16x8*)a.xg + ((int64_t)min((t.by * R + i) * 2 + (fr >> 4), mtiles - 1) * a.ngw + (g2 >> 1)) * 192 +
+                const bf16x8* gp = (const bf16x8*)a.xg + ((int64_t)min(t.r16 + 2 * i + (fr >> 4), mtiles - 1) * a.ngw + (g2 >> 1)) * 192 +
                                    lu + 32 * (g2 & 1);
 #pragma unroll
                 for (int p = 0; p < 3; p++) xg[i][p] = gld(gp + 64 * p);
@@ -964,8 +973,8 @@ __global__ __launch_bounds__(SH ? 256 : 512, 2) void rows32_kernel(RowsArgs a) {
     for (int i = 0; i < R; i++)
 #pragma unroll
         for (int q = 0; q < 4; q++) {
-            const int r0 = (t.by * R + i) * 32 + 8 * q + 4 * f;
-            if (r0 >= a.M) continue;
+            const int r0 = t.r16 * 16 + 32 * i + 8 * q + 4 * f;
+            if (r0 >= t.mend) continue;
             const f32x4 sc = gld((const f32x4*)(a.xs + r0));
 #pragma unroll
             for (int j = 0; j < C; j++)
@@ -1019,13 +1028,13 @@ __global__ __launch_bounds__(512, 2) void rows_f32_kernel(RowsArgs a) {
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int fr = lane & 15, g = lane >> 4;
     Tile t;
-    if (!t.find(a)) return;
+    if (!t.find(a, MI)) return;
     const int wn = wave % a.NW, wk = wave / a.NW;
     const int n0 = (t.bx * a.NW + wn) * 16 * NJ, N = t.N, K = a.K, nch = (K + 31) >> 5;
     const float* xr[MI];
     const float* wr[NMAT][NJ];
 #pragma unroll
-    for (int i = 0; i < MI; i++) xr[i] = (const float*)a.xp + (int64_t)min((t.by * MI + i) * 16 + fr, a.M - 1) * K;
+    for (int i = 0; i < MI; i++) xr[i] = (const float*)a.xp + (int64_t)min((t.r16 + i) * 16 + fr, a.M - 1) * K;
 #pragma unroll
     for (int m = 0; m < NMAT; m++)
 #pragma unroll
@@ -1133,7 +1142,7 @@ __global__ __launch_bounds__(512, 2) void rows_f32_kernel(RowsArgs a) {
         for (int j = 0; j < NJ; j++)
 #pragma unroll
             for (int e = 0; e < 4; e++)
-                finish<NMAT>(a, t, (t.by * MI + i) * 16 + 4 * g + e, n0 + 16 * j + fr, tot[0][i][j][e], tot[NMAT - 1][i][j][e]);
+                finish<NMAT>(a, t, (t.r16 + i) * 16 + 4 * g + e, n0 + 16 * j + fr, tot[0][i][j][e], tot[NMAT - 1][i][j][e]);
 }
 
 template <int NMAT, int MI, int NJ>
@@ -1146,8 +1155,9 @@ int launch_f32(const RowsArgs& a, hipStream_t st) {
 }
 
 // segments, tile counts and the XCD split of a launch: row tiles of tr rows,
-// column tiles of bn, weight bytes per value
-void plan_tiles(RowsArgs& a, const rina_linear_seg* segs, int nseg, int nmat, int tr, int bn, double wb, bool grouped) {
+// column tiles of bn, weight bytes per value; grouped: most row tiles in use
+// (0: rows not grouped)
+void plan_tiles(RowsArgs& a, const rina_linear_seg* segs, int nseg, int nmat, int tr, int bn, double wb, int grouped) {
     int t = 0;
     for (int s = 0; s < 3; s++) {
         const int ss = s < nseg ? s : 0;
@@ -1159,7 +1169,7 @@ void plan_tiles(RowsArgs& a, const rina_linear_seg* segs, int nseg, int nmat, in
     }
     a.nseg = nseg;
     a.w2 = nmat == 2 ? (const uint8_t*)segs[0].weight2 : nullptr;
-    a.mt = (a.M + tr - 1) / tr;
+    a.mt = grouped ? grouped : (a.M + tr - 1) / tr;
     a.nt = t;
     // the split with the fewest bytes fetched by the 8 L2s: xb x + (8 / xb) W
     // (grouped rows: every group's weights on one XCD)
@@ -1186,11 +1196,11 @@ size_t rows_split_bytes(int qt, int rows, int K) {
     return up256(mt * nks * 2048) + up256(mt * 64) + (qt == RINA_QT_GGML_Q2_K ? mt * ngw * 3072 : 0);
 }
 
-int rows_split(int qt, const float* x, const int* src, int rows, int K, int pro, const float* nw, float eps, void* buf,
+int rows_split(int qt, const float* x, const int* src, const int* used, int rows, int K, int pro, const float* nw, float eps, void* buf,
                RowsX* out, hipStream_t st) {
     const int mt = (rows + 15) / 16;
     SplitXArgs a{};
-    a.x = x; a.nw = nw; a.src = src; a.M = rows; a.K = K; a.pro = pro; a.eps = eps;
+    a.x = x; a.nw = nw; a.src = src; a.used = used; a.M = rows; a.K = K; a.pro = pro; a.eps = eps;
     a.nks = (K + 127) / 128 * 4;
     a.ngw = (K + 511) / 512;
     a.xp = (uint4*)buf;
@@ -1215,8 +1225,7 @@ int rows_split(int qt, const float* x, const int* src, int rows, int K, int pro,
     return hipGetLastError() == hipSuccess ? RINA_OK : RINA_ERR_HIP;
 }
 
-int rows_gemm(const rina_linear_seg* segs, int nseg, int qt, const RowsX& x, int epi, const int* plan, int64_t stride,
-              int rt_plan, hipStream_t st) {
+int rows_gemm(const rina_linear_seg* segs, int nseg, int qt, const RowsX& x, int epi, const RowsPlan* pl, hipStream_t st) {
     const bool two = epi == RINA_EPI_SWIGLU;
     const int nmat = two ? 2 : 1;
     RowsArgs a{};
@@ -1224,13 +1233,13 @@ int rows_gemm(const rina_linear_seg* segs, int nseg, int qt, const RowsX& x, int
     a.M = x.rows; a.K = x.K; a.epi = epi;
     a.nks = (x.K + 127) / 128 * 4;
     a.ngw = (x.K + 511) / 512;
-    a.plan = plan;
-    a.stride = stride;
+    a.plan = pl ? pl->plan : nullptr;
+    a.stride = pl ? pl->stride : 0;
     const int nss = a.nks / 4;
     // row tiles of 16, 32 or 64 rows (rt 0, 1, 2); columns per wave: 16, or 32 ct at 64 rows
-    const int rt = plan ? rt_plan : x.rows <= 16 ? 0 : x.rows <= 32 ? 1 : 2;
+    const int rt = pl ? pl->rt : x.rows <= 16 ? 0 : x.rows <= 32 ? 1 : 2;
     const int tr = 16 << rt, tc = rt < 2 ? 16 : 32;
-    const int64_t mts = (x.rows + tr - 1) / tr;
+    const int64_t mts = pl ? pl->tiles_est : (x.rows + tr - 1) / tr;
     auto tiles = [&](int ct) {
         int64_t t = 0;
         for (int s = 0; s < nseg; s++) t += (segs[s].N + tc * ct - 1) / (tc * ct);
@@ -1245,7 +1254,7 @@ int rows_gemm(const rina_linear_seg* segs, int nseg, int qt, const RowsX& x, int
     a.KW = kw;
     a.NW = kw >= 4 ? 1 : 4 / kw;
     const int BN = tc * nj * a.NW;
-    plan_tiles(a, segs, nseg, nmat, tr, BN, qt == RINA_QT_Q4_0F ? 0.625 : qt == RINA_QT_GGML_Q2_K ? 84.0 / 256 : 0.5625, plan);
+    plan_tiles(a, segs, nseg, nmat, tr, BN, qt == RINA_QT_Q4_0F ? 0.625 : qt == RINA_QT_GGML_Q2_K ? 84.0 / 256 : 0.5625, pl ? pl->tiles_max : 0);
     if (qt == RINA_QT_Q4_0) return launch_fmt<FMT_Q4_0>(a, nmat, rt, nj, st);
     if (qt == RINA_QT_Q4_0F) return launch_fmt<FMT_Q4_0F>(a, nmat, rt, nj, st);
     return x.K % 128 == 0 ? launch_fmt<FMT_Q2_K>(a, nmat, rt, nj, st) : launch_fmt<FMT_Q2_S>(a, nmat, rt, nj, st);
@@ -1277,7 +1286,7 @@ int rows_f32(const rina_linear_seg* segs, int nseg, const float* x, int M, int K
     while (kw < 8 && tiles() * kw < 2 * simds && K >= 256 * kw) kw *= 2;
     a.KW = kw;
     a.NW = kw >= 4 ? 1 : 4 / kw;
-    plan_tiles(a, segs, nseg, nmat, 16 * mi, 16 * nj * a.NW, 4.0, false);
+    plan_tiles(a, segs, nseg, nmat, 16 * mi, 16 * nj * a.NW, 4.0, 0);
     if (nmat == 2) {
         if (mi == 4) return launch_f32<2, 4, 1>(a, st);
         if (mi == 2) return nj == 1 ? launch_f32<2, 2, 1>(a, st) : launch_f32<2, 2, 2>(a, st);

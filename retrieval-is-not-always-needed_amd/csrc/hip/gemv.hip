@@ -1405,9 +1405,9 @@ extern "C" int rina_hip_linear_fused_ex(const rina_linear_seg* segs, int nseg, i
         void* buf = rina_scratch(rows_split_bytes(qt, M, K), st, kScratchRows);
         if (!buf) return RINA_ERR_HIP;
         RowsX xr;
-        int rc = rows_split(qt, input, nullptr, M, K, pro, nw, eps, buf, &xr, st);
+        int rc = rows_split(qt, input, nullptr, nullptr, M, K, pro, nw, eps, buf, &xr, st);
         for (int s0 = 0; s0 < nseg && rc == RINA_OK; s0 += 3)
-            rc = rows_gemm(segs + s0, nseg - s0 < 3 ? nseg - s0 : 3, qt, xr, epi, nullptr, 0, 0, st);
+            rc = rows_gemm(segs + s0, nseg - s0 < 3 ? nseg - s0 : 3, qt, xr, epi, nullptr, st);
         return rc;
     }
     int unit = qt == RINA_QT_GGML_Q2_K ? 16 : 32;

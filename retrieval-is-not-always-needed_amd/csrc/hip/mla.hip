@@ -26,6 +26,7 @@
 #include <vector>
 #include "rina_common.hpp"
 #include "attn_rows.hpp"
+#include "rows_gemm.hpp"
 
 namespace {
 
@@ -1136,6 +1137,82 @@ __global__ __launch_bounds__(256) void moe_topk_kernel(const float* lg, int E, i
     }
 }
 
+// The rows of a prompt's MoE block grouped by expert on the device, one
+// workgroup: expert e's rows take 16-row tiles of their own, in expert order.
+// src[slot] = the slot's row (-1: padding), slot_of[t k + j] = the slot of row
+// t's j-th selection, and the row tiles of 16 << rt rows (RowsPlan).  The order
+// of an expert's rows is not fixed; no result depends on it.
+__global__ __launch_bounds__(1024) void moe_plan_kernel(const int* ids, int tk, int k, int E, int rt, int* plan, int* src,
+                                                        int* slot_of) {
+    __shared__ int s_cnt[256], s_off[257], s_tile[257];
+    const int tid = threadIdx.x;
+    if (tid < 256) s_cnt[tid] = 0;
+    __syncthreads();
+    // ids outside the experts (a router row of NaN selects none) take no slot
+    for (int i = tid; i < tk; i += 1024) {
+        const int e = gld(ids + i);
+        if (e >= 0 && e < E) atomicAdd(&s_cnt[e], 1);
+    }
+    __syncthreads();
+    if (tid == 0) {
+        int o = 0, t = 0;
+        for (int e = 0; e < E; e++) {
+            s_off[e] = o;
+            s_tile[e] = t;
+            o += (s_cnt[e] + 15) >> 4;
+            t += (s_cnt[e] + (16 << rt) - 1) >> (4 + rt);
+        }
+        s_off[E] = o;
+        s_tile[E] = t;
+        gst(plan, t);
+        gst(plan + 1, o);
+    }
+    __syncthreads();
+    if (tid < E) {
+        const int o = s_off[tid], n = s_cnt[tid];
+        for (int i = 0; i < s_tile[tid + 1] - s_tile[tid]; i++) {
+            int* p = plan + 2 + 3 * (s_tile[tid] + i);
+            gst(p, tid);
+            gst(p + 1, o + (i << rt));
+            gst(p + 2, 16 * o + min(n, (i + 1) * (16 << rt)));
+        }
+        for (int i = n; i < 16 * (s_off[tid + 1] - o); i++) gst(src + 16 * o + i, -1);
+    }
+    __syncthreads();
+    if (tid < 256) s_cnt[tid] = 0;
+    __syncthreads();
+    for (int i = tid; i < tk; i += 1024) {
+        const int e = gld(ids + i);
+        const bool on = e >= 0 && e < E;
+        const int s = on ? 16 * s_off[e] + atomicAdd(&s_cnt[e], 1) : -1;
+        if (on) gst(src + s, i / k);
+        gst(slot_of + i, s);
+    }
+}
+
+// h[t] += sum_j probs[t k + j] Y[slot_of[t k + j]], ascending j: grid T, d / 4 threads' worth of float4 columns
+__global__ __launch_bounds__(256) void moe_combine_rows_kernel(float* h, const float* Y, const int* slot_of, const float* probs,
+                                                               int k, int d) {
+    const int t = blockIdx.x;
+    float* hr = h + (int64_t)t * d;
+    for (int c = 4 * threadIdx.x; c < d; c += 1024) {
+        float v[4];
+#pragma unroll
+        for (int e = 0; e < 4; e++) v[e] = c + e < d ? gld(hr + c + e) : 0.f;
+        for (int j = 0; j < k; j++) {
+            const int s = gld(slot_of + (int64_t)t * k + j);
+            if (s < 0) continue;
+            const float* y = Y + (int64_t)s * d + c;
+            const float p = gld(probs + (int64_t)t * k + j);
+#pragma unroll
+            for (int e = 0; e < 4; e++) v[e] = fmaf(p, c + e < d ? gld(y + e) : 0.f, v[e]);
+        }
+#pragma unroll
+        for (int e = 0; e < 4; e++)
+            if (c + e < d) gst(hr + c + e, v[e]);
+    }
+}
+
 // prompt rows of the MoE block, grouped by expert: X[i] = a2[idx[i]]
 __global__ __launch_bounds__(256) void moe_gather_kernel(const float* a2, const int* idx, int d, float* X) {
     const float* src = a2 + (int64_t)gld(idx + blockIdx.x) * d;
@@ -1445,14 +1522,61 @@ extern "C" size_t rina_hip_moe_workspace(int k, int ffn) { return (size_t)k * ff
 // The MoE block over a prompt's T rows (forward_moe, deepseek_mla_layer.cu:
 // 291-350, for every row at once): the rows' ln2 norm and fp32 router
 // logits as T-row products, the top-k of every row, the shared experts as
-// T-row products added to h, then one expert at a time (ascending id) its
-// selected rows gathered, its gate/up (SiLU * up) and down products over
-// them, and h[row] += p * y.  The selection comes to the host once to group
-// the rows (the stream is synchronized there).
+// T-row products added to h, then the routed experts: grouped on the device
+// (moe_grouped), or, for expert formats and widths the rows product does not
+// take, one expert at a time (ascending id) its selected rows gathered, its
+// gate/up (SiLU * up) and down products over them, and h[row] += p * y; the
+// selection then comes to the host once to group the rows (the stream is
+// synchronized there).
 // ---------------------------------------------------------------------------
 namespace {
 size_t up4f(size_t n) { return (n + 3) / 4 * 4; }
 }
+
+namespace {
+// The routed experts of a prompt's rows without leaving the device: the rows
+// grouped by expert (moe_plan_kernel), split once in that order, one grouped
+// product for every expert's gate/up (SiLU * up), its result split, one for
+// every down, and the weighted rows added to h.  Six launches instead of four
+// or more per expert and a host round trip: 512 rows, 64 experts top 6,
+// 2048 x 1408 Q2_K: the block 3.30 ms that way, 450 us grouped.
+int moe_grouped(float* h, const float* a2, const int* ids, const float* probs, const void* wg, const void* wu, const void* wd,
+                int qt, int64_t stride_gu, int64_t stride_dn, int T, int E, int k, int d, int F, hipStream_t st) {
+    const size_t tk = (size_t)T * k, groups = std::min((size_t)E, tk);
+    const size_t slots = (tk + 15 * groups + 15) / 16 * 16;      // every group padded to 16-row tiles
+    const size_t per = (tk + groups - 1) / groups;               // rows of an average expert
+    const int rt = per <= 16 ? 0 : per <= 32 ? 1 : 2;
+    const size_t tmax = tk / (16 << rt) + groups;
+    auto up = [](size_t n) { return (n + 255) & ~(size_t)255; };
+    const size_t b_x = up(std::max(rows_split_bytes(qt, (int)slots, d), slots * d * 4));   // split rows, later Y
+    const size_t b_g = up(slots * F * 4), b_gx = up(rows_split_bytes(qt, (int)slots, F));
+    const size_t b_p = up((2 + 3 * tmax) * 4), b_s = up(slots * 4), b_o = up(tk * 4);
+    char* p = (char*)rina_scratch(b_x + b_g + b_gx + b_p + b_s + b_o, st, kScratchMoe);
+    if (!p) return RINA_ERR_HIP;
+    void* xb = p;
+    float* G = (float*)(p + b_x);
+    void* gb = p + b_x + b_g;
+    int* plan = (int*)((char*)gb + b_gx);
+    int* src = (int*)((char*)plan + b_p);
+    int* slot_of = (int*)((char*)src + b_s);
+    hipLaunchKernelGGL(moe_plan_kernel, dim3(1), dim3(1024), 0, st, ids, (int)tk, k, E, rt, plan, src, slot_of);
+    RINA_LAUNCH_CHECK();
+    RowsX x;
+    int rc = rows_split(qt, a2, src, plan + 1, (int)slots, d, RINA_PRO_NONE, nullptr, 0.f, xb, &x, st);
+    if (rc) return rc;
+    RowsPlan pl{plan, stride_gu, rt, (int)tmax, (int)std::max(groups, tk / (16 << rt))};
+    rina_linear_seg sg{wg, wu, G, F};
+    if ((rc = rows_gemm(&sg, 1, qt, x, RINA_EPI_SWIGLU, &pl, st))) return rc;
+    if ((rc = rows_split(qt, G, nullptr, plan + 1, (int)slots, F, RINA_PRO_NONE, nullptr, 0.f, gb, &x, st))) return rc;
+    pl.stride = stride_dn;
+    float* Y = (float*)xb;
+    rina_linear_seg sd{wd, nullptr, Y, d};
+    if ((rc = rows_gemm(&sd, 1, qt, x, RINA_EPI_STORE, &pl, st))) return rc;
+    hipLaunchKernelGGL(moe_combine_rows_kernel, dim3(T), dim3(256), 0, st, h, Y, slot_of, probs, k, d);
+    RINA_LAUNCH_CHECK();
+    return RINA_OK;
+}
+}  // namespace
 
 extern "C" size_t rina_hip_moe_rows_workspace(int T, int d, int E, int k, int F, int S) {
     if (T < 1 || d < 1 || E < 1 || k < 1 || F < 1 || S < 0) return 0;
@@ -1499,6 +1623,8 @@ extern "C" int rina_hip_moe_rows(float* h, int T, const float* ln2, float eps, c
         if ((rc = rina_hip_linear_fused(&sd, 1, qt_sh, gsh, T, S, RINA_EPI_ADD, RINA_PRO_NONE, nullptr, 0.f, stream)))
             return rc;
     }
+    if (rows_gemm_ok(qt_exps, d) && rows_gemm_ok(qt_exps, F))
+        return moe_grouped(h, a2, ids, probs, gate_exps, up_exps, down_exps, qt_exps, stride_gu, stride_dn, T, E, k, d, F, st);
     // the selection on the host: rows grouped by expert, ascending
     std::vector<int> hid(tk);
     std::vector<float> hpr(tk);

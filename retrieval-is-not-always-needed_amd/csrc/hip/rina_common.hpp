@@ -183,10 +183,10 @@ int rina_num_cus();
 // Scratch owned by the library, one buffer per (device, stream, use), grown
 // on demand and never shrunk: the output of a call that aliases input and
 // output, the row of a norm that runs before a matvec as its own launch, the
-// split activation rows of a product over several rows.  The uses of one call
-// nest, so each has a buffer of its own; calls on one stream run in order and
+// split activation rows of a product over several rows, the grouped rows of a
+// MoE block.  The uses of one call nest, so each has a buffer of its own; calls on one stream run in order and
 // share them.
-enum { kScratchOut = 0, kScratchNorm = 1, kScratchRows = 2 };
+enum { kScratchOut = 0, kScratchNorm = 1, kScratchRows = 2, kScratchMoe = 3 };
 void* rina_scratch(size_t bytes, hipStream_t stream, int use);
 
 __device__ __forceinline__ int read_pos(int start_pos, const int* d_pos) {

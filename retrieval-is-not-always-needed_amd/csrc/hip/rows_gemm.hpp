@@ -16,14 +16,24 @@ bool rows_gemm_ok(int qt, int K);
 size_t rows_split_bytes(int qt, int rows, int K);
 // x [.., K] -> fragments in buf (rows_split_bytes, 256-byte aligned), with the
 // norm prologue; src != NULL: packed row r is x row src[r], a zero row where
-// src[r] < 0 (src holds whole 16-row tiles)
-int rows_split(int qt, const float* x, const int* src, int rows, int K, int pro, const float* nw, float eps, void* buf,
-               RowsX* out, hipStream_t st);
-// up to 3 segments of one quant type; plan != NULL: grouped rows, plan[0] row
-// tiles (16, 32 or 64 rows: rt_plan 0, 1, 2) in use, plan[1 + i] the group of tile i, whose
-// weights start group * stride bytes into the segment
-int rows_gemm(const rina_linear_seg* segs, int nseg, int qt, const RowsX& x, int epi, const int* plan, int64_t stride,
-              int rt_plan, hipStream_t st);
+// src[r] < 0 (src holds whole 16-row tiles); used != NULL: only the first
+// *used 16-row tiles
+int rows_split(int qt, const float* x, const int* src, const int* used, int rows, int K, int pro, const float* nw,
+               float eps, void* buf, RowsX* out, hipStream_t st);
+
+// Rows grouped by weight matrix (experts), planned on the device: plan[0] row
+// tiles in use, plan[1] 16-row tiles in use, then three ints per row tile: its
+// group (whose weights start group * stride bytes into the segment), its first
+// 16-row tile, its row limit.  A tile may run past its limit into the next
+// group's rows: those outputs are not stored.
+struct RowsPlan {
+    const int* plan;
+    int64_t stride;
+    int rt;                // rows per tile: 16 << rt
+    int tiles_max, tiles_est;   // most row tiles in use, an estimate
+};
+// up to 3 segments of one quant type (grouped: 1)
+int rows_gemm(const rina_linear_seg* segs, int nseg, int qt, const RowsX& x, int epi, const RowsPlan* pl, hipStream_t st);
 
 // fp32 weights: rows and weights 16-byte aligned, K % 4 == 0; M >= 2, up to 3 segments
 bool rows_f32_ok(const rina_linear_seg* segs, int nseg, const float* x, int K);

@@ -131,3 +131,62 @@ def test_rows_product_under_capture(rina, orc):
         g.replay()
         torch.cuda.synchronize()
         assert_close(host(y).reshape(M, N), ref, what="replay %d" % k)
+
+
+@pytest.mark.parametrize("qt", [7, 10, 6])
+@pytest.mark.parametrize("T,E,k,d,F,S", [(150, 4, 2, 256, 96, 128), (61, 8, 3, 128, 160, 0), (5, 16, 4, 256, 64, 64)])
+def test_moe_rows_groups(rina, orc, qt, T, E, k, d, F, S):
+    """The MoE block over rows grouped by expert against float64: groups of
+    more than one 64-row tile, of 16-row tiles, an expert no row selects (its
+    router row loses everywhere), no shared experts; a row of NaN selects
+    nothing and leaves the other rows alone."""
+    hip = rina.load_hip()
+    r = rng(T + E + d + qt)
+    ex = {n: [weights(orc, qt, r, F * d) for _ in range(E)] for n in ("g", "u", "dn")}
+    packed = {n: np.concatenate([w for w, _ in ex[n]]) for n in ex}
+    sh = [weights(orc, qt, r, S * d) for _ in range(3)] if S else [(None, None)] * 3
+    wr = (r.standard_normal((E, d)) * 0.2).astype(np.float32)
+    ln2 = r.uniform(0.8, 1.2, d).astype(np.float32)
+    h0 = (r.standard_normal((T, d)) * 2).astype(np.float32)
+    h0[:, 0] = 40.0                          # a common component that expert E - 1's router row opposes
+    wr[E - 1, 0] = -20.0
+    bad = T // 2
+    h0[bad, 3] = np.nan
+    hd = dev(h0)
+    keep = [dev(x) for x in (ln2, wr, packed["g"], packed["u"], packed["dn"])]
+    shd = [dev(w) if S else None for w, _ in sh]
+    ptr = [x.data_ptr() if x is not None else None for x in shd]
+    sb = packed["g"].nbytes // E
+    wb = hip.rina_hip_moe_rows_workspace(T, d, E, k, F, S)
+    ws = empty(wb // 4 + 4)
+    ok(hip.rina_hip_moe_rows(hd.data_ptr(), T, keep[0].data_ptr(), np.float32(1e-5), keep[1].data_ptr(), 6, *ptr, S, qt,
+                             keep[2].data_ptr(), keep[3].data_ptr(), keep[4].data_ptr(), qt, sb, packed["dn"].nbytes // E,
+                             E, k, d, F, ws.data_ptr(), wb, stream()), "moe rows")
+    got = host(hd).reshape(T, d)
+
+    def silu(v):
+        return v / (1 + np.exp(-v))
+
+    h = h0.astype(np.float64)
+    seen = 0
+    for t in range(T):
+        if t == bad:
+            continue
+        a = h[t] / np.sqrt((h[t] ** 2).mean() + 1e-5) * ln2
+        lg = wr.astype(np.float64) @ a
+        p = np.exp(lg - lg.max())
+        p /= p.sum()
+        order = np.argsort(-p, kind="stable")
+        assert E - 1 not in order[:k]
+        if p[order[k - 1]] - p[order[k]] < 1e-5:
+            continue                         # a tie the fp32 router may break the other way
+        ref = h[t].copy()
+        if S:
+            G, U, D = (W for _, W in sh)
+            ref += D.reshape(d, S) @ (silu(G.reshape(S, d) @ a) * (U.reshape(S, d) @ a))
+        for e in order[:k]:
+            g, u = (ex[n][e][1].reshape(F, d) @ a for n in ("g", "u"))
+            ref += p[e] * (ex["dn"][e][1].reshape(d, F) @ (silu(g) * u))
+        assert_close(got[t], ref, what="row %d" % t)
+        seen += 1
+    assert seen >= T * 3 // 4
