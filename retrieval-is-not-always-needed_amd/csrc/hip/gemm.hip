@@ -34,6 +34,7 @@
 // waves of a workgroup (NW across columns, KW along K, interleaved by 128
 // values) never wait for each other; the KW partial tiles meet in LDS once
 // at the end.
+#include <type_traits>
 #include "rina_common.hpp"
 #include "rows_gemm.hpp"
 
@@ -370,6 +371,21 @@ __device__ __forceinline__ u32x4 q2_unpack(u32x2 b, uint32_t by, int st) {
                  f16_fma(f16_field(b.y, mask), sc, m), f16_fma(f16_field(b.y >> 8, mask), sc, m)};
 }
 
+// nibble dwords and fp32 scale of a Q4 block from the five dwords at its
+// (4-byte aligned down) start; odd: a Q4_0 block that starts two bytes in
+template <int FMT>
+__device__ __forceinline__ void q4_dwords(const uint32_t (&d)[5], bool odd, uint32_t (&n)[4], uint32_t& s) {
+    if constexpr (FMT == FMT_Q4_0F) {
+        s = d[0];
+#pragma unroll
+        for (int i = 0; i < 4; i++) n[i] = d[1 + i];
+    } else {
+#pragma unroll
+        for (int i = 0; i < 4; i++) n[i] = odd ? d[1 + i] : __builtin_amdgcn_alignbyte(d[1 + i], d[i], 2);
+        s = __float_as_uint(f16_to_f32((odd ? d[0] >> 16 : d[0]) & 0xFFFFu));
+    }
+}
+
 // nibble dwords and fp32 scale of one loaded Q4 block
 template <int FMT>
 __device__ __forceinline__ void q4_block(const WRaw<FMT>& r, uint32_t (&n)[4], uint32_t& s) {
@@ -512,20 +528,13 @@ __device__ __forceinline__ void finish(const RowsArgs& a, const Tile& t, int r, 
 template <int FMT>
 struct WRaw32;
 template <>
-struct WRaw32<FMT_Q4_0F> { WRaw<FMT_Q4_0F> b[2]; };
-template <>
-struct WRaw32<FMT_Q4_0> { WRaw<FMT_Q4_0> b[2]; };
-template <>
 struct WRaw32<FMT_Q2_K> { u32x2 q[2], s; uint32_t d; };
 template <>
 struct WRaw32<FMT_Q2_S> { u32x2 q[4][2]; uint32_t s[4], d[4]; };
 
 template <int FMT>
 __device__ __forceinline__ void w_load32(const uint8_t* w, int n, int K, int ss, int f, WRaw32<FMT>& r) {
-    if constexpr (FMT == FMT_Q4_0F || FMT == FMT_Q4_0) {
-        w_load<FMT>(w, n, K, ss, f, r.b[0]);
-        w_load<FMT>(w, n, K, ss, f + 2, r.b[1]);
-    } else if constexpr (FMT == FMT_Q2_K) {
+    if constexpr (FMT == FMT_Q2_K) {
         const int64_t pg = (int64_t)n * (K >> 7) + ss;
         const uint8_t* b = w + (pg >> 1) * 84;
         const int o = (int)(pg & 1);
@@ -554,22 +563,25 @@ struct WStep32 {
     float sc[4];
     u32x2 q[FMT == FMT_Q2_S ? 4 : 1][2];
     uint32_t s[4];
-    __device__ __forceinline__ void take(const WRaw32<FMT>& r) {
-        if constexpr (FMT == FMT_Q4_0F || FMT == FMT_Q4_0) {
+    // Q4: blocks 2 b + f of the column, five dwords each (d[b])
+    __device__ __forceinline__ void take_q4(const uint32_t (&d)[2][5], bool odd) {
 #pragma unroll
-            for (int b = 0; b < 2; b++) {           // lane row 0 holds block 2 b, lane row 1 block 2 b + 1
-                uint32_t x[4], s1;
-                q4_block<FMT>(r.b[b], x, s1);
-                // [own d0, d1 of the lower row | d0, d1 of the upper row]: lane row f gets dword f (and 2 + f)
-                const auto lo = __builtin_amdgcn_permlane32_swap(x[0], x[1], false, false);
-                const auto hi = __builtin_amdgcn_permlane32_swap(x[2], x[3], false, false);
-                const auto sp = __builtin_amdgcn_permlane32_swap(s1, s1, false, false);
-                n[2 * b][0] = lo[0]; n[2 * b + 1][0] = lo[1];
-                n[2 * b][1] = hi[0]; n[2 * b + 1][1] = hi[1];
-                sc[2 * b] = __uint_as_float(sp[0]);
-                sc[2 * b + 1] = __uint_as_float(sp[1]);
-            }
-        } else if constexpr (FMT == FMT_Q2_K) {
+        for (int b = 0; b < 2; b++) {               // lane row 0 holds block 2 b, lane row 1 block 2 b + 1
+            uint32_t x[4], s1;
+            q4_dwords<FMT>(d[b], odd, x, s1);
+            // [own d0, d1 of the lower row | d0, d1 of the upper row]: lane row f gets dword f (and 2 + f)
+            const auto lo = __builtin_amdgcn_permlane32_swap(x[0], x[1], false, false);
+            const auto hi = __builtin_amdgcn_permlane32_swap(x[2], x[3], false, false);
+            const auto sp = __builtin_amdgcn_permlane32_swap(s1, s1, false, false);
+            n[2 * b][0] = lo[0]; n[2 * b + 1][0] = lo[1];
+            n[2 * b][1] = hi[0]; n[2 * b + 1][1] = hi[1];
+            sc[2 * b] = __uint_as_float(sp[0]);
+            sc[2 * b + 1] = __uint_as_float(sp[1]);
+        }
+    }
+    template <typename Raw>
+    __device__ __forceinline__ void take(const Raw& r) {
+        if constexpr (FMT == FMT_Q2_K) {
             q[0][0] = r.q[0]; q[0][1] = r.q[1];
             s[0] = r.s.x; s[1] = r.s.x >> 16; s[2] = r.s.y; s[3] = r.s.y >> 16;
             sc[0] = f16_to_f32(r.d);
@@ -742,14 +754,19 @@ __global__ __launch_bounds__(512, 2) void rows16_kernel(RowsArgs a) {
 }
 
 // ---- M > 32: v_mfma_f32_32x32x16_f16 tiles ----
-// A wave owns 32 R rows x 32 C columns (per matrix).  SH: the 4 waves of a
-// workgroup take neighbouring columns over the whole of K and share the rows'
-// fragments through LDS (two buffers of a 128-value step); else every wave
-// reads its rows' fragments itself and KW waves split K.
-template <int FMT, int NMAT, int R, int C, bool SH>
-__global__ __launch_bounds__(SH ? 256 : 512, 2) void rows32_kernel(RowsArgs a) {
+// A wave owns 32 R rows x 32 C columns (per matrix) of its K slice.  Q4 weights
+// pass through a buffer of the wave's own in LDS: the 80 (72) bytes of a
+// column's 128-value step are loaded as five 16-byte chunks by neighbouring
+// lanes and read back block by block (no barrier: only this wave uses it).
+// Loaded block by block straight into the lanes that use them, every 20-byte
+// block costs two address slots of the load unit, and the weights alone took
+// 39 of the 85 us of a 512 x 2048 x 8192 gate/up launch.
+template <int FMT, int NMAT, int R, int C>
+__global__ __launch_bounds__(512, 2) void rows32_kernel(RowsArgs a) {
     extern __shared__ __align__(16) float s_part[];
-    __shared__ __align__(16) f16x8 s_a[SH ? 2 : 1][SH ? 2 * R : 1][SH ? 8 : 1][64];
+    constexpr bool Q4 = FMT == FMT_Q4_0F || FMT == FMT_Q4_0;
+    constexpr int NCOL = 32 * NMAT * C, NCH = (5 * NCOL + 63) / 64;   // column rows, 16-byte chunks per lane
+    __shared__ __align__(16) u32x4 s_w[Q4 ? 8 : 1][Q4 ? 64 * NCH : 1];
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int fr = lane & 31, f = lane >> 5;
@@ -770,12 +787,36 @@ __global__ __launch_bounds__(SH ? 256 : 512, 2) void rows32_kernel(RowsArgs a) {
             for (int j = 0; j < C; j++)
 #pragma unroll
                 for (int e = 0; e < 16; e++) acc[m][i][j][e] = 0.f;
-    WRaw32<FMT> raw[NMAT][C];
+    typename std::conditional<Q4, char, WRaw32<Q4 ? FMT_Q2_K : FMT>>::type raw[NMAT][C];
+    // Q4: chunk i of this lane is bytes 16 c .. of column row q / 5, q = 64 i + lane, c = q % 5
+    constexpr int BB = FMT == FMT_Q4_0F ? 20 : 18;
+    const int nb = K >> 5;
+    u32x4 ch[Q4 ? NCH : 1];
+    const uint8_t* cw[Q4 ? NCH : 1];                // the chunk at step 0 (4-byte aligned)
+    int64_t cmax[Q4 ? NCH : 1];                     // the last offset from there that stays inside the matrix,
+    int cpull[Q4 ? NCH : 1];                        // and what it was pulled back by at step 0
+    if constexpr (Q4) {
+#pragma unroll
+        for (int i = 0; i < NCH; i++) {
+            const int q = min(64 * i + lane, 5 * NCOL - 1), cr = q / 5, c = q - 5 * cr;
+            const int m = cr / (32 * C), n = min(n0 + cr % (32 * C), N - 1);
+            const int64_t off = (((int64_t)n * nb * BB) & ~(int64_t)3) + 16 * c;
+            const int64_t last = (int64_t)N * nb * BB - 16;
+            cw[i] = (m ? t.w2 : t.w) + min(off, last);
+            cmax[i] = last - min(off, last);
+            cpull[i] = (int)(off - min(off, last));
+        }
+    }
     auto load_w = [&](int ss) {
+        if constexpr (Q4) {
 #pragma unroll
-        for (int m = 0; m < NMAT; m++)
+            for (int i = 0; i < NCH; i++) ch[i] = gld4(cw[i] + min((int64_t)ss * (4 * BB), cmax[i]));
+        } else {
 #pragma unroll
-            for (int j = 0; j < C; j++) w_load32<FMT>(m ? t.w2 : t.w, col[j], K, ss, f, raw[m][j]);
+            for (int m = 0; m < NMAT; m++)
+#pragma unroll
+                for (int j = 0; j < C; j++) w_load32<FMT>(m ? t.w2 : t.w, col[j], K, ss, f, raw[m][j]);
+        }
     };
     // fragment of 32-row tile i, 16-value half h, part p of a 32-value step:
     // 16-row tile 2 i + (row / 16), lane row 2 h + f of its 64-unit chunk
@@ -824,57 +865,61 @@ __global__ __launch_bounds__(SH ? 256 : 512, 2) void rows32_kernel(RowsArgs a) {
                 }
             }
     };
-    auto take = [&](WStep32<FMT> (&ws)[NMAT][C]) {
+    bool edge = false;                              // a chunk of this wave ends past the matrix in the last step
+    if constexpr (Q4) {
 #pragma unroll
-        for (int m = 0; m < NMAT; m++)
+        for (int i = 0; i < NCH; i++) edge |= cpull[i] > 0 || cmax[i] < (int64_t)(nss - 1) * (4 * BB);
+        edge = __any(edge);
+    }
+    auto take = [&](WStep32<FMT> (&ws)[NMAT][C], int ss) {
+        if constexpr (Q4) {
+            u32x4* wb = s_w[wave];
+            if (!edge || ss < nss - 1) {
 #pragma unroll
-            for (int j = 0; j < C; j++) ws[m][j].take(raw[m][j]);
-    };
-    if constexpr (SH) {
-        // wave wn moves a quarter of a step: two of the eight (step, part)
-        // chunks of every 16-row tile
-        const f16x8* ap[2 * R];
+                for (int i = 0; i < NCH; i++) wb[64 * i + lane] = ch[i];
+            } else {
+                // chunks that were pulled back into the matrix go where their bytes
+                // belong (over the chunk before, with the same bytes; a step has
+                // one block at least, so never before the row's first)
 #pragma unroll
-        for (int i = 0; i < 2 * R; i++) ap[i] = (const f16x8*)a.xp + (int64_t)min(t.r16 + i, mtiles - 1) * a.nks * 128 + lane;
-        f16x8 sr[2 * R][2];
-        auto load_s = [&](int ss) {
+                for (int i = 0; i < NCH; i++) {
+                    const int64_t back = (int64_t)ss * (4 * BB) + cpull[i] - cmax[i];
+                    uint16_t* d = (uint16_t*)(wb + 64 * i + lane) - (back > 0 ? back / 2 : 0);   // (18-byte blocks: an even count)
+                    const uint32_t v[4] = {ch[i].x, ch[i].y, ch[i].z, ch[i].w};
 #pragma unroll
-            for (int i = 0; i < 2 * R; i++)
-#pragma unroll
-                for (int c = 0; c < 2; c++) sr[i][c] = gld(ap[i] + (int64_t)ss * 512 + (2 * wn + c) * 64);
-        };
-        auto store_s = [&](int buf) {
-#pragma unroll
-            for (int i = 0; i < 2 * R; i++)
-#pragma unroll
-                for (int c = 0; c < 2; c++) s_a[buf][i][2 * wn + c][lane] = sr[i][c];
-        };
-        load_s(0);
-        load_w(0);
-        store_s(0);
-        __syncthreads();
-        for (int ss = 0; ss < nss; ss++) {
-            const int sn = ss + 1 < nss ? ss + 1 : ss;     // the last step loads itself again
-            load_s(sn);
-            WStep32<FMT> ws[NMAT][C];
-            take(ws);
-            load_w(sn);
-            __builtin_amdgcn_sched_barrier(0);      // issued before this step's products
-#pragma unroll
-            for (int st = 0; st < 4; st++) {
-                f16x8 at[R][2][2];
-#pragma unroll
-                for (int i = 0; i < R; i++)
-#pragma unroll
-                    for (int h = 0; h < 2; h++)
-#pragma unroll
-                        for (int p = 0; p < 2; p++) at[i][h][p] = s_a[ss & 1][2 * i + (fr >> 4)][2 * st + p][lu + 32 * h];
-                mul(ws, at, st);
+                    for (int k = 0; k < 4; k++) { d[2 * k] = (uint16_t)v[k]; d[2 * k + 1] = (uint16_t)(v[k] >> 16); }
+                }
             }
-            store_s((ss & 1) ^ 1);                  // that buffer's readers are past the last barrier
-            __syncthreads();
+            __builtin_amdgcn_wave_barrier();
+#pragma unroll
+            for (int m = 0; m < NMAT; m++)
+#pragma unroll
+                for (int j = 0; j < C; j++) {
+                    // a row that starts two bytes past a dword (Q4_0, odd n nb): its blocks shift by two
+                    const uint32_t* r = (const uint32_t*)wb + 20 * (32 * (m * C + j) + fr);
+                    const int lead = FMT == FMT_Q4_0 ? 2 * ((col[j] & nb) & 1) : 0;
+                    uint32_t d[2][5];
+                    const bool odd = FMT == FMT_Q4_0 && ((lead + BB * f) & 2);
+#pragma unroll
+                    for (int b = 0; b < 2; b++)
+#pragma unroll
+                        for (int i = 0; i < 5; i++) d[b][i] = r[min((lead + BB * (2 * b + f)) / 4 + i, 19)];
+                    ws[m][j].take_q4(d, odd);
+                    if (4 * ss + 4 > nb) {          // blocks past the row: x is zero there, their bytes may be anything
+#pragma unroll
+                        for (int b = 0; b < 4; b++)
+                            if (4 * ss + b >= nb) ws[m][j].sc[b] = 0.f;
+                    }
+                }
+            __builtin_amdgcn_wave_barrier();
+        } else {
+#pragma unroll
+            for (int m = 0; m < NMAT; m++)
+#pragma unroll
+                for (int j = 0; j < C; j++) ws[m][j].take(raw[m][j]);
         }
-    } else {
+    };
+    {
         const f16x8* ap[R];
 #pragma unroll
         for (int i = 0; i < R; i++) ap[i] = (const f16x8*)a.xp + (int64_t)min(t.r16 + 2 * i + (fr >> 4), mtiles - 1) * a.nks * 128 + lu;
@@ -894,7 +939,7 @@ __global__ __launch_bounds__(SH ? 256 : 512, 2) void rows32_kernel(RowsArgs a) {
         for (int ss = wk; ss < nss; ss += a.KW) {
             const int sn = ss + a.KW < nss ? ss + a.KW : ss;   // the last step loads itself again
             WStep32<FMT> ws[NMAT][C];
-            take(ws);
+            take(ws, ss);
 #pragma unroll
             for (int st = 0; st < 4; st++) {
                 load_a(af[(st & 1) ^ 1], st < 3 ? 4 * ss + st + 1 : 4 * sn);
@@ -932,7 +977,7 @@ __global__ __launch_bounds__(SH ? 256 : 512, 2) void rows32_kernel(RowsArgs a) {
                 }
         }
     }
-    if constexpr (!SH) {
+    {
         // the KW partial tiles, halved per round (as rows16_kernel)
         f32x4* sp = (f32x4*)s_part;
         constexpr int NR = NMAT * R * C * 4;
@@ -993,13 +1038,8 @@ int launch16(const RowsArgs& a, hipStream_t st) {
 
 template <int FMT, int NMAT, int R, int C>
 int launch32(const RowsArgs& a, hipStream_t st) {
-    const dim3 grid(8 * a.mpp * a.npp);
-    if (a.NW == 4) {
-        hipLaunchKernelGGL((rows32_kernel<FMT, NMAT, R, C, true>), grid, dim3(256), 0, st, a);
-    } else {
-        const size_t lds = a.KW > 1 ? (size_t)(a.KW / 2) * a.NW * NMAT * R * C * 4096 : 0;
-        hipLaunchKernelGGL((rows32_kernel<FMT, NMAT, R, C, false>), grid, dim3(64 * a.NW * a.KW), lds, st, a);
-    }
+    const size_t lds = a.KW > 1 ? (size_t)(a.KW / 2) * a.NW * NMAT * R * C * 4096 : 0;
+    hipLaunchKernelGGL((rows32_kernel<FMT, NMAT, R, C>), dim3(8 * a.mpp * a.npp), dim3(64 * a.NW * a.KW), lds, st, a);
     return hipGetLastError() == hipSuccess ? RINA_OK : RINA_ERR_HIP;
 }
 
