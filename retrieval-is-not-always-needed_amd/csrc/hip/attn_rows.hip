@@ -108,40 +108,34 @@ __global__ __launch_bounds__(256 * NSET) void attn_rows_kernel(RowsAttnArgs a, i
     f32x4 o[ND];                                                 // tile dt: dims ND (4 g + e) + dt
 #pragma unroll
     for (int dt = 0; dt < ND; dt++) o[dt] = f32x4{0.f, 0.f, 0.f, 0.f};
-    if constexpr (SRC == ROWS_DQ) {
-        const int pos = pos0 + rowc, dq = a.da + a.db;
-        const float* qa = a.qa + ((int64_t)rowc * a.H + h) * a.da;
-        const float* qb = a.qb + ((int64_t)rowc * a.H + h) * a.db;
-        const float* ka = a.ka + ((int64_t)rowc * a.Hkv + kvh) * a.da;
-        const float* kb = a.kb + ((int64_t)rowc * a.Hkv + kvh) * a.db;
-        float own = 0.f;
-#pragma unroll
-        for (int i = 0; i < DQ / 4; i++) {
-            const int d = DQ / 4 * g + i, dc = d < dq ? d : dq - 1;
-            const float x = dq_dim(qa, qb, a.qc, a.qs, a.da, a.db, pos, dc);
-            const float y = dq_dim(ka, kb, a.kc, a.ks, a.da, a.db, pos, dc);
-            qv[i] = d < dq ? x * qsc : 0.f;
-            own = fmaf(qv[i], y, own);
-            if (i % 4 == 3) __builtin_amdgcn_sched_barrier(0);   // a few loads at a time: all of them would spill
-        }
-        own += __shfl_xor(own, 16);
-        own += __shfl_xor(own, 32);
-        if (set == 0 && blockIdx.z == 0) {
-            const float* vp = a.v + ((int64_t)rowc * a.Hkv + kvh) * DV + ND * 4 * g;
-            m = own;
-            l = 1.f;
-#pragma unroll
-            for (int e = 0; e < 4; e++)
-#pragma unroll
-                for (int dt = 0; dt < ND; dt++) o[dt][e] = gld(vp + ND * e + dt);
-        }
-    } else {
+    {
+        // (RINA-MLA rows are DQ wide here, zero past their own width)
         const f32x4* qp = (const f32x4*)(a.q + ((int64_t)rowc * a.H + h) * DQ + DQ / 4 * g);
 #pragma unroll
         for (int i = 0; i < Q4; i++) {
             const f32x4 v = gld(qp + i);
             qv[4 * i] = v.x * qsc; qv[4 * i + 1] = v.y * qsc; qv[4 * i + 2] = v.z * qsc; qv[4 * i + 3] = v.w * qsc;
         }
+    }
+    if (SRC == ROWS_DQ && set == 0 && blockIdx.z == 0) {
+        // the row's own position: its fp32 key and value
+        const f32x4* kp = (const f32x4*)(a.k + ((int64_t)rowc * a.Hkv + kvh) * DQ + DQ / 4 * g);
+        float own = 0.f;
+#pragma unroll
+        for (int i = 0; i < Q4; i++) {
+            const f32x4 v = gld(kp + i);
+#pragma unroll
+            for (int c = 0; c < 4; c++) own = fmaf(qv[4 * i + c], v[c], own);
+        }
+        own += __shfl_xor(own, 16);
+        own += __shfl_xor(own, 32);
+        const float* vp = a.v + ((int64_t)rowc * a.Hkv + kvh) * DV + ND * 4 * g;
+        m = own;
+        l = 1.f;
+#pragma unroll
+        for (int e = 0; e < 4; e++)
+#pragma unroll
+            for (int dt = 0; dt < ND; dt++) o[dt][e] = gld(vp + ND * e + dt);
     }
     // staging: thread ts of a set moves 4 NK key dims and 4 NV value dims of
     // key j0 + ts / TPK (clamped to the last key: such keys are masked)
@@ -401,6 +395,22 @@ __global__ __launch_bounds__(256 * NSET) void attn_rows_kernel(RowsAttnArgs a, i
         }
 }
 
+// RINA-MLA rows: query [qa | HF-RoPE(qb)] and key [ka | HF-RoPE(kb)] rows, w
+// wide (zeros past da + db), into q [T][H][w] and k [T][Hkv][w]: once per row,
+// not in every workgroup that reads it.  Grid (T, H + Hkv), 64 threads.
+__global__ __launch_bounds__(64) void dq_rotate_kernel(RowsAttnArgs a, float* q, float* k, int w) {
+    const int t = blockIdx.x, y = blockIdx.y, dq = a.da + a.db, pos = a.start_pos + t;
+    const bool isq = y < a.H;
+    const int n = isq ? a.H : a.Hkv, h = isq ? y : y - a.H;
+    const float* xa = (isq ? a.qa : a.ka) + ((int64_t)t * n + h) * a.da;
+    const float* xb = (isq ? a.qb : a.kb) + ((int64_t)t * n + h) * a.db;
+    float* o = (isq ? q : k) + ((int64_t)t * n + h) * w;
+    for (int i = threadIdx.x; i < w; i += 64) {
+        const float v = dq_dim(xa, xb, isq ? a.qc : a.kc, isq ? a.qs : a.ks, a.da, a.db, pos, i < dq ? i : dq - 1);
+        gst(o + i, i < dq ? v : 0.f);
+    }
+}
+
 // one wave per (row, head): the ks_n partials merged and normalized
 template <int DV>
 __global__ __launch_bounds__(256) void rows_combine_kernel(RowsAttnArgs a) {
@@ -433,17 +443,25 @@ int launch(RowsAttnArgs a, hipStream_t st) {
     // the output)
     const int max_pos = a.d_pos ? a.max_seq : a.start_pos + a.T;
     const int nblk = (max_pos + KB - 1) / KB;
-    int ks = rina_num_cus() / (groups * ntile);
+    int ks = (2 * rina_num_cus() + groups * ntile / 2) / (groups * ntile);
     if (ks > nblk / (2 * NSET)) ks = nblk / (2 * NSET);
     if (ks > 16) ks = 16;
     if (ks < 1) ks = 1;
     a.ks_n = ks;
-    if (ks > 1) {
-        const size_t n = (size_t)ks * a.T * a.H;
-        float* p = (float*)rina_scratch(n * (DV + 2) * sizeof(float), st, kScratchOut);
+    const size_t n = ks > 1 ? (size_t)ks * a.T * a.H : 0;
+    const size_t rot = SRC == ROWS_DQ ? (size_t)a.T * (a.H + a.Hkv) * DQ : 0;
+    if (n + rot) {
+        float* p = (float*)rina_scratch((rot + n * (DV + 2)) * sizeof(float), st, kScratchOut);
         if (!p) return RINA_ERR_HIP;
-        a.po = p;
-        a.pm = p + n * DV;
+        if (rot) {
+            float* kr = p + (size_t)a.T * a.H * DQ;
+            hipLaunchKernelGGL(dq_rotate_kernel, dim3(a.T, a.H + a.Hkv), dim3(64), 0, st, a, p, kr, DQ);
+            if (hipGetLastError() != hipSuccess) return RINA_ERR_HIP;
+            a.q = p;
+            a.k = kr;
+        }
+        a.po = p + rot;
+        a.pm = a.po + n * DV;
         a.pl = a.pm + n;
     }
     hipLaunchKernelGGL((attn_rows_kernel<SRC, PK, DQ, DV, KB, NSET>), dim3(groups, ntile, ks), dim3(256 * NSET), 0, st, a, hpw);
