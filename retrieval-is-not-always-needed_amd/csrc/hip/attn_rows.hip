@@ -450,8 +450,9 @@ int launch(RowsAttnArgs a, hipStream_t st) {
     a.ks_n = ks;
     const size_t n = ks > 1 ? (size_t)ks * a.T * a.H : 0;
     const size_t rot = SRC == ROWS_DQ ? (size_t)a.T * (a.H + a.Hkv) * DQ : 0;
+    RinaScratch scratch;
     if (n + rot) {
-        float* p = (float*)rina_scratch((rot + n * (DV + 2)) * sizeof(float), st, kScratchOut);
+        float* p = (float*)scratch.get((rot + n * (DV + 2)) * sizeof(float), st, kScratchOut);
         if (!p) return RINA_ERR_HIP;
         if (rot) {
             float* kr = p + (size_t)a.T * a.H * DQ;

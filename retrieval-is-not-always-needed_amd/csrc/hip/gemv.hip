@@ -1400,9 +1400,10 @@ extern "C" int rina_hip_linear_fused_ex(const rina_linear_seg* segs, int nseg, i
         if ((uintptr_t)segs[s].weight % 4 || (segs[s].weight2 && (uintptr_t)segs[s].weight2 % 4)) return RINA_ERR_ARG;
     }
     hipStream_t st = as_stream(stream);
+    RinaScratch scratch;
     if (M > 1 && rows_gemm_ok(qt, K)) {
         // several rows: split once (with the prologue), then 3 segments per launch
-        void* buf = rina_scratch(rows_split_bytes(qt, M, K), st, kScratchRows);
+        void* buf = scratch.get(rows_split_bytes(qt, M, K), st, kScratchRows);
         if (!buf) return RINA_ERR_HIP;
         RowsX xr;
         int rc = rows_split(qt, input, nullptr, nullptr, M, K, pro, nw, eps, buf, &xr, st);
@@ -1423,7 +1424,7 @@ extern "C" int rina_hip_linear_fused_ex(const rina_linear_seg* segs, int nseg, i
     if (pro != RINA_PRO_NONE && (!fused_pro || (norm_out && !direct))) {
         // normalize first (into norm_out when given, else library scratch):
         // prompt rows, unusual shapes
-        float* tmp = norm_out ? norm_out : (float*)rina_scratch((size_t)M * K * 4, as_stream(stream), kScratchNorm);
+        float* tmp = norm_out ? norm_out : (float*)scratch.get((size_t)M * K * 4, st, kScratchNorm);
         if (!tmp) return RINA_ERR_HIP;
         int rc = pro == RINA_PRO_RMSNORM ? rina_hip_rms_norm(input, tmp, nw, M, K, eps, stream)
                                          : rina_hip_layer_norm(input, tmp, nw, M, K, eps, stream);
@@ -1489,8 +1490,9 @@ extern "C" int rina_hip_linear(const void* weight, int qt, const float* input, f
     const char* oe = ob + (size_t)M * N * 4;
     bool alias = ib < oe && ob < ie;
     float* dst = output;
+    RinaScratch scratch;
     if (alias) {
-        dst = (float*)rina_scratch((size_t)M * N * 4, st, kScratchOut);
+        dst = (float*)scratch.get((size_t)M * N * 4, st, kScratchOut);
         if (!dst) return RINA_ERR_HIP;
     }
     rina_linear_seg seg{weight, nullptr, dst, N};

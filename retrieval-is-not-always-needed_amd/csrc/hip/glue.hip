@@ -250,7 +250,7 @@ struct DevState {
 DevState g_dev[64];
 std::mutex g_mu;
 
-// Library scratch, one buffer per (device, stream): work on different
+// Library scratch, one buffer per (device, stream, use): work on different
 // streams never shares it, and work on one stream is ordered.  A buffer
 // that must grow is replaced by one of at least twice its size; the old
 // one may still be read by queued work, so it is kept (retired) until the
@@ -263,6 +263,9 @@ struct ScratchSlot {
 };
 std::vector<ScratchSlot> g_scratch;
 std::vector<void*> g_retired;
+// by stream handle; streams that share one only wait for each other's launches to be queued
+constexpr int kQueueLocks = 61;
+std::recursive_mutex g_queue[kQueueLocks];
 
 }  // namespace
 
@@ -288,9 +291,12 @@ static void* alloc_scratch(size_t bytes) {
     return p;
 }
 
-void* rina_scratch(size_t bytes, hipStream_t st, int use) {
+void* RinaScratch::get(size_t bytes, hipStream_t st, int use) {
+    static thread_local char per_thread;   // hipStreamPerThread is another stream in every thread
+    if (st == hipStreamPerThread) st = (hipStream_t)&per_thread;
     int dev = 0;
     if (hipGetDevice(&dev) != hipSuccess || dev < 0) return nullptr;
+    if (!lk_.owns_lock()) lk_ = std::unique_lock<std::recursive_mutex>(g_queue[((uintptr_t)st >> 4) % kQueueLocks]);
     std::lock_guard<std::mutex> lk(g_mu);
     for (ScratchSlot& s : g_scratch) {
         if (s.dev != dev || s.st != st || s.use != use) continue;

@@ -1551,7 +1551,8 @@ int moe_grouped(float* h, const float* a2, const int* ids, const float* probs, c
     const size_t b_x = up(std::max(rows_split_bytes(qt, (int)slots, d), slots * d * 4));   // split rows, later Y
     const size_t b_g = up(slots * F * 4), b_gx = up(rows_split_bytes(qt, (int)slots, F));
     const size_t b_p = up((2 + 3 * tmax) * 4), b_s = up(slots * 4), b_o = up(tk * 4);
-    char* p = (char*)rina_scratch(b_x + b_g + b_gx + b_p + b_s + b_o, st, kScratchMoe);
+    RinaScratch scratch;
+    char* p = (char*)scratch.get(b_x + b_g + b_gx + b_p + b_s + b_o, st, kScratchMoe);
     if (!p) return RINA_ERR_HIP;
     void* xb = p;
     float* G = (float*)(p + b_x);

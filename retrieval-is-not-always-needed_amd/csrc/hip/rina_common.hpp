@@ -2,6 +2,7 @@
 #pragma once
 #include <hip/hip_runtime.h>
 #include <stdint.h>
+#include <mutex>
 #include "rina_hip.h"
 
 #define RINA_WAVE 64
@@ -184,10 +185,21 @@ int rina_num_cus();
 // on demand and never shrunk: the output of a call that aliases input and
 // output, the row of a norm that runs before a matvec as its own launch, the
 // split activation rows of a product over several rows, the grouped rows of a
-// MoE block.  The uses of one call nest, so each has a buffer of its own; calls on one stream run in order and
-// share them.
+// MoE block.  The uses of one call nest, so each has a buffer of its own; calls
+// on one stream run in order and share them.
+// A call writes its buffer in one launch and reads it in a later one, so it
+// holds the stream's lock from get() until its last launch is queued (the
+// object's lifetime): the launches of two host threads that call on one stream
+// never interleave.  Recursive, since the uses nest; a call takes the lock of
+// its own stream only.  get() returns NULL when out of memory.
 enum { kScratchOut = 0, kScratchNorm = 1, kScratchRows = 2, kScratchMoe = 3 };
-void* rina_scratch(size_t bytes, hipStream_t stream, int use);
+class RinaScratch {
+public:
+    void* get(size_t bytes, hipStream_t stream, int use);
+
+private:
+    std::unique_lock<std::recursive_mutex> lk_;
+};
 
 __device__ __forceinline__ int read_pos(int start_pos, const int* d_pos) {
     return start_pos + (d_pos ? *d_pos : 0);

@@ -190,3 +190,37 @@ def test_moe_rows_groups(rina, orc, qt, T, E, k, d, F, S):
         assert_close(got[t], ref, what="row %d" % t)
         seen += 1
     assert seen >= T * 3 // 4
+
+
+@pytest.mark.parametrize("qt,M", [(7, 16), (10, 40)])
+def test_rows_product_two_threads_one_stream(rina, orc, qt, M):
+    """Two host threads on one stream, each with rows of its own: the split
+    rows of one call are never another's (the products repeat bit for bit)."""
+    import threading
+
+    import torch
+
+    hip, N, K, st = rina.load_hip(), 64, 256, stream()
+    w, _ = weights(orc, qt, rng(qt), N * K)
+    wd = dev(w)
+    xs = [dev(rng(s).standard_normal((M, K)).astype(np.float32)) for s in (1, 2)]
+    ys = [[empty(M * N) for _ in range(300)] for _ in xs]
+    rcs = [[], []]
+
+    def calls(i, n0, n1):
+        for y in ys[i][n0:n1]:
+            seg = rina.LinearSeg(wd.data_ptr(), None, y.data_ptr(), N)
+            rcs[i].append(hip.rina_hip_linear_fused(C.byref(seg), 1, qt, xs[i].data_ptr(), M, K, 0, 0, None, 0.0, st))
+
+    for i in (0, 1):
+        calls(i, 0, 1)                      # alone: the expected products
+    ts = [threading.Thread(target=calls, args=(i, 1, 300)) for i in (0, 1)]
+    for t in ts:
+        t.start()
+    for t in ts:
+        t.join()
+    torch.cuda.synchronize()
+    for i in (0, 1):
+        assert rcs[i] == [0] * 300
+        assert all(torch.equal(y, ys[i][0]) for y in ys[i])
+    assert not torch.equal(ys[0][0], ys[1][0])
