@@ -989,22 +989,38 @@ __global__ __launch_bounds__(256) void dq_split_kernel(DqArgs a, SplitArgs p) {
 }
 
 // A prompt's T rows (rows at positions start_pos + t) over the fp32 caches
-// (QKV 0) or the q2k_q1v cache (QKV 1).  dq_pack_rows_kernel, grid (T, Hkv),
-// one wave per (row, KV head): the row's key and value as
-// dq_split_kernel<QKV> appends them at its position (the same dims, lanes
-// and, packed, block codec).  attn_rows (ROWS_DQ) then reads, for row t, the
-// positions before it from the cache and its own position from its fp32 rows,
-// as the decode step of that row would.
+// (QKV 0) or the q2k_q1v cache (QKV 1).  dq_pack_rows_kernel, grid
+// (T, Hkv + H), one wave per (row, head): for a KV head the row's key and value
+// as dq_split_kernel<QKV> appends them at its position (the same dims, lanes
+// and, packed, block codec), and for every head the rotated row
+// [xa | HF-RoPE(xb)], w wide (zeros past da + db), into k [T][Hkv][w] or
+// q [T][H][w], so that no workgroup of the attention rotates it again.  One
+// launch for both: a call of a few rows is bound by its dependent launches
+// (two rows 12.7 -> 11.1 us,
+// 1900 rows of the q2k_q1v cache 112 -> 107 us against a launch of its own).  attn_rows (ROWS_DQ) then reads, for row t, the positions before it
+// from the cache and its own position from its fp32 rows, as the decode step
+// of that row would.
 template <int QKV>
-__global__ __launch_bounds__(64) void dq_pack_rows_kernel(DqArgs a) {
+__global__ __launch_bounds__(64) void dq_pack_rows_kernel(DqArgs a, float* q, float* k, int w) {
     const int lane = threadIdx.x, t = blockIdx.x, kvh = blockIdx.y;
-    const int pos = a.start_pos + t, dq = a.da + a.db;
+    const int pos = a.start_pos + t, dq = a.da + a.db;       // 64 <= dq <= w <= 128
     const int i1 = lane + 64 < dq ? lane + 64 : dq - 1;
+    if (kvh >= a.Hkv) {
+        const int64_t r = (int64_t)t * a.H + (kvh - a.Hkv);
+        const float x0 = dq_dim(a.qa + r * a.da, a.qb + r * a.db, a.qc, a.qs, a.da, a.db, pos, lane);
+        const float x1 = dq_dim(a.qa + r * a.da, a.qb + r * a.db, a.qc, a.qs, a.da, a.db, pos, i1);
+        gst(q + r * w + lane, x0);
+        if (lane + 64 < w) gst(q + r * w + lane + 64, lane + 64 < dq ? x1 : 0.f);
+        return;
+    }
     const float* ka = a.ka + ((int64_t)t * a.Hkv + kvh) * a.da;
     const float* kb = a.kb + ((int64_t)t * a.Hkv + kvh) * a.db;
     const float kc0 = dq_dim(ka, kb, a.kc, a.ks, a.da, a.db, pos, lane);
     const float kc1 = dq_dim(ka, kb, a.kc, a.ks, a.da, a.db, pos, i1);
     const float vc = gld(a.v + ((int64_t)t * a.Hkv + kvh) * a.dv + lane);
+    float* kw = k + ((int64_t)t * a.Hkv + kvh) * w;
+    gst(kw + lane, kc0);
+    if (lane + 64 < w) gst(kw + lane + 64, lane + 64 < dq ? kc1 : 0.f);
     const int64_t row = (int64_t)pos * a.Hkv + kvh;
     if (QKV == 0) {
         float* kd = a.ck + row * dq;
@@ -1458,12 +1474,16 @@ extern "C" int rina_hip_dq_prompt_attention_kv(const float* qa, const float* qb,
     a.H = H; a.Hkv = Hkv; a.da = da; a.db = db; a.dv = dv; a.start_pos = start_pos; a.max_seq = max_seq;
     a.scale = 1.0f / sqrtf((float)(da + db));
     hipStream_t st = as_stream(stream);
-    if (packed) hipLaunchKernelGGL(dq_pack_rows_kernel<1>, dim3(T, Hkv), dim3(64), 0, st, a);
-    else hipLaunchKernelGGL(dq_pack_rows_kernel<0>, dim3(T, Hkv), dim3(64), 0, st, a);
+    const int w = dq_rows_width(da + db);
+    RinaScratch scratch;
+    float* qr = (float*)scratch.get((size_t)T * (H + Hkv) * w * sizeof(float), st, kScratchRows);
+    if (!qr) return RINA_ERR_HIP;
+    float* kr = qr + (size_t)T * H * w;
+    if (packed) hipLaunchKernelGGL(dq_pack_rows_kernel<1>, dim3(T, Hkv + H), dim3(64), 0, st, a, qr, kr, w);
+    else hipLaunchKernelGGL(dq_pack_rows_kernel<0>, dim3(T, Hkv + H), dim3(64), 0, st, a, qr, kr, w);
     RINA_LAUNCH_CHECK();
     RowsAttnArgs r{};
-    r.qa = qa; r.qb = qb; r.ka = ka; r.kb = kb; r.v = v;
-    r.qc = rope_q_cos; r.qs = rope_q_sin; r.kc = rope_k_cos; r.ks = rope_k_sin;
+    r.q = qr; r.k = kr; r.v = v;
     r.ck = (const uint8_t*)cache_k; r.cv = (const uint8_t*)cache_v; r.ckr = cache_kr;
     r.out = out; r.mode = kv_mode; r.T = T; r.H = H; r.Hkv = Hkv; r.da = da; r.db = db;
     r.start_pos = start_pos; r.max_seq = max_seq; r.scale = a.scale;

@@ -395,22 +395,6 @@ __global__ __launch_bounds__(256 * NSET) void attn_rows_kernel(RowsAttnArgs a, i
         }
 }
 
-// RINA-MLA rows: query [qa | HF-RoPE(qb)] and key [ka | HF-RoPE(kb)] rows, w
-// wide (zeros past da + db), into q [T][H][w] and k [T][Hkv][w]: once per row,
-// not in every workgroup that reads it.  Grid (T, H + Hkv), 64 threads.
-__global__ __launch_bounds__(64) void dq_rotate_kernel(RowsAttnArgs a, float* q, float* k, int w) {
-    const int t = blockIdx.x, y = blockIdx.y, dq = a.da + a.db, pos = a.start_pos + t;
-    const bool isq = y < a.H;
-    const int n = isq ? a.H : a.Hkv, h = isq ? y : y - a.H;
-    const float* xa = (isq ? a.qa : a.ka) + ((int64_t)t * n + h) * a.da;
-    const float* xb = (isq ? a.qb : a.kb) + ((int64_t)t * n + h) * a.db;
-    float* o = (isq ? q : k) + ((int64_t)t * n + h) * w;
-    for (int i = threadIdx.x; i < w; i += 64) {
-        const float v = dq_dim(xa, xb, isq ? a.qc : a.kc, isq ? a.qs : a.ks, a.da, a.db, pos, i < dq ? i : dq - 1);
-        gst(o + i, i < dq ? v : 0.f);
-    }
-}
-
 // one wave per (row, head): the ks_n partials merged and normalized
 template <int DV>
 __global__ __launch_bounds__(256) void rows_combine_kernel(RowsAttnArgs a) {
@@ -449,19 +433,11 @@ int launch(RowsAttnArgs a, hipStream_t st) {
     if (ks < 1) ks = 1;
     a.ks_n = ks;
     const size_t n = ks > 1 ? (size_t)ks * a.T * a.H : 0;
-    const size_t rot = SRC == ROWS_DQ ? (size_t)a.T * (a.H + a.Hkv) * DQ : 0;
     RinaScratch scratch;
-    if (n + rot) {
-        float* p = (float*)scratch.get((rot + n * (DV + 2)) * sizeof(float), st, kScratchOut);
+    if (n) {
+        float* p = (float*)scratch.get(n * (DV + 2) * sizeof(float), st, kScratchOut);
         if (!p) return RINA_ERR_HIP;
-        if (rot) {
-            float* kr = p + (size_t)a.T * a.H * DQ;
-            hipLaunchKernelGGL(dq_rotate_kernel, dim3(a.T, a.H + a.Hkv), dim3(64), 0, st, a, p, kr, DQ);
-            if (hipGetLastError() != hipSuccess) return RINA_ERR_HIP;
-            a.q = p;
-            a.k = kr;
-        }
-        a.po = p + rot;
+        a.po = p;
         a.pm = a.po + n * DV;
         a.pl = a.pm + n;
     }
@@ -476,9 +452,10 @@ int launch(RowsAttnArgs a, hipStream_t st) {
 
 template <bool PK>
 int launch_dq(const RowsAttnArgs& a, int dq, hipStream_t st) {
-    if (dq <= 64) return launch<ROWS_DQ, PK, 64, 64, 64, 2>(a, st);
-    if (dq <= 80) return launch<ROWS_DQ, PK, 80, 64, 64, 2>(a, st);
-    if (dq <= 96) return launch<ROWS_DQ, PK, 96, 64, 64, 2>(a, st);
+    const int w = dq_rows_width(dq);
+    if (w == 64) return launch<ROWS_DQ, PK, 64, 64, 64, 2>(a, st);
+    if (w == 80) return launch<ROWS_DQ, PK, 80, 64, 64, 2>(a, st);
+    if (w == 96) return launch<ROWS_DQ, PK, 96, 64, 64, 2>(a, st);
     return launch<ROWS_DQ, PK, 128, 64, 64, 2>(a, st);
 }
 

@@ -10,12 +10,10 @@ enum RowsSrc {
 };
 
 struct RowsAttnArgs {
-    const float *q, *k, *v;             // GQA / MLA: rows [T, H, dq]; current K, V rows (MLA: K_nope, V)
+    const float *q, *k, *v;             // rows [T, H, dq] (DQ: dq_rows_width wide); current K, V rows (MLA: K_nope, V)
     const uint8_t *ck, *cv;             // caches (DQ q2k_q1v: key content, values); MLA: the latent records (ck)
     const float* ckr;                   // DQ q2k_q1v: key RoPE part
     const float *rkc, *rks;             // GQA pre-RoPE caches: tables that rotate cached keys
-    const float *qa, *qb, *ka, *kb;     // DQ rows
-    const float *qc, *qs, *kc, *ks;     // DQ: HF RoPE tables
     float* out;                         // [T, H, dv]
     int mode, pre_rope, T, H, Hkv, start_pos, max_seq;
     int da, db;                         // DQ: key content / RoPE widths; MLA: record offset of k_pe, record width
@@ -25,6 +23,9 @@ struct RowsAttnArgs {
     int kf, vf, ks_n, vec;
     float *pm, *pl, *po;                // partials of the ks_n key splits
 };
+
+// width of the DQ rows (zeros past da + db)
+static inline int dq_rows_width(int dq) { return dq <= 64 ? 64 : dq <= 80 ? 80 : dq <= 96 ? 96 : 128; }
 
 // Launches the attention (RINA_ERR_SHAPE, before any launch: a shape or
 // alignment it does not take).  dq, dv: ROWS_GQA 64, 64; ROWS_DQ da + db <= 128, 64;
