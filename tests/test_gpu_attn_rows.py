@@ -34,7 +34,7 @@ def test_rows_device_position(rina, orc, mode, P, T):
     assert_close_elem(got, ref, what="device position mode %d P %d T %d" % (mode, P, T))
 
 
-@pytest.mark.parametrize("T,start,H,Hkv,da,db,mode", [(17, 400, 3, 3, 80, 34, 0), (5, 700, 6, 2, 64, 10, 5),
+@pytest.mark.parametrize("T,start,H,Hkv,da,db,mode", [(63, 1, 10, 5, 64, 32, 0), (2, 63, 10, 5, 64, 16, 5), (17, 400, 3, 3, 80, 34, 0), (5, 700, 6, 2, 64, 10, 5),
                                                       (65, 63, 10, 5, 64, 64, 5), (33, 1, 8, 2, 48, 22, 0)])
 def test_dq_rows_other_widths(rina, T, start, H, Hkv, da, db, mode):
     dq_rows_case(rina, T, start, H, Hkv, da, db, mode)
