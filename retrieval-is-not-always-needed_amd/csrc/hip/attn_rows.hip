@@ -16,6 +16,10 @@
 // one query row (l % 16), the row maximum and sum take two cross-lane steps,
 // and those scores are directly the B operand of O^T += V^T P^T (dim
 // ND (l % 16) + dt of tile dt).  Scores carry log2 e: weights are exp2 values.
+// A row's result holds no value past its position, also where that value is
+// inf or NaN (a weight of zero times it would not be zero): a block that ends
+// past a wave's first row and holds such values is added key by key, over the
+// keys that each row sees.
 // Where the row tiles leave the chip idle (few rows over a long cache), the
 // key range is split over ks_n workgroups whose (m, l, O) partials
 // rows_combine_kernel merges.
@@ -74,6 +78,15 @@ __device__ __forceinline__ void half_values(int fmt, const Half& r, float (&v)[1
     }
 }
 
+// 0, or NaN if one of the values is inf or NaN
+template <int N>
+__device__ __forceinline__ float zero_or_nan(const float (&v)[N]) {
+    float t = 0.f;
+#pragma unroll
+    for (int i = 0; i < N; i++) t = fmaf(v[i], 0.f, t);
+    return t;
+}
+
 // DQ: query / key width held (a multiple of 16; dims past a.da + a.db are
 // zero), DV: value width, KB: keys per block.  PK: the cache is packed.
 // NSET sets of 4 waves.
@@ -83,6 +96,7 @@ __global__ __launch_bounds__(256 * NSET) void attn_rows_kernel(RowsAttnArgs a, i
     constexpr int TPK = 256 / KB, NK = DQ / TPK / 4, NV = DV / TPK / 4;   // threads per key, float4 each
     __shared__ __align__(16) float s_k[NSET][KB][LDK];
     __shared__ __align__(16) float s_v[NSET][KB][LDV];
+    __shared__ int s_bad[NSET];                                  // 1 + the last block whose values are not all finite
     const int tid = threadIdx.x, lane = tid & 63;
     const int set = __builtin_amdgcn_readfirstlane(tid >> 8);
     const int ts = tid & 255;
@@ -209,7 +223,8 @@ __global__ __launch_bounds__(256 * NSET) void attn_rows_kernel(RowsAttnArgs a, i
             for (int i = 0; i < NV; i++) vr[i] = gld(vp + i);
         }
     };
-    auto store_blk = [&]() {
+    // (check: returns NaN if one of the thread's values is not finite)
+    auto store_blk = [&](bool check) -> float {
         float* kd = s_k[set][sk];
         float* vd = s_v[set][sk];
         if (SRC == ROWS_GQA && jl < pos0) {
@@ -238,6 +253,7 @@ __global__ __launch_bounds__(256 * NSET) void attn_rows_kernel(RowsAttnArgs a, i
                 *(f32x4*)&kd[16 * sq + 4 * i] = f32x4{kv[4 * i], kv[4 * i + 1], kv[4 * i + 2], kv[4 * i + 3]};
                 *(f32x4*)&vd[16 * sq + 4 * i] = f32x4{vv[4 * i], vv[4 * i + 1], vv[4 * i + 2], vv[4 * i + 3]};
             }
+            return check ? zero_or_nan(vv) : 0.f;
         } else if (SRC == ROWS_DQ && PK) {
             float kv[16], vv[16];
             half_values(RINA_KVF_Q2_1, kh, kv);
@@ -250,19 +266,28 @@ __global__ __launch_bounds__(256 * NSET) void attn_rows_kernel(RowsAttnArgs a, i
             }
 #pragma unroll
             for (int i = 0; i < NR / 4; i++) *(f32x4*)&kd[64 + NR * sq + 4 * i] = kr[i];
+            return check ? zero_or_nan(vv) : 0.f;
         } else {
 #pragma unroll
             for (int i = 0; i < NK; i++) *(f32x4*)&kd[4 * NK * sq + 4 * i] = kr[i];
 #pragma unroll
             for (int i = 0; i < NV; i++) *(f32x4*)&vd[4 * NV * sq + 4 * i] = vr[i];
+            float vv[4 * NV];
+#pragma unroll
+            for (int i = 0; i < 4 * NV; i++) vv[i] = vr[i / 4][i % 4];
+            return check ? zero_or_nan(vv) : 0.f;
         }
     };
+    // the first keys that the workgroup's and this wave's first row do not see
+    constexpr int OWN = SRC == ROWS_DQ ? 0 : 1;
+    const int lim_wg = pos0 + t0 + OWN, lim_wave = lim_wg + 16 * (w / hpw);
+    if (ts == 0) s_bad[set] = 0;
     const int nit = b1 > b0 ? (b1 - b0 + NSET - 1) / NSET : 0;
     if (nit > 0) load_blk(min(b0 + set, b1 - 1));
     for (int it = 0; it < nit; it++) {
         const int blk = b0 + NSET * it + set;                    // past b1: nothing (same for the set)
         __syncthreads();                                         // the previous block's operands are read
-        store_blk();
+        if (store_blk((blk + 1) * KB > lim_wg && blk < b1) != 0.f) s_bad[set] = blk + 1;
         __syncthreads();
         load_blk(min(blk + NSET, b1 - 1));                       // unconditional: clamped past the end
         if (blk >= b1) continue;
@@ -321,6 +346,22 @@ __global__ __launch_bounds__(256 * NSET) void attn_rows_kernel(RowsAttnArgs a, i
         f32x4 ob[ND];
 #pragma unroll
         for (int dt = 0; dt < ND; dt++) ob[dt] = f32x4{0.f, 0.f, 0.f, 0.f};
+        if (j0 + KB > lim_wave && s_bad[set] == blk + 1) {
+            // lane group k4 holds the weights of keys 16 kt + 4 k4 + e
+#pragma unroll
+            for (int kt = 0; kt < KT; kt++)
+#pragma unroll
+                for (int e = 0; e < 4; e++)
+#pragma unroll 1
+                    for (int k4 = 0; k4 < 4; k4++) {
+                        const int key = 16 * kt + 4 * k4 + e;
+                        const float p = __shfl(s[kt][e], fr + 16 * k4);
+                        if (j0 + key >= lim) continue;
+#pragma unroll
+                        for (int i = 0; i < 4 * ND; i++)
+                            ob[i % ND][i / ND] = fmaf(p, s_v[set][key][4 * ND * g + i], ob[i % ND][i / ND]);
+                    }
+        } else
 #pragma unroll
         for (int kt = 0; kt < KT; kt++)
 #pragma unroll
