@@ -296,7 +296,8 @@ int rina_hip_mla_prompt_attention(const float* q, const float* kva, const float*
 
 /* Router top-k of deepseek_mla_layer.cu:310-326 on the device: softmax of
  * the E logits, insertion top-k kept ascending (strict ">", the earlier
- * expert wins ties).  ids/probs [k] in that order.  E <= 256, k <= 16. */
+ * expert wins ties).  ids/probs [k] in that order; ids -1 where the softmax is
+ * NaN (a logit of NaN or +inf).  E <= 256, k <= 16. */
 int rina_hip_moe_topk(const float* logits, int n_experts, int k, int* ids,
                       float* probs, void* stream);
 

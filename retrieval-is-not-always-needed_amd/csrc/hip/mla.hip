@@ -1096,7 +1096,9 @@ __global__ __launch_bounds__(256) void mla_expand_kernel(MlaArgs a, const float*
 // insertion loop.  That loop keeps the k largest probabilities with strict
 // ">" (of equal values the earlier expert stays) in ascending order, equal
 // values ending up later-expert first.  Here every expert computes its rank
-// against the others in parallel, which gives the same set and order.
+// against the others in parallel, which gives the same set and order.  Logits
+// that hold NaN or +inf give NaN probabilities, of which the loop selects none:
+// ids -1, probs -1e10 (the loop's initial values).
 // grid = rows: workgroup r selects from logits row r into ids / probs row r
 __global__ __launch_bounds__(256) void moe_topk_kernel(const float* lg, int E, int k, int* ids, float* probs) {
     __shared__ float s_p[256];
@@ -1121,6 +1123,13 @@ __global__ __launch_bounds__(256) void moe_topk_kernel(const float* lg, int E, i
     }
     __syncthreads();
     const float p = ex * s_inv;
+    if (!(s_inv == s_inv)) {
+        if (tid < k) {
+            gst(ids + tid, -1);
+            gst(probs + tid, -1e10f);
+        }
+        return;
+    }
     __syncthreads();
     s_p[tid] = p;
     __syncthreads();
@@ -1148,7 +1157,7 @@ __global__ __launch_bounds__(1024) void moe_plan_kernel(const int* ids, int tk, 
     const int tid = threadIdx.x;
     if (tid < 256) s_cnt[tid] = 0;
     __syncthreads();
-    // ids outside the experts (a router row of NaN selects none) take no slot
+    // ids outside the experts (a row that selects none) take no slot
     for (int i = tid; i < tk; i += 1024) {
         const int e = gld(ids + i);
         if (e >= 0 && e < E) atomicAdd(&s_cnt[e], 1);

@@ -195,6 +195,44 @@ def test_moe_topk_matches_oracle(rina, orc):
     assert checked >= 30
 
 
+@pytest.mark.parametrize("bad", [float("nan"), float("inf")])
+def test_moe_topk_of_a_non_finite_row(rina, orc, bad):
+    """Logits that hold NaN (or +inf: inf - inf) give NaN probabilities: no
+    expert is selected, as in the oracle, whatever the buffers held."""
+    hip = rina.load_hip()
+    lg = rng(5).standard_normal(64).astype(np.float32)
+    lg[9] = bad
+    ids, pr = dev(np.arange(6, dtype=np.int32)), dev(np.full(6, 0.5, np.float32))
+    ok(hip.rina_hip_moe_topk(dev(lg).data_ptr(), 64, 6, ids.data_ptr(), pr.data_ptr(), stream()), "topk")
+    ids_o, _ = orc.moe_topk(lg, 6)
+    assert host(ids).tolist() == ids_o.tolist() == [-1] * 6
+
+
+def test_moe_rows_of_a_non_finite_router(rina, orc):
+    """Router logits of NaN over finite rows (a router weight of NaN): no row
+    selects an expert, so the rows get the shared experts alone, whatever
+    selection the workspace held before."""
+    hip, T, d, F, E, k = rina.load_hip(), 20, 128, 64, 4, 2
+    r = rng(8)
+    w = [dev(orc.pack(7, (r.standard_normal(E * F * d) * 0.05).astype(np.float32))) for _ in range(3)]
+    wr = (r.standard_normal((E, d)) * 0.2).astype(np.float32)
+    h0 = r.standard_normal((T, d)).astype(np.float32)
+    ln2 = dev(np.ones(d, np.float32))
+    wb = hip.rina_hip_moe_rows_workspace(T, d, E, k, F, 0)
+    ws = empty(wb // 4 + 4)
+
+    def call(router):
+        h = dev(h0)
+        ok(hip.rina_hip_moe_rows(h.data_ptr(), T, ln2.data_ptr(), np.float32(1e-5), dev(router).data_ptr(), FP32, None, None,
+                                 None, 0, 7, w[0].data_ptr(), w[1].data_ptr(), w[2].data_ptr(), 7, F * d // 32 * 20,
+                                 F * d // 32 * 20, E, k, d, F, ws.data_ptr(), wb, stream()), "moe rows")
+        return host(h).reshape(T, d)
+
+    assert not np.array_equal(call(wr), h0)
+    wr[2, 5] = np.nan
+    assert np.array_equal(call(wr), h0)
+
+
 def packed_only(orc, qt, rows, cols, r):
     if qt == Q2K:
         return mt.q2k_random(r, rows * cols)

@@ -88,25 +88,73 @@ def test_rows_product_magnitudes(rina, orc, qt):
 
 
 @pytest.mark.parametrize("qt", [5, 7, 10])
-def test_rows_product_nonfinite(rina, orc, qt):
-    """inf and NaN stay in their rows: Q4 rows give fp32's results (inf where
-    the weight is not zero, NaN where it is), Q2_K rows are not finite."""
+@pytest.mark.parametrize("M", [5, 24, 70])
+def test_rows_product_outlier_facing_zero_weights(rina, orc, qt, M):
+    """A value 2^12 .. 2^60 times the others whose weights are zero adds
+    nothing: the product of the others is as close as without it.  fp32 sums of
+    480 terms in chains of at most 16 blocks: below 1e-6 of sum |w x|."""
+    r = rng(qt + M)
+    N, K, at = 48, 480, 37
+    w, _ = weights(orc, qt, r, N * K)
+    if qt == 10:                             # scale and minimum of the group of 16 that holds it
+        g = (np.arange(N) * K + at) // 16
+        w = w.reshape(-1, 84).copy()
+        w[g // 16, g % 16] = 0
+        w = w.reshape(-1)
+    else:
+        wf = (r.standard_normal((N, K)) * 0.02).astype(np.float32)
+        wf[:, at] = 0
+        w = orc.pack(qt, wf.reshape(-1))
+    W = orc.dequant(qt, w, N * K).astype(np.float64).reshape(N, K)
+    assert not W[:, at].any()
+    x = r.standard_normal((M, K)).astype(np.float32)
+    x[:, at] = (2.0 ** np.linspace(12, 60, M)).astype(np.float32)
+    got = product(rina, w, qt, x, N, K).astype(np.float64)
+    x[:, at] = 0
+    ref, scale = x.astype(np.float64) @ W.T, np.abs(x.astype(np.float64)) @ np.abs(W.T)
+    assert np.all(np.abs(got - ref) <= 1e-6 * scale)
+
+
+@pytest.mark.parametrize("qt", [5, 7, 10])
+@pytest.mark.parametrize("M,K", [(20, 256), (20, 416), (70, 256), (70, 416)])
+def test_rows_product_nonfinite(rina, orc, qt, M, K):
+    """inf and NaN stay in their rows, and rows that hold them give what the
+    fp32 products give: an infinity of the weight's sign, NaN where the weight
+    is zero, the row holds NaN or infinities of both signs meet."""
     r = rng(qt + 50)
-    M, N, K = 20, 32, 256
+    N = 100
     w, W = weights(orc, qt, r, N * K)
     x = r.standard_normal((M, K)).astype(np.float32)
-    x[3, 77], x[7, 5], x[18, 200] = np.inf, np.nan, -np.inf
+    x[3, 77], x[7, 5], x[18, 200], x[11, 64], x[11, 65] = np.inf, np.nan, -np.inf, np.inf, -np.inf
     got = product(rina, w, qt, x, N, K)
     W = W.reshape(N, K)
     with np.errstate(invalid="ignore"):
         ref = np.stack([(W * xr).sum(1) for xr in x.astype(np.float64)])
-    fine = [m for m in range(M) if m not in (3, 7, 18)]
+    bad = [3, 7, 11, 18]
+    fine = [m for m in range(M) if m not in bad]
     assert_close(got[fine], ref[fine], what="finite rows")
-    assert not np.isfinite(got[[3, 7, 18]]).any()
-    if qt != 10:
-        assert np.array_equal(np.isnan(got[[3, 18]]), np.isnan(ref[[3, 18]]))
-        m = ~np.isnan(ref[[3, 18]])
-        assert np.array_equal(got[[3, 18]][m], ref[[3, 18]][m].astype(np.float32))
+    assert not np.isfinite(ref[bad]).any()
+    assert np.array_equal(got[bad], ref[bad].astype(np.float32), equal_nan=True)
+
+
+@pytest.mark.parametrize("qt", [10])
+@pytest.mark.parametrize("M,epi", [(12, 1), (40, 1), (12, 2), (40, 2)])
+def test_rows_product_nonfinite_epilogues(rina, orc, qt, M, epi):
+    """The same through the residual add (the infinity stays) and SiLU * up."""
+    r = rng(qt + M + epi)
+    N, K = 40, 288
+    w, W = weights(orc, qt, r, N * K)
+    w2, W2 = weights(orc, qt, r, N * K)
+    x = r.standard_normal((M, K)).astype(np.float32)
+    x[4, 99] = np.inf
+    y0 = r.standard_normal((M, N)).astype(np.float32)
+    got = product(rina, w, qt, x, N, K, epi=epi, w2=w2 if epi == 2 else None, y0=y0 if epi == 1 else None)
+    with np.errstate(invalid="ignore", over="ignore"):
+        g, u = ((m.reshape(N, K)[None] * x.astype(np.float64)[:, None]).sum(2) for m in (W, W2))
+        ref = y0 + g if epi == 1 else g / (1 + np.exp(-g)) * u
+    fine = np.arange(M) != 4
+    assert_close(got[fine], ref[fine], what="finite rows")
+    assert np.array_equal(got[4], ref[4].astype(np.float32), equal_nan=True)
 
 
 def test_rows_product_under_capture(rina, orc):
