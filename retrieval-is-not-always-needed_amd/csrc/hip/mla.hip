@@ -1604,6 +1604,10 @@ extern "C" int rina_hip_moe_rows(float* h, int T, const float* ln2, float eps, c
     if (!h || !ln2 || !gate_inp || !gate_exps || !up_exps || !down_exps || T < 1 || E < 1 || E > 256 || k < 1 ||
         k > 16 || k > E || d < 1 || F < 1 || S < 0 || (S > 0 && (!gate_sh || !up_sh || !down_sh)))
         return RINA_ERR_ARG;
+    // weights at 4-byte alignment, as every product takes them
+    if (((uintptr_t)gate_exps | (uintptr_t)up_exps | (uintptr_t)down_exps) % 4 ||
+        (E > 1 && (stride_gu % 4 || stride_dn % 4)))
+        return RINA_ERR_ARG;
     const size_t need = rina_hip_moe_rows_workspace(T, d, E, k, F, S);
     if (!workspace || ws_bytes < need || (uintptr_t)workspace % 16) return RINA_ERR_WORKSPACE;
     hipStream_t st = as_stream(stream);

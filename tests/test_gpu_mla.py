@@ -233,6 +233,29 @@ def test_moe_rows_of_a_non_finite_router(rina, orc):
     assert np.array_equal(call(wr), h0)
 
 
+@pytest.mark.parametrize("qt", [Q2K, Q40, Q4F, FP32])
+def test_moe_rows_rejects_unaligned_experts(rina, qt):
+    """Expert weights or strides off the 4-byte alignment: RINA_ERR_ARG before
+    any launch (nothing is written), whichever way the experts are grouped."""
+    hip, T, d, F, E, k = rina.load_hip(), 4, 64, 32, 4, 2
+    buf = empty(1 << 16)
+    p = buf.data_ptr()
+    wb = hip.rina_hip_moe_rows_workspace(T, d, E, k, F, 0)
+    assert wb <= 1 << 18
+
+    def call(g, u, dn, sgu, sdn):
+        return hip.rina_hip_moe_rows(p, T, p, np.float32(1e-5), p, FP32, None, None, None, 0, qt, g, u, dn, qt, sgu, sdn, E, k,
+                                     d, F, p, wb, stream())
+
+    for off in (1, 2, 3):
+        assert call(p + off, p, p, 8192, 8192) == -1
+        assert call(p, p + off, p, 8192, 8192) == -1
+        assert call(p, p, p + off, 8192, 8192) == -1
+        assert call(p, p, p, 8192 + off, 8192) == -1
+        assert call(p, p, p, 8192, 8192 + off) == -1
+    assert not host(buf).any()
+
+
 def packed_only(orc, qt, rows, cols, r):
     if qt == Q2K:
         return mt.q2k_random(r, rows * cols)
