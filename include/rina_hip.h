@@ -2,8 +2,19 @@
  * rina_hip.h — C-ABI of the MI355X (gfx950) decode hot path of the RINA
  * engine (rina-engine).  Plain pointers and sizes; every pointer argument
  * is device memory unless stated; `stream` is a hipStream_t (NULL = the
- * null stream).  Every entry point is stream-ordered, never synchronizes,
- * and returns RINA_OK (0) or a negative status.
+ * null stream).  Every entry point is stream-ordered, never synchronizes
+ * (exceptions are stated), and returns RINA_OK (0) or a negative status.
+ *
+ * Library scratch.  Calls over several rows (products of M > 1 rows, attention
+ * of T > 1 rows, the MoE block over rows) and aliased or separately normalized
+ * matvecs keep intermediate rows in device memory that the library owns: one
+ * buffer per stream and use, allocated on the first call that needs it and on
+ * growth (RINA_ERR_HIP when that fails), kept for later calls on that stream.
+ * Under stream capture the buffers belong to the graph instead: they are
+ * allocated during the capture and go back when the graph and its executables
+ * are destroyed, so graphs may be replayed on any stream, beside other graphs
+ * and other calls.  Two executables of one captured graph share them (as they
+ * share the caller's own buffers) and must not run at the same time.
  *
  * Each declaration names the reference interface it replaces
  * (paths relative to the reference repository root).
@@ -467,7 +478,7 @@ int rina_hip_dq_decode_attention_kv(const float* qa, const float* qb, const floa
  * v [T, Hkv*dv]; out [T, H*dv].  dv == 64, 64 <= da + db <= 128, db even;
  * q2k_q1v: da == 64, caches 2-byte aligned; fp32: caches 4-byte aligned
  * (else RINA_ERR_SHAPE); start_pos + T <= max_seq (else RINA_ERR_RANGE).
- * No workspace. */
+ * No workspace argument (library scratch past 64 positions). */
 int rina_hip_dq_prompt_attention_kv(const float* qa, const float* qb, const float* ka,
                                     const float* kb, const float* v, const float* rope_q_cos,
                                     const float* rope_q_sin, const float* rope_k_cos,

@@ -2,6 +2,8 @@
 // SiLU*up, add, saxpy, greedy argmax) and the library's runtime helpers.
 #include "rina_common.hpp"
 #include "kv_formats.hpp"
+#include <algorithm>
+#include <atomic>
 #include <mutex>
 #include <vector>
 
@@ -250,22 +252,59 @@ struct DevState {
 DevState g_dev[64];
 std::mutex g_mu;
 
-// Library scratch, one buffer per (device, stream, use): work on different
-// streams never shares it, and work on one stream is ordered.  A buffer
-// that must grow is replaced by one of at least twice its size; the old
-// one may still be read by queued work, so it is kept (retired) until the
-// process ends: at most log2 of the largest request buffers per stream.
+// Library scratch: a buffer per (device, stream, use), and within a stream
+// capture a buffer of that capture: a graph may be replayed on any stream, also
+// beside work on the stream it was captured on.  A buffer that must grow is
+// replaced by one of at least twice its size; the old one may still be read by
+// queued work, so it stays (a stream's: at most log2 of its largest request
+// such buffers).  A capture's buffers go back when its graph and every
+// executable of it are gone (a user object of the graph says so), a thread's
+// (hipStreamPerThread) when the thread ends.
 struct ScratchSlot {
     int dev, use;
-    hipStream_t st;
+    uintptr_t st;                  // stream handle, or the thread's id
+    unsigned long long cap;        // capture id, 0: not captured
     void* p;
     size_t bytes;
+    bool old;                      // replaced by a larger one
 };
-std::vector<ScratchSlot> g_scratch;
-std::vector<void*> g_retired;
-// by stream handle; streams that share one only wait for each other's launches to be queued
+// by stream; streams that share one only wait for each other's launches to be queued
 constexpr int kQueueLocks = 61;
-std::recursive_mutex g_queue[kQueueLocks];
+// (never destroyed: threads and graphs may end after the process's statics)
+struct ScratchState {
+    std::mutex mu;
+    std::vector<ScratchSlot> slots;
+    std::recursive_mutex queue[kQueueLocks];
+    std::atomic<bool> done{false};         // one of the lists below is not empty
+    std::mutex done_mu;                    // held around nothing but them
+    std::vector<void*> done_bufs;          // buffers of graphs that are gone
+    std::vector<uintptr_t> done_threads;   // ids of threads that ended
+};
+ScratchState& scratch_state() {
+    static ScratchState* s = new ScratchState;
+    return *s;
+}
+
+// hipStreamPerThread is another stream in every thread.  Ids are odd (handles
+// are not) and never used again: a new thread does not take the buffer of one
+// whose work may still be queued.
+struct ThreadId {
+    uintptr_t id;
+    ThreadId() {
+        static std::atomic<uintptr_t> next{1};
+        id = 2 * next.fetch_add(1) + 1;
+    }
+    ~ThreadId() {
+        ScratchState& g = scratch_state();
+        std::lock_guard<std::mutex> lk(g.done_mu);
+        g.done_threads.push_back(id);
+        g.done = true;
+    }
+};
+uintptr_t thread_id() {
+    static thread_local ThreadId t;
+    return t.id;
+}
 
 }  // namespace
 
@@ -280,38 +319,109 @@ int rina_num_cus() {
     return g_dev[dev].cus;
 }
 
-// hipMalloc that a stream capture of the calling thread does not forbid (the
-// buffer outlives the graph: it is never freed)
-static void* alloc_scratch(size_t bytes) {
+// allocations that a stream capture of the calling thread does not forbid
+struct RelaxedCapture {
     hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
-    const bool swapped = hipThreadExchangeStreamCaptureMode(&mode) == hipSuccess;
+    bool swapped;
+    RelaxedCapture() : swapped(hipThreadExchangeStreamCaptureMode(&mode) == hipSuccess) {}
+    ~RelaxedCapture() {
+        if (swapped) (void)hipThreadExchangeStreamCaptureMode(&mode);
+    }
+};
+
+static void* alloc_scratch(size_t bytes) {
+    RelaxedCapture rc;
     void* p = nullptr;
-    if (hipMalloc(&p, bytes) != hipSuccess) p = nullptr;
-    if (swapped) (void)hipThreadExchangeStreamCaptureMode(&mode);
-    return p;
+    return hipMalloc(&p, bytes) == hipSuccess ? p : nullptr;
+}
+
+// a graph is gone (called by the runtime: no HIP call, no lock that is held around one)
+static void scratch_graph_done(void* p) {
+    ScratchState& g = scratch_state();
+    std::lock_guard<std::mutex> lk(g.done_mu);
+    g.done_bufs.push_back(p);
+    g.done = true;
+}
+
+// frees what ended graphs and threads left (hipFree waits for work that still reads it)
+static void scratch_reap(ScratchState& g) {
+    if (!g.done) return;
+    std::vector<void*> gone;
+    {
+        std::vector<uintptr_t> threads;
+        std::lock_guard<std::mutex> lk(g.mu);
+        {
+            std::lock_guard<std::mutex> dk(g.done_mu);
+            gone.swap(g.done_bufs);
+            threads.swap(g.done_threads);
+            g.done = false;
+        }
+        auto is_gone = [&](const ScratchSlot& s) {
+            if (std::find(gone.begin(), gone.end(), s.p) != gone.end()) return true;
+            if (s.cap || std::find(threads.begin(), threads.end(), s.st) == threads.end()) return false;
+            gone.push_back(s.p);
+            return true;
+        };
+        for (size_t i = 0; i < g.slots.size();) {
+            if (is_gone(g.slots[i])) {
+                g.slots[i] = g.slots.back();
+                g.slots.pop_back();
+            } else {
+                i++;
+            }
+        }
+    }
+    RelaxedCapture rc;
+    for (void* p : gone) (void)hipFree(p);
 }
 
 void* RinaScratch::get(size_t bytes, hipStream_t st, int use) {
-    static thread_local char per_thread;   // hipStreamPerThread is another stream in every thread
-    if (st == hipStreamPerThread) st = (hipStream_t)&per_thread;
+    ScratchState& g = scratch_state();
+    if (st == hipStreamLegacy) st = nullptr;       // the null stream
+    const uintptr_t key = st == hipStreamPerThread ? thread_id() : (uintptr_t)st;
     int dev = 0;
     if (hipGetDevice(&dev) != hipSuccess || dev < 0) return nullptr;
-    if (!lk_.owns_lock()) lk_ = std::unique_lock<std::recursive_mutex>(g_queue[((uintptr_t)st >> 4) % kQueueLocks]);
-    std::lock_guard<std::mutex> lk(g_mu);
-    for (ScratchSlot& s : g_scratch) {
-        if (s.dev != dev || s.st != st || s.use != use) continue;
-        if (s.bytes >= bytes) return s.p;
-        size_t nb = bytes > 2 * s.bytes ? bytes : 2 * s.bytes;
-        void* p = alloc_scratch(nb);
-        if (!p) return nullptr;
-        g_retired.push_back(s.p);
-        s.p = p;
-        s.bytes = nb;
-        return p;
+    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+    unsigned long long cap = 0;
+    hipGraph_t graph = nullptr;
+    // (the null stream is never captured, and may not be asked while another stream is)
+    if (st && hipStreamGetCaptureInfo_v2(st, &cs, &cap, &graph, nullptr, nullptr) != hipSuccess) return nullptr;
+    if (cs != hipStreamCaptureStatusActive) {
+        cap = 0;
+        scratch_reap(g);
     }
-    void* p = alloc_scratch(bytes);
+    if (!lk_.owns_lock()) lk_ = std::unique_lock<std::recursive_mutex>(g.queue[key % kQueueLocks]);
+    auto find = [&]() -> ScratchSlot* {
+        for (ScratchSlot& s : g.slots)
+            if (s.dev == dev && s.st == key && s.use == use && s.cap == cap && !s.old) return &s;
+        return nullptr;
+    };
+    {
+        std::lock_guard<std::mutex> lk(g.mu);
+        if (ScratchSlot* s = find()) {
+            if (s->bytes >= bytes) return s->p;
+            bytes = std::max(bytes, 2 * s->bytes);
+        }
+    }
+    void* p = alloc_scratch(bytes);                // (outside the lock: the runtime may run scratch_graph_done)
     if (!p) return nullptr;
-    g_scratch.push_back({dev, use, st, p, bytes});
+    if (cap) {
+        hipUserObject_t obj = nullptr;
+        if (hipUserObjectCreate(&obj, p, scratch_graph_done, 1, hipUserObjectNoDestructorSync) != hipSuccess) {
+            (void)hipGetLastError();
+            RelaxedCapture rc;
+            (void)hipFree(p);
+            return nullptr;
+        }
+        if (hipGraphRetainUserObject(graph, obj, 1, hipGraphUserObjectMove) != hipSuccess) {
+            (void)hipGetLastError();
+            (void)hipUserObjectRelease(obj, 1);    // leaves the buffer to scratch_reap
+            return nullptr;
+        }
+    }
+    std::lock_guard<std::mutex> lk(g.mu);
+    if (ScratchSlot* s = find()) s->old = true;
+    g.slots.push_back({dev, use, key, cap, p, bytes, false});
     return p;
 }
 

@@ -181,12 +181,15 @@ static inline hipStream_t as_stream(void* s) { return (hipStream_t)s; }
 // Number of compute units of the current device (cached per device).
 int rina_num_cus();
 
-// Scratch owned by the library, one buffer per (device, stream, use), grown
-// on demand and never shrunk: the output of a call that aliases input and
-// output, the row of a norm that runs before a matvec as its own launch, the
-// split activation rows of a product over several rows, the grouped rows of a
-// MoE block.  The uses of one call nest, so each has a buffer of its own; calls
-// on one stream run in order and share them.
+// Scratch owned by the library, grown on demand: the output of a call that
+// aliases input and output, the row of a norm that runs before a matvec as its
+// own launch, the split activation rows of a product over several rows, the
+// rotated rows and partials of an attention over several rows, the grouped rows
+// of a MoE block.  The uses of one call nest, so each has a buffer of its own.
+// One buffer per (device, stream, use): calls on one stream run in order and
+// share them.  Calls that are captured into a graph take buffers of that
+// capture, which live as long as the graph: its replays share them with nothing
+// else (a graph's own replays follow each other).
 // A call writes its buffer in one launch and reads it in a later one, so it
 // holds the stream's lock from get() until its last launch is queued (the
 // object's lifetime): the launches of two host threads that call on one stream

@@ -159,7 +159,9 @@ def test_rows_product_nonfinite_epilogues(rina, orc, qt, M, epi):
 
 def test_rows_product_under_capture(rina, orc):
     """A first product captured into a graph (its scratch is allocated during
-    the capture), replayed with other work between, equals the eager result."""
+    the capture), replayed with larger eager products on the capture stream
+    between (they overwrite and grow the stream's scratch), equals the eager
+    result."""
     import torch
     r = rng(9)
     M, N, K = 300, 96, 3200
@@ -167,18 +169,135 @@ def test_rows_product_under_capture(rina, orc):
     x = r.standard_normal((M, K)).astype(np.float32)
     hip, wd, xd, y = rina.load_hip(), dev(w), dev(x), empty(M * N)
     seg = rina.LinearSeg(wd.data_ptr(), None, y.data_ptr(), N)
+    big, yb = dev(r.standard_normal((4 * M, K)).astype(np.float32)), empty(4 * M * N)
+    segb = rina.LinearSeg(wd.data_ptr(), None, yb.data_ptr(), N)
     s = torch.cuda.Stream()
     torch.cuda.synchronize()
     g = torch.cuda.CUDAGraph()
     with torch.cuda.graph(g, stream=s):
         ok(hip.rina_hip_linear_fused(C.byref(seg), 1, 7, xd.data_ptr(), M, K, 0, 0, None, 0.0, s.cuda_stream), "captured")
     ref = x.astype(np.float64) @ W.reshape(N, K).T
-    for k in range(3):
+    for k in range(4):
         y.zero_()
+        ok(hip.rina_hip_linear_fused(C.byref(segb), 1, 7, big.data_ptr(), (k + 1) * M, K, 0, 0, None, 0.0, s.cuda_stream), "eager")
         torch.cuda.synchronize()
         g.replay()
         torch.cuda.synchronize()
         assert_close(host(y).reshape(M, N), ref, what="replay %d" % k)
+
+
+@pytest.mark.parametrize("qt", [7, 10])
+def test_graphs_of_one_capture_stream_replayed_on_two(rina, orc, qt):
+    """Two graphs captured on one stream and replayed on two others, beside
+    eager products on the capture stream: every product has its own rows (the
+    same bits as alone)."""
+    import torch
+    hip, M, N, K = rina.load_hip(), 40, 64, 2048
+    w, _ = weights(orc, qt, rng(qt), N * K)
+    wd = dev(w)
+    xs = [dev(rng(s).standard_normal((M, K)).astype(np.float32)) for s in range(3)]
+    alone = [empty(M * N) for _ in xs]
+    n = 60
+    ys = [[empty(M * N) for _ in range(n)] for _ in xs]
+
+    def call(i, y, st):
+        seg = rina.LinearSeg(wd.data_ptr(), None, y.data_ptr(), N)
+        ok(hip.rina_hip_linear_fused(C.byref(seg), 1, qt, xs[i].data_ptr(), M, K, 0, 0, None, 0.0, st.cuda_stream), "product")
+
+    cap, s1, s2 = (torch.cuda.Stream() for _ in range(3))
+    torch.cuda.synchronize()
+    for i in range(3):
+        call(i, alone[i], cap)
+    torch.cuda.synchronize()
+    graphs = [torch.cuda.CUDAGraph() for _ in range(2)]
+    for i, g in enumerate(graphs):
+        with torch.cuda.graph(g, stream=cap):
+            for y in ys[i]:
+                call(i, y, cap)
+    for k in range(5):
+        for i in (0, 1):
+            for y in ys[i]:
+                y.zero_()
+        torch.cuda.synchronize()
+        for g, s in zip(graphs, (s1, s2)):
+            with torch.cuda.stream(s):
+                g.replay()
+        for y in ys[2]:
+            call(2, y, cap)
+        torch.cuda.synchronize()
+        for i in range(3):
+            assert all(torch.equal(y, alone[i]) for y in ys[i]), "replay %d, rows %d" % (k, i)
+
+
+def test_scratch_of_graphs_goes_back(rina, orc):
+    """Graphs captured and destroyed one after the other: what their captures
+    allocated (the split rows of 1024 x 8192: 48 MB and more) goes back."""
+    import gc
+
+    import torch
+    hip, M, N, K = rina.load_hip(), 1024, 32, 8192
+    w, _ = weights(orc, 7, rng(3), N * K)
+    wd, xd, y = dev(w), dev(rng(4).standard_normal((M, K)).astype(np.float32)), empty(M * N)
+    seg = rina.LinearSeg(wd.data_ptr(), None, y.data_ptr(), N)
+    s = torch.cuda.Stream()
+
+    def call():
+        ok(hip.rina_hip_linear_fused(C.byref(seg), 1, 7, xd.data_ptr(), M, K, 0, 0, None, 0.0, s.cuda_stream), "product")
+
+    call()
+    torch.cuda.synchronize()
+    want = y.clone()
+    low = []
+    for k in range(24):
+        g = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(g, stream=s):
+            call()
+        y.zero_()
+        torch.cuda.synchronize()
+        g.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(y, want)
+        del g
+        gc.collect()
+        call()
+        torch.cuda.synchronize()
+        low.append(torch.cuda.mem_get_info()[0])
+    assert low[-1] > low[3] - 5 * M * K * 4     # far less than the 20 buffers of the captures between
+
+
+def test_scratch_of_ended_threads(rina, orc):
+    """Threads on their own default streams (hipStreamPerThread), one after the
+    other without a synchronization between: a new thread's split rows are
+    never written over those of one that ended, and what ended threads held
+    (48 MB and more each) goes back."""
+    import threading
+
+    import torch
+    hip, M, N, K, per_thread = rina.load_hip(), 1024, 32, 8192, 2
+    w, _ = weights(orc, 7, rng(5), N * K)
+    wd = dev(w)
+    xs = [dev(rng(s).standard_normal((M, K)).astype(np.float32)) for s in range(2)]
+    n = 24
+    ys = [empty(M * N) for _ in range(n)]
+    rcs = []
+    low = []
+
+    def call(k):
+        seg = rina.LinearSeg(wd.data_ptr(), None, ys[k].data_ptr(), N)
+        rcs.append(hip.rina_hip_linear_fused(C.byref(seg), 1, 7, xs[k % 2].data_ptr(), M, K, 0, 0, None, 0.0, per_thread))
+
+    torch.cuda.synchronize()
+    for k in range(n):
+        t = threading.Thread(target=call, args=(k,))
+        t.start()
+        t.join()
+        low.append(torch.cuda.mem_get_info()[0])
+    torch.cuda.synchronize()
+    assert rcs == [0] * n
+    for k in range(2, n):
+        assert torch.equal(ys[k], ys[k % 2])
+    assert not torch.equal(ys[0], ys[1])
+    assert low[-1] > low[3] - 5 * M * K * 4
 
 
 @pytest.mark.parametrize("qt", [7, 10, 6])
