@@ -1,47 +1,52 @@
 // Matrix products over several activation rows (prompts, short turns, the
 // rows of an expert) with quantized weights: out[M, N] = x[M, K] . W[N, K]^T
-// for Q4_0, Q4_0F and Q2_K, M >= 2, on the f16 matrix cores
-// (v_mfma_f32_16x16x32_f16) with fp32 sums.
+// for Q4_0, Q4_0F and Q2_K, M >= 2, on the bf16 matrix cores
+// (v_mfma_f32_16x16x32_bf16, v_mfma_f32_32x32x16_bf16) with fp32 sums.
 //
 // Two launches.  x_split_kernel (with the RMSNorm / LayerNorm prologue, or a
-// row gather, fused in) writes every row once as two f16 parts in matrix-core
-// fragment order; rows_gemm_kernel multiplies.
+// row gather, fused in) writes every row once as three bf16 parts in
+// matrix-core fragment order; rows16_kernel / rows32_kernel multiply.
 //
 // Precision.  A row is scaled by a power of two so that its largest magnitude
-// lies in [2^13, 2^14), then split x = h + l, h = f16(x), l = f16(x - h):
-// 22 significant bits at least (the split drops at most the last of the 24,
-// for one value in four), products with the small weight integers are exact
-// in the matrix core's fp32, sums are fp32.  The row scale comes out again in
-// the epilogue, exactly.  inf and NaN stay themselves in h (l = 0), so Q4 rows
-// that hold them give what fp32 products give; Q2_K rows give NaN (the minima
-// are a second product).  Against 64-bit
-// products the result is as close as with an exact three-part bf16 split and
-// one serial K loop (M 512, K 2048 / 8192: see the launch rules below), since
-// the K dimension is summed in up to eight independent slices.
+// lies in [2^13, 2^14), then split into three bf16 parts, 8 bits each: exact
+// for all 24 bits of every value down to 2^-123 of the row's largest.
+// Products with the small weight integers are exact in the matrix core's
+// fp32, sums are fp32; the row scale comes out again in the epilogue, exactly.
+// (Two f16 parts, a third less to load and multiply, lose the last bit of one
+// value in four and more below 2^-16 of the row's largest: 512 x 2048 x 8192
+// gate/up 82 us against 115, error against 64 bits 8.7e-8 against 7.0e-8 at K
+// 512, where the exact split it would have to match has 8.4e-8.)
+// inf and NaN stay in the first part: rows that hold them give what fp32
+// products give.  (Q2_K rows that hold infinities are added up in a path of
+// their own at the end, as their minima are a second product.)
+// Error against 64-bit products, Q4_0F, 512 rows: 1.0e-7 at K 2048, 1.8e-7 at
+// 8192 (1.56e-7 and 3.05e-7 in one serial K loop): the K dimension is summed
+// in up to eight independent slices.
 //
-// Weights.  Q4: q - 7 is exact in f16, one fp32 fma per output and 32-value
-// block applies the block scale.  Q2_K: sc * q <= 45 is exact in f16; d is
+// Weights.  Q4: q - 7 is exact in bf16, one fp32 fma per output and 32-value
+// block applies the block scale.  Q2_K: sc * q <= 45 is exact in bf16; d is
 // applied per 128-value page (per 32-value slice where rows do not start at
 // pages); the minima are a second, 16 times shorter contraction
 // -(dmin m) . X16 over the sums X16 of each 16 values of x: bf16 parts, two
 // of dmin m (exact: 15 bits) and three of X16 (exact).
 //
-// Structure.  A wave owns 16 MI rows x 16 NJ columns (per matrix) over its
-// share of K and reads its operands straight into registers: A fragments as
-// contiguous 1 KiB loads, weights as whole blocks (a lane loads one Q4 block,
-// v_permlane16/32_swap transposes the four blocks of a 128-value step across
-// the wave's four lane rows).  No LDS and no barrier in the K loop, so the
-// waves of a workgroup (NW across columns, KW along K, interleaved by 128
-// values) never wait for each other; the KW partial tiles meet in LDS once
-// at the end.
+// Structure.  A wave owns 16 MI rows x 16 columns, or 32 R rows x 32 C columns
+// (per matrix), over its share of K and reads its operands straight into
+// registers: A fragments as contiguous loads, weights as whole blocks (16-row
+// tiles: a lane loads one Q4 block, v_permlane16/32_swap transposes the four
+// blocks of a 128-value step across the wave's four lane rows; 32-row tiles:
+// through LDS of the wave's own).  No barrier in the K loop, so the waves of a
+// workgroup (NW across columns, KW along K, interleaved by 128 values) never
+// wait for each other; the KW partial tiles meet in LDS once at the end.
+// What bounds the 32-row tiles: 512 x 2048 x 8192 gate/up (114 us) without its
+// A loads in the K loop 94 us, without the block scales 107, without the
+// unpacking 114; matrix cores busy 47 % of its cycles.
 #include <type_traits>
 #include "rina_common.hpp"
 #include "rows_gemm.hpp"
 
 namespace {
 
-typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
-typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
@@ -60,24 +65,28 @@ __device__ __forceinline__ u32x2 gld2(const uint8_t* p) {
     return *(const __attribute__((address_space(1))) T*)p;
 }
 
+// the upper halves of two fp32 values as one dword
+__device__ __forceinline__ uint32_t hi16_pair(uint32_t lo, uint32_t hi) { return __builtin_amdgcn_perm(hi, lo, 0x07060302u); }
+
+constexpr int kParts = 3;              // bf16 parts of an activation
+constexpr int kStep = 64 * kParts;     // 16-byte units of a 16-row tile's 32-value step
+
 __device__ __forceinline__ float silu_mul(float g, float u) { return g / (1.0f + expf(-g)) * u; }
 
 // ---------------------------------------------------------------------------
 // activation rows -> f16 fragments
 // ---------------------------------------------------------------------------
-// Layout: 16-row tile mt, 32-value step ks, part p (0: h, 1: l), 64 lanes of
-// 16 bytes; lane (r, f) holds row 16 mt + r, values 32 ks + 8 f .. + 7 in the
-// order in which the weight bytes unpack: Q4 dword j = values (j, j + 4);
-// Q2_K dwords = values (0, 2), (1, 3), (4, 6), (5, 7).  Q2_K also gets the
-// sums of 16 values as three bf16 parts: 16-row tile, window of 32 sums,
-// part, lane (r, f) = sums 8 f .. + 7 of row r.  K is padded with zeros to
-// whole 128-value steps (and windows), rows to whole tiles.
+// Layout: 16-row tile mt, 32-value step ks, part p (the largest first), 64
+// lanes of 16 bytes; lane (r, f) holds row 16 mt + r, values 32 ks + 8 f .. + 7.
+// Q2_K also gets the sums of 16 values as three bf16 parts: 16-row tile, window
+// of 32 sums, part, lane (r, f) = sums 8 f .. + 7 of row r.  K is padded with
+// zeros to whole 128-value steps (and windows), rows to whole tiles.
 struct SplitXArgs {
     const float* x;
     const float* nw;
     const int* src;        // row gather: packed row r is x row src[r] (< 0: zero row)
     uint4* xp;
-    float* xs;             // [rows] 2^-e of the row scale 2^e
+    float* xs;             // [rows] 2^-e of the row scale 2^e (Q2_K: -2^-e if the row holds inf and no NaN)
     uint16_t* xg;          // Q2_K: group-sum fragments
     const int* used;       // grouped rows: 16-row tiles in use (NULL: all)
     int M, K, nks, ngw;
@@ -95,7 +104,7 @@ constexpr int kSplitRows = 4;
 
 template <bool Q2, int NU>
 __global__ __launch_bounds__(256 * kSplitRows) void x_split_kernel(SplitXArgs a) {
-    __shared__ float s_red[3][kSplitRows][4];
+    __shared__ float s_red[4][kSplitRows][4];
     const int r = threadIdx.x >> 8, tid = threadIdx.x & 255, wave = tid >> 6, lane = tid & 63;
     const int row = blockIdx.x * kSplitRows + r, mt = row >> 4;
     if (a.used && mt >= __builtin_amdgcn_readfirstlane(gld(a.used))) return;   // the whole workgroup: 4 rows of one tile
@@ -181,7 +190,7 @@ __global__ __launch_bounds__(256 * kSplitRows) void x_split_kernel(SplitXArgs a)
 #pragma unroll
         for (int i = 0; i < NU; i++) normed(tid + 256 * i, v[i][0], v[i][1]);
     }
-    float mx = 0.f;                                 // largest finite magnitude
+    float mx = 0.f, bad = 0.f;                      // largest finite magnitude; 1: inf, 2: NaN
     each([&](int u, const f32x4& p0, const f32x4& q0) {
         f32x4 p = p0, q = q0;
         if (NU == 0) normed(u, p, q);
@@ -189,37 +198,49 @@ __global__ __launch_bounds__(256 * kSplitRows) void x_split_kernel(SplitXArgs a)
         for (int i = 0; i < 4; i++) {
             mx = fmaxf(mx, fabsf(p[i]) < INFINITY ? fabsf(p[i]) : 0.f);
             mx = fmaxf(mx, fabsf(q[i]) < INFINITY ? fabsf(q[i]) : 0.f);
+            if (Q2) {
+                bad = fmaxf(bad, fabsf(p[i]) < INFINITY ? 0.f : p[i] == p[i] ? 1.f : 2.f);
+                bad = fmaxf(bad, fabsf(q[i]) < INFINITY ? 0.f : q[i] == q[i] ? 1.f : 2.f);
+            }
         }
     });
     mx = wave_max(mx);
-    if (lane == 0) s_red[2][r][wave] = mx;
+    if (Q2) bad = wave_max(bad);
+    if (lane == 0) {
+        s_red[2][r][wave] = mx;
+        if (Q2) s_red[3][r][wave] = bad;
+    }
     __syncthreads();
     mx = fmaxf(fmaxf(s_red[2][r][0], s_red[2][r][1]), fmaxf(s_red[2][r][2], s_red[2][r][3]));
+    if (Q2) bad = fmaxf(fmaxf(s_red[3][r][0], s_red[3][r][1]), fmaxf(s_red[3][r][2], s_red[3][r][3]));
     // 2^e with mx 2^e in [2^13, 2^14); rows of zeros keep 2^0
     const int ex = (int)((__float_as_uint(mx) >> 23) & 0xFF) - 127;
     const int e = mx > 0.f ? min(max(13 - ex, -126), 126) : 0;
     const float sc = __uint_as_float((uint32_t)(e + 127) << 23);
-    if (tid == 0) gst(a.xs + row, __uint_as_float((uint32_t)(127 - e) << 23));
-    uint4* xp = a.xp + (int64_t)mt * a.nks * 128 + (row & 15);
+    if (tid == 0) gst(a.xs + row, __uint_as_float((uint32_t)(127 - e) << 23 | (bad == 1.f ? 0x80000000u : 0u)));
+    uint4* xp = a.xp + (int64_t)mt * a.nks * kStep + (row & 15);
     each([&](int u, const f32x4& p0, const f32x4& q0) {
         f32x4 p = p0, q = q0;
         if (NU == 0) normed(u, p, q);
         float w[8];
-        _Float16 h[8], l[8];
 #pragma unroll
         for (int i = 0; i < 4; i++) { w[i] = p[i] * sc; w[4 + i] = q[i] * sc; }
+        uint4* d = xp + (int64_t)(u >> 2) * kStep + (u & 3) * 16;
+        float r[8];
 #pragma unroll
-        for (int i = 0; i < 8; i++) {
-            h[i] = (_Float16)w[i];
-            l[i] = fabsf(w[i]) < INFINITY ? (_Float16)(w[i] - (float)h[i]) : (_Float16)0.0f;
+        for (int i = 0; i < 8; i++) r[i] = w[i];
+#pragma unroll
+        for (int k = 0; k < kParts; k++) {
+            uint32_t b[8];
+#pragma unroll
+            for (int i = 0; i < 8; i++) {
+                b[i] = __float_as_uint(r[i]);
+                const bool fin = fabsf(r[i]) < INFINITY;
+                if (!(r[i] == r[i])) b[i] = 0x7FC00000u;            // (the low half of a NaN may be all it has)
+                r[i] = fin ? r[i] - __uint_as_float(b[i] & 0xFFFF0000u) : 0.f;
+            }
+            gst((u32x4*)(d + 64 * k), u32x4{hi16_pair(b[0], b[1]), hi16_pair(b[2], b[3]), hi16_pair(b[4], b[5]), hi16_pair(b[6], b[7])});
         }
-        constexpr int O[2][8] = {{0, 4, 1, 5, 2, 6, 3, 7}, {0, 2, 1, 3, 4, 6, 5, 7}};
-        f16x8 hv, lv;
-#pragma unroll
-        for (int i = 0; i < 8; i++) { hv[i] = h[O[Q2][i]]; lv[i] = l[O[Q2][i]]; }
-        uint4* d = xp + (int64_t)(u >> 2) * 128 + (u & 3) * 16;
-        gst((f16x8*)d, hv);
-        gst((f16x8*)(d + 64), lv);
         if (Q2) {
             // sums of 16 values: threads 2 i, 2 i + 1 hold the two units
             float s = ((w[0] + w[1]) + (w[2] + w[3])) + ((w[4] + w[5]) + (w[6] + w[7]));
@@ -339,36 +360,32 @@ __device__ __forceinline__ void w_load(const uint8_t* w, int n, int K, int ss, i
     }
 }
 
-// (v & mask) | 0x64006400: bit fields of both halves as f16 1024 + field (one
-// v_and_or_b32; written out because the compiler splits it into two literals)
-__device__ __forceinline__ f16x2 f16_field(uint32_t v, uint32_t mask) {
-    uint32_t r;
-    asm("v_and_or_b32 %0, %1, %2, %3" : "=v"(r) : "v"(v), "s"(mask), "v"(0x64006400u));
-    return __builtin_bit_cast(f16x2, r);
-}
-__device__ __forceinline__ f16x2 f16_both(float v) { return f16x2{(_Float16)v, (_Float16)v}; }
-__device__ __forceinline__ uint32_t f16_fma(f16x2 a, f16x2 b, f16x2 c) {
-    return __builtin_bit_cast(uint32_t, __builtin_elementwise_fma(a, b, c));
-}
-// the eight nibbles of a dword -> q - 7 as f16, dword j = nibbles (j, j + 4);
-// a field at bit 4 of its half is 1024 + 16 q: the scale by 1/16 is exact
+// the eight nibbles of a dword -> q - 7 as bf16, in order (small integers: exact)
 __device__ __forceinline__ u32x4 q4_unpack(uint32_t x) {
-    const uint32_t y = x >> 8;
-    const f16x2 one = f16_both(1.0f), m7 = f16_both(-1031.0f), sx = f16_both(0.0625f), m71 = f16_both(-71.0f);
-    return u32x4{f16_fma(f16_field(x, 0x000F000Fu), one, m7), f16_fma(f16_field(x, 0x00F000F0u), sx, m71),
-                 f16_fma(f16_field(y, 0x000F000Fu), one, m7), f16_fma(f16_field(y, 0x00F000F0u), sx, m71)};
+    const uint32_t lo = and_opaque(x, 0x0F0F0F0Fu), hi = and_opaque(x >> 4, 0x0F0F0F0Fu);
+    u32x4 r;
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+        const float f0 = (float)((lo >> (8 * j)) & 0xFF) - 7.0f, f1 = (float)((hi >> (8 * j)) & 0xFF) - 7.0f;
+        r[j] = hi16_pair(__float_as_uint(f0), __float_as_uint(f1));
+    }
+    return r;
 }
-// sc * q as f16 for the 2-bit fields at bit 2 st of eight bytes, dwords =
-// bytes (0, 2), (1, 3), (4, 6), (5, 7); a field there is 1024 + 4^st q, so the
-// factor is sc 4^-st and every step is exact (sc <= 15); by: the scale byte
+// sc * q as bf16 (at most 45: exact) for the 2-bit fields at bit 2 st of eight
+// bytes, in order; by: the scale byte
 __device__ __forceinline__ u32x4 q2_unpack(u32x2 b, uint32_t by, int st) {
-    const float f = st == 0 ? 1.0f : st == 1 ? 0.25f : st == 2 ? 0.0625f : 0.015625f;
-    const uint32_t mask = 0x00030003u << (2 * st);
-    const f16x2 t = f16_field(__builtin_amdgcn_perm(by, by, 0x0C000C00u), 0x000F000Fu);
-    const f16x2 sc = __builtin_bit_cast(f16x2, f16_fma(t, f16_both(f), f16_both(-1024.0f * f)));
-    const f16x2 m = sc * f16_both(-1024.0f);
-    return u32x4{f16_fma(f16_field(b.x, mask), sc, m), f16_fma(f16_field(b.x >> 8, mask), sc, m),
-                 f16_fma(f16_field(b.y, mask), sc, m), f16_fma(f16_field(b.y >> 8, mask), sc, m)};
+    const float sc = (float)(by & 15u);
+    u32x4 r;
+#pragma unroll
+    for (int h = 0; h < 2; h++) {
+        const uint32_t q = and_opaque((h ? b.y : b.x) >> (2 * st), 0x03030303u);
+        float f[4];
+#pragma unroll
+        for (int j = 0; j < 4; j++) f[j] = sc * (float)((q >> (8 * j)) & 0xFF);
+        r[2 * h] = hi16_pair(__float_as_uint(f[0]), __float_as_uint(f[1]));
+        r[2 * h + 1] = hi16_pair(__float_as_uint(f[2]), __float_as_uint(f[3]));
+    }
+    return r;
 }
 
 // nibble dwords and fp32 scale of a Q4 block from the five dwords at its
@@ -433,10 +450,10 @@ struct WStep {
             }
         }
     }
-    __device__ __forceinline__ f16x8 frag(int st) const {
-        if constexpr (FMT == FMT_Q4_0F || FMT == FMT_Q4_0) return __builtin_bit_cast(f16x8, q4_unpack(n[st]));
-        else if constexpr (FMT == FMT_Q2_K) return __builtin_bit_cast(f16x8, q2_unpack(q[0], s[st], st));
-        else return __builtin_bit_cast(f16x8, q2_unpack(u32x2{q[st].x >> (s[st] >> 8), q[st].y >> (s[st] >> 8)}, s[st], 0));
+    __device__ __forceinline__ bf16x8 frag(int st) const {
+        if constexpr (FMT == FMT_Q4_0F || FMT == FMT_Q4_0) return __builtin_bit_cast(bf16x8, q4_unpack(n[st]));
+        else if constexpr (FMT == FMT_Q2_K) return __builtin_bit_cast(bf16x8, q2_unpack(q[0], s[st], st));
+        else return __builtin_bit_cast(bf16x8, q2_unpack(u32x2{q[st].x >> (s[st] >> 8), q[st].y >> (s[st] >> 8)}, s[st], 0));
     }
 };
 
@@ -523,7 +540,49 @@ __device__ __forceinline__ void finish(const RowsArgs& a, const Tile& t, int r, 
     else gst(o, v);
 }
 
-// The same for 32-column tiles (two lane rows of 32 columns): a lane holds
+// Q2_K rows of a tile that hold infinities (xs < 0): the sums over those
+// values alone (the others are finite) with the weights dequantized, as fp32
+// products give them: the infinity of the weight's sign, NaN for a weight of
+// zero or where both signs meet.  Column c per lane, COLS lanes of columns, the
+// 64 / COLS lane rows g along K.
+template <int NMAT, int COLS>
+__device__ void inf_rows(const RowsArgs& a, const Tile& t, int r0, int rows, int c, int g) {
+    const int n = c < t.N ? c : 0;
+    auto weight = [&](const uint8_t* w, int k) {
+        const int64_t e = (int64_t)n * a.K + k;
+        const uint8_t* b = w + (e >> 8) * 84;
+        const int i = (int)(e & 255);
+        const int sc = gld(b + (i >> 4)), q = (gld(b + 16 + 32 * (i >> 7) + (i & 31)) >> (2 * ((i & 127) >> 5))) & 3;
+        return fmaf(f16_to_f32(gld((const uint16_t*)(b + 80))) * (float)(sc & 15), (float)q,
+                    -(f16_to_f32(gld((const uint16_t*)(b + 82))) * (float)(sc >> 4)));
+    };
+#pragma unroll 1
+    for (int r = r0; r < min(r0 + rows, t.mend); r++) {
+        if (!(gld(a.xs + r) < 0.f)) continue;
+        float v = 0.f, u = 0.f;
+        const u32x4* xp = (const u32x4*)a.xp + (int64_t)(r >> 4) * a.nks * kStep + (r & 15);
+#pragma unroll 1
+        for (int un = g; un < a.K >> 3; un += 64 / COLS) {
+            const u32x4 x = gld(xp + (int64_t)(un >> 2) * kStep + (un & 3) * 16);
+#pragma unroll 1
+            for (int i = 0; i < 8; i++) {
+                const uint32_t d = i < 2 ? x.x : i < 4 ? x.y : i < 6 ? x.z : x.w, h = (i & 1) ? d >> 16 : d & 0xFFFFu;
+                if ((h & 0x7FFFu) != 0x7F80u) continue;
+                const float xi = __uint_as_float(h << 16);
+                v = fmaf(xi, weight(t.w, 8 * un + i), v);
+                if (NMAT == 2) u = fmaf(xi, weight(t.w2, 8 * un + i), u);
+            }
+        }
+#pragma unroll
+        for (int m = COLS; m < 64; m *= 2) {
+            v += __shfl_xor(v, m);
+            u += __shfl_xor(u, m);
+        }
+        if (g == 0) finish<NMAT>(a, t, r, c, v, u);
+    }
+}
+
+// Weights as loaded for 32-column tiles (two lane rows of 32 columns): a lane holds
 // blocks 4 ss + f and 4 ss + 2 + f of its column, or its half of a page
 template <int FMT>
 struct WRaw32;
@@ -595,12 +654,12 @@ struct WStep32 {
         }
     }
     // weights of 16-value half h of 32-value step st
-    __device__ __forceinline__ f16x8 frag(int st, int h) const {
-        if constexpr (FMT == FMT_Q4_0F || FMT == FMT_Q4_0) return __builtin_bit_cast(f16x8, q4_unpack(n[st][h]));
-        else if constexpr (FMT == FMT_Q2_K) return __builtin_bit_cast(f16x8, q2_unpack(q[0][h], s[st] >> (8 * h), st));
+    __device__ __forceinline__ bf16x8 frag(int st, int h) const {
+        if constexpr (FMT == FMT_Q4_0F || FMT == FMT_Q4_0) return __builtin_bit_cast(bf16x8, q4_unpack(n[st][h]));
+        else if constexpr (FMT == FMT_Q2_K) return __builtin_bit_cast(bf16x8, q2_unpack(q[0][h], s[st] >> (8 * h), st));
         else {
             const uint32_t sh = s[st] >> 16;
-            return __builtin_bit_cast(f16x8, q2_unpack(u32x2{q[st][h].x >> sh, q[st][h].y >> sh}, s[st] >> (8 * h), 0));
+            return __builtin_bit_cast(bf16x8, q2_unpack(u32x2{q[st][h].x >> sh, q[st][h].y >> sh}, s[st] >> (8 * h), 0));
         }
     }
 };
@@ -627,16 +686,16 @@ __global__ __launch_bounds__(512, 2) void rows16_kernel(RowsArgs a) {
     const int c0 = (t.bx * a.NW + wn) * 16 + fr, N = t.N;
     const int K = a.K, nss = a.nks >> 2, col = c0 < N ? c0 : 0;
     const int mtiles = (a.M + 15) >> 4;
-    const f16x8* ap[MI];
+    const bf16x8* ap[MI];
 #pragma unroll
-    for (int i = 0; i < MI; i++) ap[i] = (const f16x8*)a.xp + (int64_t)min(t.r16 + i, mtiles - 1) * a.nks * 128 + lane;
+    for (int i = 0; i < MI; i++) ap[i] = (const bf16x8*)a.xp + (int64_t)min(t.r16 + i, mtiles - 1) * a.nks * kStep + lane;
     f32x4 acc[NMAT][MI];
 #pragma unroll
     for (int m = 0; m < NMAT; m++)
 #pragma unroll
         for (int i = 0; i < MI; i++) acc[m][i] = f32x4{0.f, 0.f, 0.f, 0.f};
     WRaw<FMT> raw[BT][NMAT];
-    f16x8 af[MI][8];
+    bf16x8 af[MI][2 * kParts];                      // 64 values: half a step
     // batch b: steps BT b .. + BT - 1 (past the end: the last step again, not multiplied)
     auto load_w = [&](int b) {
 #pragma unroll
@@ -644,17 +703,17 @@ __global__ __launch_bounds__(512, 2) void rows16_kernel(RowsArgs a) {
 #pragma unroll
             for (int m = 0; m < NMAT; m++) w_load<FMT>(m ? t.w2 : t.w, col, K, min(BT * b + s, nss - 1), f, raw[s][m]);
     };
-    auto load_a = [&](int ss) {
+    auto load_a = [&](int ss, int half) {
 #pragma unroll
         for (int i = 0; i < MI; i++)
 #pragma unroll
-            for (int c = 0; c < 8; c++) af[i][c] = gld(ap[i] + (int64_t)min(ss, nss - 1) * 512 + 64 * c);
+            for (int c = 0; c < 2 * kParts; c++) af[i][c] = gld(ap[i] + (int64_t)(4 * min(ss, nss - 1) + 2 * half) * kStep + 64 * c);
     };
     constexpr bool PAGE = FMT == FMT_Q2_K;          // one scale per 128-value step
     const int nb = (nss + BT - 1) / BT;
     if (wk < nb) {
         load_w(wk);
-        load_a(BT * wk);
+        load_a(BT * wk, 0);
     }
     for (int b = wk; b < nb; b += a.KW) {
         WStep<FMT> ws[BT][NMAT];
@@ -665,32 +724,36 @@ __global__ __launch_bounds__(512, 2) void rows16_kernel(RowsArgs a) {
         const int bn = b + a.KW < nb ? b + a.KW : b;   // the last batch loads itself again
 #pragma unroll
         for (int s = 0; s < BT; s++) {
-            f16x8 at[MI][8];
+            f32x4 d[NMAT][MI];
 #pragma unroll
-            for (int i = 0; i < MI; i++)
+            for (int half = 0; half < 2; half++) {
+                bf16x8 at[MI][2 * kParts];
 #pragma unroll
-                for (int c = 0; c < 8; c++) at[i][c] = af[i][c];
-            load_a(s + 1 < BT ? BT * b + s + 1 : BT * bn);
-            if (s == 0) load_w(bn);
-            __builtin_amdgcn_sched_barrier(0);      // issued before this step's products
-            if (BT > 1 && BT * b + s >= nss) continue;
+                for (int i = 0; i < MI; i++)
 #pragma unroll
-            for (int m = 0; m < NMAT; m++) {
-                f32x4 d[MI];
+                    for (int c = 0; c < 2 * kParts; c++) at[i][c] = af[i][c];
+                load_a(half == 0 ? BT * b + s : s + 1 < BT ? BT * b + s + 1 : BT * bn, half ^ 1);
+                if (s == 0 && half == 0) load_w(bn);
+                __builtin_amdgcn_sched_barrier(0);  // issued before these products
+                if (BT > 1 && BT * b + s >= nss) continue;
 #pragma unroll
-                for (int st = 0; st < 4; st++) {
-                    const f16x8 w = ws[s][m].frag(st);
+                for (int m = 0; m < NMAT; m++) {
 #pragma unroll
-                    for (int i = 0; i < MI; i++) {
-                        if (!PAGE || st == 0) d[i] = f32x4{0.f, 0.f, 0.f, 0.f};
-                        d[i] = __builtin_amdgcn_mfma_f32_16x16x32_f16(at[i][2 * st + 1], w, d[i], 0, 0, 0);
-                    }
+                    for (int st = 2 * half; st < 2 * half + 2; st++) {
+                        const bf16x8 w = ws[s][m].frag(st);
+                        // smallest parts first
 #pragma unroll
-                    for (int i = 0; i < MI; i++) {
-                        d[i] = __builtin_amdgcn_mfma_f32_16x16x32_f16(at[i][2 * st], w, d[i], 0, 0, 0);
+                        for (int p = kParts - 1; p >= 0; p--)
+#pragma unroll
+                            for (int i = 0; i < MI; i++) {
+                                if (p == kParts - 1 && (!PAGE || st == 0)) d[m][i] = f32x4{0.f, 0.f, 0.f, 0.f};
+                                d[m][i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(at[i][kParts * (st & 1) + p], w, d[m][i], 0, 0, 0);
+                            }
                         if (!PAGE || st == 3) {
 #pragma unroll
-                            for (int e = 0; e < 4; e++) acc[m][i][e] = fmaf(ws[s][m].sc[PAGE ? 0 : st], d[i][e], acc[m][i][e]);
+                            for (int i = 0; i < MI; i++)
+#pragma unroll
+                                for (int e = 0; e < 4; e++) acc[m][i][e] = fmaf(ws[s][m].sc[PAGE ? 0 : st], d[m][i][e], acc[m][i][e]);
                         }
                     }
                 }
@@ -743,14 +806,20 @@ __global__ __launch_bounds__(512, 2) void rows16_kernel(RowsArgs a) {
         __syncthreads();
     }
     if (wk > 0) return;
+    constexpr bool Q2 = FMT == FMT_Q2_K || FMT == FMT_Q2_S;
+    bool inf = false;                               // rows of inf_rows
 #pragma unroll
     for (int i = 0; i < MI; i++) {
         const int r0 = (t.r16 + i) * 16 + 4 * f;
         if (r0 >= t.mend) continue;
         const f32x4 sc = gld((const f32x4*)(a.xs + r0));
 #pragma unroll
-        for (int e = 0; e < 4; e++) finish<NMAT>(a, t, r0 + e, c0, acc[0][i][e] * sc[e], acc[NMAT - 1][i][e] * sc[e]);
+        for (int e = 0; e < 4; e++) {
+            if (Q2 && sc[e] < 0.f) inf |= r0 + e < t.mend;
+            else finish<NMAT>(a, t, r0 + e, c0, acc[0][i][e] * sc[e], acc[NMAT - 1][i][e] * sc[e]);
+        }
     }
+    if (Q2 && __any(inf)) inf_rows<NMAT, 16>(a, t, t.r16 * 16, 16 * MI, c0, f);
 }
 
 // ---- M > 32: v_mfma_f32_32x32x16_f16 tiles ----
@@ -792,25 +861,26 @@ __global__ __launch_bounds__(512, 2) void rows32_kernel(RowsArgs a) {
     constexpr int BB = FMT == FMT_Q4_0F ? 20 : 18;
     const int nb = K >> 5;
     u32x4 ch[Q4 ? NCH : 1];
-    const uint8_t* cw[Q4 ? NCH : 1];                // the chunk at step 0 (4-byte aligned)
-    int64_t cmax[Q4 ? NCH : 1];                     // the last offset from there that stays inside the matrix,
-    int cpull[Q4 ? NCH : 1];                        // and what it was pulled back by at step 0
+    // the tile's matrices from their first column (4-byte aligned down), the
+    // chunk's offset there at step 0 and the last one that stays inside the
+    // matrix (a tile's columns are far below 2 GB)
+    const int64_t tile0 = ((int64_t)n0 * nb * BB) & ~(int64_t)3;
+    int co[Q4 ? NCH : 1];
+    const int clast = Q4 ? (int)min((int64_t)N * nb * BB - 16 - tile0, (int64_t)0x7FFFFFFF) : 0;
+    const uint8_t* const wt[2] = {t.w + tile0, NMAT == 2 ? t.w2 + tile0 : nullptr};
+    auto chunk_m = [&](int i) { return NMAT == 2 && min(64 * i + lane, 5 * NCOL - 1) >= 5 * 32 * C; };
     if constexpr (Q4) {
 #pragma unroll
         for (int i = 0; i < NCH; i++) {
             const int q = min(64 * i + lane, 5 * NCOL - 1), cr = q / 5, c = q - 5 * cr;
-            const int m = cr / (32 * C), n = min(n0 + cr % (32 * C), N - 1);
-            const int64_t off = (((int64_t)n * nb * BB) & ~(int64_t)3) + 16 * c;
-            const int64_t last = (int64_t)N * nb * BB - 16;
-            cw[i] = (m ? t.w2 : t.w) + min(off, last);
-            cmax[i] = last - min(off, last);
-            cpull[i] = (int)(off - min(off, last));
+            const int n = min(n0 + cr % (32 * C), N - 1);
+            co[i] = (int)((((int64_t)n * nb * BB) & ~(int64_t)3) - tile0) + 16 * c;
         }
     }
     auto load_w = [&](int ss) {
         if constexpr (Q4) {
 #pragma unroll
-            for (int i = 0; i < NCH; i++) ch[i] = gld4(cw[i] + min((int64_t)ss * (4 * BB), cmax[i]));
+            for (int i = 0; i < NCH; i++) ch[i] = gld4((chunk_m(i) ? wt[1] : wt[0]) + min(co[i] + ss * (4 * BB), clast));
         } else {
 #pragma unroll
             for (int m = 0; m < NMAT; m++)
@@ -823,52 +893,48 @@ __global__ __launch_bounds__(512, 2) void rows32_kernel(RowsArgs a) {
     const int lu = (fr & 15) + 16 * f;
     constexpr bool PAGE = FMT == FMT_Q2_K;          // one scale per 128-value step
     f32x16 pd[PAGE ? NMAT : 1][PAGE ? R : 1][PAGE ? C : 1];
-    // the products of step st (32 values) of a 128-value step; at[i][h][p]
-    auto mul = [&](const WStep32<FMT> (&ws)[NMAT][C], const f16x8 (&at)[R][2][2], int st) {
+    // the products of step st (32 values) of a 128-value step for column tile j
+    // of matrix m: rows x[half][row tile][part]
+    auto mul = [&](const WStep32<FMT>& w, const bf16x8 (&x)[2][R][kParts], int st, int m, int j) {
+        f32x16 d[R];
+        const bf16x8 b[2] = {w.frag(st, 0), w.frag(st, 1)};
+        // smallest parts first, of all 32 values: the sum is rounded at its full size twice
 #pragma unroll
-        for (int m = 0; m < NMAT; m++)
+        for (int p = kParts - 1; p >= 0; p--)
 #pragma unroll
-            for (int j = 0; j < C; j++) {
-                f32x16 d[R];
-#pragma unroll
-                for (int h = 0; h < 2; h++) {
-                    const f16x8 b = ws[m][j].frag(st, h);
-#pragma unroll
-                    for (int p = 1; p >= 0; p--)
-#pragma unroll
-                        for (int i = 0; i < R; i++) {
-                            f32x16 c;
-                            if (h == 0 && p == 1) {
-                                if (PAGE && st > 0) c = pd[PAGE ? m : 0][PAGE ? i : 0][PAGE ? j : 0];
-                                else {
-#pragma unroll
-                                    for (int e = 0; e < 16; e++) c[e] = 0.f;
-                                }
-                            } else {
-                                c = d[i];
-                            }
-                            d[i] = __builtin_amdgcn_mfma_f32_32x32x16_f16(at[i][h][p], b, c, 0, 0, 0);
-                        }
-                }
+            for (int h = 0; h < 2; h++)
 #pragma unroll
                 for (int i = 0; i < R; i++) {
-                    if constexpr (PAGE) pd[m][i][j] = d[i];
-                    if (!PAGE || st == 3) {
-                        const float sc = ws[m][j].sc[PAGE ? 0 : st];
+                    f32x16 c;
+                    if (h == 0 && p == kParts - 1) {
+                        if (PAGE && st > 0) c = pd[PAGE ? m : 0][PAGE ? i : 0][PAGE ? j : 0];
+                        else {
 #pragma unroll
-                        for (int e = 0; e < 16; e++) acc[m][i][j][e] = fmaf(sc, d[i][e], acc[m][i][j][e]);
+                            for (int e = 0; e < 16; e++) c[e] = 0.f;
+                        }
+                    } else {
+                        c = d[i];
                     }
-                    // consumed here: left alone, the compiler defers the scale
-                    // products of a whole step and spills
-                    if constexpr (PAGE) asm volatile("" : "+v"(pd[m][i][j]));
-                    else asm volatile("" : "+v"(acc[m][i][j]));
+                    d[i] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(x[h][i][p], b[h], c, 0, 0, 0);
                 }
+#pragma unroll
+        for (int i = 0; i < R; i++) {
+            if constexpr (PAGE) pd[m][i][j] = d[i];
+            if (!PAGE || st == 3) {
+                const float sc = w.sc[PAGE ? 0 : st];
+#pragma unroll
+                for (int e = 0; e < 16; e++) acc[m][i][j][e] = fmaf(sc, d[i][e], acc[m][i][j][e]);
             }
+            // consumed here: left alone, the compiler defers the scale
+            // products of a whole step and spills
+            if constexpr (PAGE) asm volatile("" : "+v"(pd[m][i][j]));
+            else asm volatile("" : "+v"(acc[m][i][j]));
+        }
     };
     bool edge = false;                              // a chunk of this wave ends past the matrix in the last step
     if constexpr (Q4) {
 #pragma unroll
-        for (int i = 0; i < NCH; i++) edge |= cpull[i] > 0 || cmax[i] < (int64_t)(nss - 1) * (4 * BB);
+        for (int i = 0; i < NCH; i++) edge |= co[i] + (nss - 1) * (4 * BB) > clast;
         edge = __any(edge);
     }
     auto take = [&](WStep32<FMT> (&ws)[NMAT][C], int ss) {
@@ -883,7 +949,7 @@ __global__ __launch_bounds__(512, 2) void rows32_kernel(RowsArgs a) {
                 // one block at least, so never before the row's first)
 #pragma unroll
                 for (int i = 0; i < NCH; i++) {
-                    const int64_t back = (int64_t)ss * (4 * BB) + cpull[i] - cmax[i];
+                    const int back = co[i] + ss * (4 * BB) - clast;
                     uint16_t* d = (uint16_t*)(wb + 64 * i + lane) - (back > 0 ? back / 2 : 0);   // (18-byte blocks: an even count)
                     const uint32_t v[4] = {ch[i].x, ch[i].y, ch[i].z, ch[i].w};
 #pragma unroll
@@ -920,17 +986,17 @@ __global__ __launch_bounds__(512, 2) void rows32_kernel(RowsArgs a) {
         }
     };
     {
-        const f16x8* ap[R];
+        const bf16x8* ap[R];
 #pragma unroll
-        for (int i = 0; i < R; i++) ap[i] = (const f16x8*)a.xp + (int64_t)min(t.r16 + 2 * i + (fr >> 4), mtiles - 1) * a.nks * 128 + lu;
-        f16x8 af[2][R][2][2];
-        auto load_a = [&](f16x8 (&x)[R][2][2], int ks) {
+        for (int i = 0; i < R; i++) ap[i] = (const bf16x8*)a.xp + (int64_t)min(t.r16 + 2 * i + (fr >> 4), mtiles - 1) * a.nks * kStep + lu;
+        bf16x8 af[2][2][R][kParts];                 // two 32-value steps, by halves
+        auto load_a = [&](bf16x8 (&x)[2][R][kParts], int ks) {
 #pragma unroll
-            for (int i = 0; i < R; i++)
+            for (int h = 0; h < 2; h++)
 #pragma unroll
-                for (int h = 0; h < 2; h++)
+                for (int i = 0; i < R; i++)
 #pragma unroll
-                    for (int p = 0; p < 2; p++) x[i][h][p] = gld(ap[i] + (int64_t)ks * 128 + 64 * p + 32 * h);
+                    for (int p = 0; p < kParts; p++) x[h][i][p] = gld(ap[i] + (int64_t)ks * kStep + 64 * p + 32 * h);
         };
         if (wk < nss) {
             load_w(wk);
@@ -945,7 +1011,10 @@ __global__ __launch_bounds__(512, 2) void rows32_kernel(RowsArgs a) {
                 load_a(af[(st & 1) ^ 1], st < 3 ? 4 * ss + st + 1 : 4 * sn);
                 if (st == 0) load_w(sn);
                 __builtin_amdgcn_sched_barrier(0);  // issued before this step's products
-                mul(ws, af[st & 1], st);
+#pragma unroll
+                for (int m = 0; m < NMAT; m++)
+#pragma unroll
+                    for (int j = 0; j < C; j++) mul(ws[m][j], af[st & 1], st, m, j);
             }
         }
     }
@@ -1013,6 +1082,8 @@ __global__ __launch_bounds__(512, 2) void rows32_kernel(RowsArgs a) {
         }
         if (wk > 0) return;
     }
+    constexpr bool Q2 = FMT == FMT_Q2_K || FMT == FMT_Q2_S;
+    bool inf = false;                               // rows of inf_rows
     // result element e of lane l: row 8 (e / 4) + 4 f + e % 4, column l % 32
 #pragma unroll
     for (int i = 0; i < R; i++)
@@ -1024,9 +1095,15 @@ __global__ __launch_bounds__(512, 2) void rows32_kernel(RowsArgs a) {
 #pragma unroll
             for (int j = 0; j < C; j++)
 #pragma unroll
-                for (int e = 0; e < 4; e++)
-                    finish<NMAT>(a, t, r0 + e, n0 + 32 * j + fr, acc[0][i][j][4 * q + e] * sc[e], acc[NMAT - 1][i][j][4 * q + e] * sc[e]);
+                for (int e = 0; e < 4; e++) {
+                    if (Q2 && sc[e] < 0.f) inf |= r0 + e < t.mend;
+                    else finish<NMAT>(a, t, r0 + e, n0 + 32 * j + fr, acc[0][i][j][4 * q + e] * sc[e], acc[NMAT - 1][i][j][4 * q + e] * sc[e]);
+                }
         }
+    if (Q2 && __any(inf)) {
+#pragma unroll 1
+        for (int j = 0; j < C; j++) inf_rows<NMAT, 32>(a, t, t.r16 * 16, 32 * R, n0 + 32 * j + fr, f);
+    }
 }
 
 template <int FMT, int NMAT, int MI>
@@ -1233,7 +1310,7 @@ bool rows_gemm_ok(int qt, int K) {
 
 size_t rows_split_bytes(int qt, int rows, int K) {
     const size_t mt = (rows + 15) / 16, nks = (size_t)(K + 127) / 128 * 4, ngw = (K + 511) / 512;
-    return up256(mt * nks * 2048) + up256(mt * 64) + (qt == RINA_QT_GGML_Q2_K ? mt * ngw * 3072 : 0);
+    return up256(mt * nks * 16 * kStep) + up256(mt * 64) + (qt == RINA_QT_GGML_Q2_K ? mt * ngw * 3072 : 0);
 }
 
 int rows_split(int qt, const float* x, const int* src, const int* used, int rows, int K, int pro, const float* nw, float eps, void* buf,
@@ -1244,7 +1321,7 @@ int rows_split(int qt, const float* x, const int* src, const int* used, int rows
     a.nks = (K + 127) / 128 * 4;
     a.ngw = (K + 511) / 512;
     a.xp = (uint4*)buf;
-    a.xs = (float*)((char*)buf + up256((size_t)mt * a.nks * 2048));
+    a.xs = (float*)((char*)buf + up256((size_t)mt * a.nks * 16 * kStep));
     a.xg = (uint16_t*)((char*)a.xs + up256((size_t)mt * 64));
     const dim3 grid(mt * 16 / kSplitRows), blk(256 * kSplitRows);
     const int nu = (K + 2047) / 2048;
