@@ -71,6 +71,17 @@ __device__ __forceinline__ uint32_t hi16_pair(uint32_t lo, uint32_t hi) { return
 constexpr int kParts = 3;              // bf16 parts of an activation
 constexpr int kStep = 64 * kParts;     // 16-byte units of a 16-row tile's 32-value step
 
+// LDS of one wave: its lanes' accesses before are done before those after (no
+// wait: a wave's LDS accesses run in order)
+__device__ __forceinline__ void wave_fence() {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+}
+// words of a buffer that is written and read at several widths
+typedef uint16_t __attribute__((may_alias)) u16_any;
+typedef uint32_t __attribute__((may_alias)) u32_any;
+
 __device__ __forceinline__ float silu_mul(float g, float u) { return g / (1.0f + expf(-g)) * u; }
 
 // ---------------------------------------------------------------------------
@@ -950,19 +961,19 @@ __global__ __launch_bounds__(512, 2) void rows32_kernel(RowsArgs a) {
 #pragma unroll
                 for (int i = 0; i < NCH; i++) {
                     const int back = co[i] + ss * (4 * BB) - clast;
-                    uint16_t* d = (uint16_t*)(wb + 64 * i + lane) - (back > 0 ? back / 2 : 0);   // (18-byte blocks: an even count)
+                    u16_any* d = (u16_any*)(wb + 64 * i + lane) - (back > 0 ? back / 2 : 0);   // (18-byte blocks: an even count)
                     const uint32_t v[4] = {ch[i].x, ch[i].y, ch[i].z, ch[i].w};
 #pragma unroll
                     for (int k = 0; k < 4; k++) { d[2 * k] = (uint16_t)v[k]; d[2 * k + 1] = (uint16_t)(v[k] >> 16); }
                 }
             }
-            __builtin_amdgcn_wave_barrier();
+            wave_fence();
 #pragma unroll
             for (int m = 0; m < NMAT; m++)
 #pragma unroll
                 for (int j = 0; j < C; j++) {
                     // a row that starts two bytes past a dword (Q4_0, odd n nb): its blocks shift by two
-                    const uint32_t* r = (const uint32_t*)wb + 20 * (32 * (m * C + j) + fr);
+                    const u32_any* r = (const u32_any*)wb + 20 * (32 * (m * C + j) + fr);
                     const int lead = FMT == FMT_Q4_0 ? 2 * ((col[j] & nb) & 1) : 0;
                     uint32_t d[2][5];
                     const bool odd = FMT == FMT_Q4_0 && ((lead + BB * f) & 2);
@@ -977,7 +988,7 @@ __global__ __launch_bounds__(512, 2) void rows32_kernel(RowsArgs a) {
                             if (4 * ss + b >= nb) ws[m][j].sc[b] = 0.f;
                     }
                 }
-            __builtin_amdgcn_wave_barrier();
+            wave_fence();
         } else {
 #pragma unroll
             for (int m = 0; m < NMAT; m++)
