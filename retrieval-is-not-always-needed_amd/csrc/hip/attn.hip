@@ -1142,8 +1142,8 @@ __global__ __launch_bounds__(256) void dq_prompt_kv_kernel(DqArgs a) {
 }
 
 // ---------------------------------------------------------------------------
-// Generic causal kernel: head widths other than 64 up to 256, and rows whose
-// alignment attn_rows does not take.  One wave per
+// Generic causal kernel: head widths other than 64 up to 256, and packed
+// caches at odd addresses.  One wave per
 // (query head, query row); keys in order with the online normalized update
 // of flash_fp32.cu:55-81, parallel over dims.
 // ---------------------------------------------------------------------------
@@ -1336,7 +1336,7 @@ extern "C" int rina_hip_gqa_attention(const float* q, const float* kcur, const f
         r.start_pos = start_pos; r.max_seq = max_seq; r.d_pos = d_pos;
         r.scale = 1.0f / sqrtf((float)dh);
         const int rc = attn_rows(ROWS_GQA, r, 64, 64, st);
-        if (rc != RINA_ERR_SHAPE) return rc;         // alignment it does not take: the generic kernel
+        if (rc != RINA_ERR_SHAPE) return rc;         // a cache alignment it does not take: the generic kernel
     }
     AttnArgs a{};
     a.q = q; a.kcur = kcur; a.vcur = vcur;

@@ -42,6 +42,12 @@ __device__ __forceinline__ T gld_a2(const uint8_t* p) {   // a load at 2-byte al
     return *(const __attribute__((address_space(1))) U*)p;
 }
 
+// four floats at 4-byte alignment (one load all the same)
+__device__ __forceinline__ f32x4 gld_f4(const float* p) {
+    typedef f32x4 __attribute__((aligned(4))) U;
+    return *(const __attribute__((address_space(1))) U*)p;
+}
+
 // 16 values (half h of a 32-value block) of a packed cache: code bytes and fp16 scale as loaded
 struct Half {
     u32x4 c;
@@ -124,10 +130,10 @@ __global__ __launch_bounds__(256 * NSET) void attn_rows_kernel(RowsAttnArgs a, i
     for (int dt = 0; dt < ND; dt++) o[dt] = f32x4{0.f, 0.f, 0.f, 0.f};
     {
         // (RINA-MLA rows are DQ wide here, zero past their own width)
-        const f32x4* qp = (const f32x4*)(a.q + ((int64_t)rowc * a.H + h) * DQ + DQ / 4 * g);
+        const float* qp = a.q + ((int64_t)rowc * a.H + h) * DQ + DQ / 4 * g;
 #pragma unroll
         for (int i = 0; i < Q4; i++) {
-            const f32x4 v = gld(qp + i);
+            const f32x4 v = gld_f4(qp + 4 * i);
             qv[4 * i] = v.x * qsc; qv[4 * i + 1] = v.y * qsc; qv[4 * i + 2] = v.z * qsc; qv[4 * i + 3] = v.w * qsc;
         }
     }
@@ -169,10 +175,10 @@ __global__ __launch_bounds__(256 * NSET) void attn_rows_kernel(RowsAttnArgs a, i
                 half_load(a.vf, a.cv + b * kvq::block_bytes(a.vf), sq & 1, vh);
             } else {
                 const int64_t off = ((int64_t)(cached ? j : j - pos0) * a.Hkv + kvh) * 64 + 16 * sq;
-                const f32x4* kp = (const f32x4*)((cached ? (const float*)a.ck : a.k) + off);
-                const f32x4* vp = (const f32x4*)((cached ? (const float*)a.cv : a.v) + off);
+                const float* kp = (cached ? (const float*)a.ck : a.k) + off;
+                const float* vp = (cached ? (const float*)a.cv : a.v) + off;
 #pragma unroll
-                for (int i = 0; i < 4; i++) { kr[i] = gld(kp + i); vr[i] = gld(vp + i); }
+                for (int i = 0; i < 4; i++) { kr[i] = gld_f4(kp + 4 * i); vr[i] = gld_f4(vp + 4 * i); }
             }
         } else if constexpr (SRC == ROWS_DQ) {
             const int64_t r = (int64_t)j * a.Hkv + kvh;
@@ -216,11 +222,11 @@ __global__ __launch_bounds__(256 * NSET) void attn_rows_kernel(RowsAttnArgs a, i
 #pragma unroll
             for (int i = 0; i < NK; i++) {
                 const int d = 4 * NK * sq + 4 * i;
-                kr[i] = gld((const f32x4*)((d < 128 ? kn : kp) + d));
+                kr[i] = gld_f4((d < 128 ? kn : kp) + d);
             }
-            const f32x4* vp = (const f32x4*)(a.v + ((int64_t)j * a.H + kvh) * 128 + 16 * sq);
+            const float* vp = a.v + ((int64_t)j * a.H + kvh) * 128 + 16 * sq;
 #pragma unroll
-            for (int i = 0; i < NV; i++) vr[i] = gld(vp + i);
+            for (int i = 0; i < NV; i++) vr[i] = gld_f4(vp + 4 * i);
         }
     };
     // (check: returns NaN if one of the thread's values is not finite)
@@ -505,9 +511,9 @@ int launch_dq(const RowsAttnArgs& a, int dq, hipStream_t st) {
 int attn_rows(RowsSrc src, RowsAttnArgs a, int dq, int dv, hipStream_t st) {
     auto al = [](const void* p, int n) { return (uintptr_t)p % n == 0; };
     if (src == ROWS_GQA) {
-        if (dq != 64 || dv != 64 || !al(a.q, 16) || !al(a.k, 16) || !al(a.v, 16)) return RINA_ERR_SHAPE;
+        if (dq != 64 || dv != 64) return RINA_ERR_SHAPE;
         const bool cache = a.d_pos || a.start_pos > 0, packed = a.mode != RINA_KV_FP32;
-        if (cache && (!al(a.ck, packed ? 2 : 16) || !al(a.cv, packed ? 2 : 16))) return RINA_ERR_SHAPE;
+        if (cache && (!al(a.ck, packed ? 2 : 4) || !al(a.cv, packed ? 2 : 4))) return RINA_ERR_SHAPE;
         if (packed) kvq::mode_formats_host(a.mode, a.kf, a.vf);
         return packed && cache ? launch<ROWS_GQA, true, 64, 64, 64, 2>(a, st) : launch<ROWS_GQA, false, 64, 64, 64, 2>(a, st);
     }
@@ -516,7 +522,6 @@ int attn_rows(RowsSrc src, RowsAttnArgs a, int dq, int dv, hipStream_t st) {
         a.vec = dq % 4 == 0 && al(a.ck, 16) && al(a.cv, 16);
         return a.mode == RINA_KV_FP32 ? launch_dq<false>(a, dq, st) : launch_dq<true>(a, dq, st);
     }
-    if (dq != 192 || dv != 128 || !al(a.q, 16) || !al(a.k, 16) || !al(a.v, 16) || !al(a.ck, 16) || a.da % 4 || a.db % 4)
-        return RINA_ERR_SHAPE;
+    if (dq != 192 || dv != 128) return RINA_ERR_SHAPE;
     return launch<ROWS_MLA, false, 192, 128, 32, 2>(a, st);
 }

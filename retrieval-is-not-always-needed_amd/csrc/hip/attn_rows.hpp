@@ -27,8 +27,8 @@ struct RowsAttnArgs {
 // width of the DQ rows (zeros past da + db)
 static inline int dq_rows_width(int dq) { return dq <= 64 ? 64 : dq <= 80 ? 80 : dq <= 96 ? 96 : 128; }
 
-// Launches the attention (RINA_ERR_SHAPE, before any launch: a shape or
-// alignment it does not take).  dq, dv: ROWS_GQA 64, 64; ROWS_DQ da + db <= 128, 64;
+// Launches the attention (RINA_ERR_SHAPE, before any launch: a shape or cache
+// alignment it does not take; rows need 4-byte alignment only).  dq, dv: ROWS_GQA 64, 64; ROWS_DQ da + db <= 128, 64;
 // ROWS_MLA 192, 128.
 int attn_rows(RowsSrc src, RowsAttnArgs a, int dq, int dv, hipStream_t st);
 

@@ -1502,8 +1502,7 @@ extern "C" int rina_hip_mla_prompt_attention(const float* q, const float* kva, c
         r.da = dc; r.db = dc + rope;
         r.out = out; r.T = T; r.H = H; r.Hkv = H; r.max_seq = max_seq;
         r.scale = 1.0f / sqrtf((float)D);
-        rc = attn_rows(ROWS_MLA, r, D, v_dim, st);
-        if (rc != RINA_ERR_SHAPE) return rc;         // alignment it does not take: the general form
+        return attn_rows(ROWS_MLA, r, D, v_dim, st);
     }
     hipLaunchKernelGGL(mla_expand_kernel, dim3(T, H), dim3(256), 0, st, a, k_nope, v_rows, k_full, v_full);
     RINA_LAUNCH_CHECK();

@@ -146,3 +146,29 @@ def test_mla_rows_before_a_non_finite_row(rina, orc, T, bad):
         return host(out).reshape(T, -1)
 
     earlier_rows(call, T, bad, 5)
+
+
+@pytest.mark.parametrize("mode,P,T,H,Hkv", [(0, 0, 70, 8, 4), (0, 33, 20, 8, 2), (1, 0, 70, 32, 8), (1, 80, 5, 4, 4)])
+@pytest.mark.parametrize("off", [1, 2, 3])
+def test_rows_at_4_byte_alignment(rina, orc, mode, P, T, H, Hkv, off):
+    """Query, key, value and output rows (and an fp32 cache) that start `off`
+    floats past a 16-byte boundary: the same bits as aligned ones."""
+    hip, kvd, max_seq = rina.load_hip(), Hkv * 64, P + T
+    r = rng(P + T + mode)
+    rows = [r.standard_normal(n * w).astype(np.float32) for n, w in ((T, H * 64), (T, kvd), (T, kvd))]
+    kv = [r.standard_normal((max_seq, kvd)).astype(np.float32) for _ in range(2)]
+    if mode:
+        cache = [dev(orc.kv_quantize(f, x)) for f, x in zip(orc.kv_mode_formats(mode), kv)]
+
+    def at(x, o):
+        return dev(np.concatenate([np.zeros(o, np.float32), x.reshape(-1)])).data_ptr() + 4 * o
+
+    def call(o):
+        q, k, v = (at(x, o) for x in rows)
+        ck, cv = (c.data_ptr() for c in cache) if mode else (at(x, o) for x in kv)
+        out = empty(o + T * H * 64)
+        ok(hip.rina_hip_gqa_attention(q, k, v, ck, cv, mode, 0, None, None, T, H, Hkv, 64, P, None, max_seq,
+                                      out.data_ptr() + 4 * o, None, 0, stream()), "attention")
+        return host(out)[o:]
+
+    assert np.array_equal(call(off), call(0))
