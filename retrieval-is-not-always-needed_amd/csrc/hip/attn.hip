@@ -997,10 +997,10 @@ __global__ __launch_bounds__(256) void dq_split_kernel(DqArgs a, SplitArgs p) {
 // [xa | HF-RoPE(xb)], w wide (zeros past da + db), into k [T][Hkv][w] or
 // q [T][H][w], so that no workgroup of the attention rotates it again.  One
 // launch for both: a call of a few rows is bound by its dependent launches
-// (two rows 12.7 -> 11.1 us,
-// 1900 rows of the q2k_q1v cache 112 -> 107 us against a launch of its own).  attn_rows (ROWS_DQ) then reads, for row t, the positions before it
-// from the cache and its own position from its fp32 rows, as the decode step
-// of that row would.
+// (1900 rows of the q2k_q1v cache 112 -> 107 us against a launch of its own).
+// attn_rows (ROWS_DQ) then reads, for row t, the positions before it from the
+// cache and its own position from its fp32 rows, as the decode step of that row
+// would.
 template <int QKV>
 __global__ __launch_bounds__(64) void dq_pack_rows_kernel(DqArgs a, float* q, float* k, int w) {
     const int lane = threadIdx.x, t = blockIdx.x, kvh = blockIdx.y;
@@ -1038,13 +1038,22 @@ __global__ __launch_bounds__(64) void dq_pack_rows_kernel(DqArgs a, float* q, fl
     }
 }
 
-// The attention of rows over at most kDqShort positions, grid (T, H), four
-// waves per (row, query head): bound by its one chain of loads, where the
-// tiles of attn_rows pay two staged blocks and their barriers.  10 / 5 heads:
-// 2 rows from 0 7.7 us against 11.1 with attn_rows, 24 rows from 0 7.7 against
-// 11.5, 3 rows after 40 8.6 against 11.2; one position at a time, it is behind
-// further on (100 rows after 300 48 against 35).
-constexpr int kDqShort = 64;
+// The attention of a few rows over short caches, grid (T, H), four waves per
+// (row, query head): bound by its one chain of loads (0.04 us a position in
+// fp32, 0.05 packed, one position at a time), where the tiles of attn_rows pay
+// two staged key blocks, their barriers and, past 128 positions, the launch
+// that merges the key splits.
+// The line between them (10 / 5 heads, 64 + 32, us per-row / tiles, fp32 and
+// packed): 2 rows after 200 13.0 / 16.3 and 16.7 / 18.5, after 300 17.5 / 16.9
+// and 21.3 / 19.0; 24 rows after 200 13.7 / 17.7 and 17.2 / 20.1, after 300
+// 18.4 / 18.2 and 23.2 / 20.6; 64 rows after 60 13.2 / 15.6 and 16.7 / 17.7,
+// after 150 19.4 / 18.2 and 24.7 / 20.8; 100 rows from 0 12.6 / 15.8 and 16.0 /
+// 17.4, after 100 20.7 / 19.0 and 26.3 / 22.3; 160 rows from 0 20.9 / 19.9 and
+// 27.7 / 21.5.
+bool dq_per_row(int T, int H, int positions) {
+    const int64_t cus = rina_num_cus();
+    return positions <= 256 && positions * ((int64_t)T * H + 2 * cus) <= 768 * cus;
+}
 
 template <int QKV>
 __global__ __launch_bounds__(256) void dq_prompt_kv_kernel(DqArgs a) {
@@ -1142,8 +1151,8 @@ __global__ __launch_bounds__(256) void dq_prompt_kv_kernel(DqArgs a) {
 }
 
 // ---------------------------------------------------------------------------
-// Generic causal kernel: head widths other than 64 up to 256, and packed
-// caches at odd addresses.  One wave per
+// Generic causal kernel: head widths other than 64 up to 256, prompts of a few
+// rows, packed caches at odd addresses.  One wave per
 // (query head, query row); keys in order with the online normalized update
 // of flash_fp32.cu:55-81, parallel over dims.
 // ---------------------------------------------------------------------------
@@ -1300,6 +1309,12 @@ extern "C" size_t rina_hip_gqa_attention_workspace(int T, int H, int dh, int max
     return split_ws_bytes(H, (max_pos + cs - 1) / cs);
 }
 
+// Prompts of up to kGqaShort rows from position 0 take one wave per (row, head),
+// done before a tile of attn_rows has staged its keys: 32 / 8 heads, 2 rows 2.8
+// us against 8.5, 12 rows 6.4 against 7.6, 16 rows 7.8 against 7.9 (8 / 8 heads
+// 7.6 against 7.3).
+constexpr int kGqaShort = 12;
+
 extern "C" int rina_hip_gqa_attention(const float* q, const float* kcur, const float* vcur, const void* cache_k,
                                       const void* cache_v, int mode, int pre_rope, const float* rkc, const float* rks,
                                       int T, int H, int Hkv, int dh, int start_pos, const int* d_pos, int max_seq,
@@ -1327,7 +1342,7 @@ extern "C" int rina_hip_gqa_attention(const float* q, const float* kcur, const f
         sa.scale = 1.0f / sqrtf((float)dh);
         return launch_split_mode<false>(sa, rep, ws_bytes, workspace, st);
     }
-    if (dh == 64) {
+    if (dh == 64 && (T == 1 || need_cache || T > kGqaShort)) {
         RowsAttnArgs r{};
         r.q = q; r.k = kcur; r.v = vcur;
         r.ck = (const uint8_t*)cache_k; r.cv = (const uint8_t*)cache_v;
@@ -1580,7 +1595,7 @@ extern "C" int rina_hip_dq_prompt_attention_kv(const float* qa, const float* qb,
     a.H = H; a.Hkv = Hkv; a.da = da; a.db = db; a.dv = dv; a.start_pos = start_pos; a.max_seq = max_seq;
     a.scale = 1.0f / sqrtf((float)(da + db));
     hipStream_t st = as_stream(stream);
-    if (start_pos + T <= kDqShort) {
+    if (dq_per_row(T, H, start_pos + T)) {
         a.out = out;
         float* none = nullptr;
         if (packed) {

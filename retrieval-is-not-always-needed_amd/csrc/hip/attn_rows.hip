@@ -465,19 +465,39 @@ __global__ __launch_bounds__(256) void rows_combine_kernel(RowsAttnArgs a) {
     for (int i = 0; i < DV / 64; i++) gst(a.out + r * DV + 64 * i + lane, o[i] / lt);
 }
 
+// Key splits of a launch: the count with the least estimated time.  wg
+// workgroups, one per CU at a time (their registers), the longest first; nblk
+// key blocks for the last row tile, avg for the one in the middle (causal); tb
+// us per block and set.  A round takes as long as its longest workgroup where
+// all are alike and as their average where they differ; a split adds the second
+// launch (3 us) and its partials (part bytes each, written and read at 4 TB/s).
+// us before (two workgroups per CU, two blocks per set at least) / after, 32 / 8
+// heads, q8: 2 rows after 400 27.8 / 15.7, 64 rows after 1536 25.9 / 23.1, 128
+// rows after 1536 45.2 / 31.7, 512 rows from 0 29.0 / 25.9, after 1536 99.7 /
+// 95.9; 300 rows after 1536 70 either way (three splits).
+int key_splits(int wg, int nblk, double avg, int nset, double tb, double part) {
+    const double tf = 3.5, cus = rina_num_cus();
+    int best = 1;
+    double least = 1e30;
+    for (int ks = 1; ks <= 16 && (ks == 1 || ks * nset < nblk + nset); ks++) {
+        const double r = wg * (double)ks / cus, up = ceil(r);
+        const double longest = tb * (((nblk + ks - 1) / ks + nset - 1) / nset) + tf;
+        const double mean = fmin(longest, tb * fmax(1.0, avg / (ks * nset) + 0.25) + tf);
+        const double t = fmax(longest, mean * (r + (up - r) * mean / longest)) + (ks > 1 ? 3.0 + 2.0 * ks * part / 4e6 : 0.0);
+        if (t < least) { least = t; best = ks; }
+    }
+    return best;
+}
+
 template <int SRC, bool PK, int DQ, int DV, int KB, int NSET>
 int launch(RowsAttnArgs a, hipStream_t st) {
     const int rep = a.H / a.Hkv, hpw = rep % 4 == 0 ? 4 : rep % 2 == 0 ? 2 : 1;
     const int rw = 16 * (4 / hpw), ntile = (a.T + rw - 1) / rw, groups = a.H / hpw;
-    // split the keys until there are about two workgroups per CU, two blocks
-    // per set at least (the partials of a split cost a write and a read of
-    // the output)
     const int max_pos = a.d_pos ? a.max_seq : a.start_pos + a.T;
     const int nblk = (max_pos + KB - 1) / KB;
-    int ks = (2 * rina_num_cus() + groups * ntile / 2) / (groups * ntile);
-    if (ks > nblk / (2 * NSET)) ks = nblk / (2 * NSET);
-    if (ks > 16) ks = 16;
-    if (ks < 1) ks = 1;
+    const double avg = a.d_pos ? nblk : (a.start_pos + 0.5 * (a.T + rw)) / KB;
+    const int ks = key_splits(groups * ntile, nblk, avg, NSET, 5.6 * KB * (DQ + DV) / (64 * 128.0),
+                              (double)a.T * a.H * (DV + 2) * sizeof(float));
     a.ks_n = ks;
     const size_t n = ks > 1 ? (size_t)ks * a.T * a.H : 0;
     RinaScratch scratch;
