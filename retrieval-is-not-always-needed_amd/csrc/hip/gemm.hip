@@ -682,7 +682,7 @@ struct WStep32 {
 template <int FMT, int NMAT, int MI>
 struct Batch16 { static constexpr int BT = FMT == FMT_Q2_S ? 1 : NMAT * MI >= 4 ? 2 : 4; };
 
-// ---- M <= 32: v_mfma_f32_16x16x32_f16 tiles ----
+// ---- 16- and 32-row tiles: v_mfma_f32_16x16x32_bf16 ----
 // MI 16-row tiles (all the rows of a group), 16 columns (per matrix) per wave.
 template <int FMT, int NMAT, int MI>
 __global__ __launch_bounds__(512, 2) void rows16_kernel(RowsArgs a) {
@@ -735,7 +735,9 @@ __global__ __launch_bounds__(512, 2) void rows16_kernel(RowsArgs a) {
         const int bn = b + a.KW < nb ? b + a.KW : b;   // the last batch loads itself again
 #pragma unroll
         for (int s = 0; s < BT; s++) {
-            f32x4 d[NMAT][MI];
+            // (a page's sum: the largest parts and the others apart, or every
+            // small product rounds the whole sum)
+            f32x4 d[NMAT][MI], ds[NMAT][MI];
 #pragma unroll
             for (int half = 0; half < 2; half++) {
                 bf16x8 at[MI][2 * kParts];
@@ -757,14 +759,18 @@ __global__ __launch_bounds__(512, 2) void rows16_kernel(RowsArgs a) {
                         for (int p = kParts - 1; p >= 0; p--)
 #pragma unroll
                             for (int i = 0; i < MI; i++) {
-                                if (p == kParts - 1 && (!PAGE || st == 0)) d[m][i] = f32x4{0.f, 0.f, 0.f, 0.f};
-                                d[m][i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(at[i][kParts * (st & 1) + p], w, d[m][i], 0, 0, 0);
+                                f32x4& t = PAGE && p > 0 ? ds[m][i] : d[m][i];
+                                if (PAGE ? st == 0 && p != 1 : p == kParts - 1) t = f32x4{0.f, 0.f, 0.f, 0.f};
+                                t = __builtin_amdgcn_mfma_f32_16x16x32_bf16(at[i][kParts * (st & 1) + p], w, t, 0, 0, 0);
                             }
                         if (!PAGE || st == 3) {
 #pragma unroll
                             for (int i = 0; i < MI; i++)
 #pragma unroll
-                                for (int e = 0; e < 4; e++) acc[m][i][e] = fmaf(ws[s][m].sc[PAGE ? 0 : st], d[m][i][e], acc[m][i][e]);
+                                for (int e = 0; e < 4; e++) {
+                                    const float v = PAGE ? d[m][i][e] + ds[m][i][e] : d[m][i][e];
+                                    acc[m][i][e] = fmaf(ws[s][m].sc[PAGE ? 0 : st], v, acc[m][i][e]);
+                                }
                         }
                     }
                 }
@@ -833,7 +839,7 @@ __global__ __launch_bounds__(512, 2) void rows16_kernel(RowsArgs a) {
     if (Q2 && __any(inf)) inf_rows<NMAT, 16>(a, t, t.r16 * 16, 16 * MI, c0, f);
 }
 
-// ---- M > 32: v_mfma_f32_32x32x16_f16 tiles ----
+// ---- 64-row tiles: v_mfma_f32_32x32x16_bf16 ----
 // A wave owns 32 R rows x 32 C columns (per matrix) of its K slice.  Q4 weights
 // pass through a buffer of the wave's own in LDS: the 80 (72) bytes of a
 // column's 128-value step are loaded as five 16-byte chunks by neighbouring
@@ -1364,8 +1370,18 @@ int rows_gemm(const rina_linear_seg* segs, int nseg, int qt, const RowsX& x, int
     a.plan = pl ? pl->plan : nullptr;
     a.stride = pl ? pl->stride : 0;
     const int nss = a.nks / 4;
-    // row tiles of 16, 32 or 64 rows (rt 0, 1, 2); columns per wave: 16, or 32 ct at 64 rows
-    const int rt = pl ? pl->rt : x.rows <= 16 ? 0 : x.rows <= 32 ? 1 : 2;
+    // row tiles of 16, 32 or 64 rows (rt 0, 1, 2); columns per wave: 16, or 32 ct
+    // at 64 rows.  More than 32 rows take the 64-row tiles where these give every
+    // SIMD a wave with K split as far as it goes (us 64-row / 32-row, Q4_0F): N
+    // 2048, K 8192: 64 rows (512 waves) 58.0 / 38.8, 96 rows (1024) 58.7 / 59.2,
+    // 160 rows 62 / 70; N 512, K 1024: 256 rows (256 waves) 15.9 / 11.7; N 8192 x 2,
+    // K 2048: 33 rows (2048 waves) 29.3 / 30.4, 256 rows 70.7 / 88.9.
+    const int64_t simds = 4LL * rina_num_cus();
+    int64_t w64 = 0;
+    for (int s = 0; s < nseg; s++) w64 += (segs[s].N + 31) / 32;
+    w64 *= (x.rows + 63) / 64;
+    for (int kw = 1; kw < 8 && nss >= 2 * kw; kw *= 2) w64 *= 2;
+    const int rt = pl ? pl->rt : x.rows <= 16 ? 0 : x.rows <= 32 || w64 < simds ? 1 : 2;
     const int tr = 16 << rt, tc = rt < 2 ? 16 : 32;
     const int64_t mts = pl ? pl->tiles_est : (x.rows + tr - 1) / tr;
     auto tiles = [&](int ct) {
@@ -1373,10 +1389,11 @@ int rows_gemm(const rina_linear_seg* segs, int nseg, int qt, const RowsX& x, int
         for (int s = 0; s < nseg; s++) t += (segs[s].N + tc * ct - 1) / (tc * ct);
         return t * mts;
     };
-    // K slices until there are two waves per SIMD; 64 columns per wave only
-    // where that leaves every SIMD a wave without splitting K
-    const int64_t simds = 4LL * rina_num_cus();
+    // 64 columns per wave only where that leaves every SIMD a wave without
+    // splitting K
     const int nj = nmat == 1 && rt == 2 && tiles(2) >= simds ? 2 : 1;
+    // K slices until there are two waves per SIMD: each slice is also a shorter
+    // chain of sums
     int kw = 1;
     while (kw < 8 && tiles(nj) * kw < 2 * simds && nss >= 2 * kw) kw *= 2;
     a.KW = kw;

@@ -1401,7 +1401,7 @@ extern "C" int rina_hip_linear_fused_ex(const rina_linear_seg* segs, int nseg, i
     }
     hipStream_t st = as_stream(stream);
     RinaScratch scratch;
-    if (M > 1 && rows_gemm_ok(qt, K)) {
+    if (M > 1 && rows_gemm_ok(qt, K) && !rows_bf3_ok(segs, nseg, qt, input, M, K, epi)) {
         // several rows: split once (with the prologue), then 3 segments per launch
         void* buf = scratch.get(rows_split_bytes(qt, M, K), st, kScratchRows);
         if (!buf) return RINA_ERR_HIP;
@@ -1442,6 +1442,7 @@ extern "C" int rina_hip_linear_fused_ex(const rina_linear_seg* segs, int nseg, i
         return RINA_OK;
     }
     if (M > 1) {
+        if (rows_bf3_ok(segs, nseg, qt, input, M, K, epi)) return rows_bf3(segs, nseg, qt, input, M, K, epi, st);
         if (qt == RINA_QT_FP32 && rows_f32_ok(segs, nseg, input, K)) return rows_f32(segs, nseg, input, M, K, epi, st);
         for (int s = 0; s < nseg; s++) {
             int rc = gemm_tiled(segs[s], qt, input, M, K, epi, st);

@@ -35,6 +35,11 @@ struct RowsPlan {
 // up to 3 segments of one quant type (grouped: 1)
 int rows_gemm(const rina_linear_seg* segs, int nseg, int qt, const RowsX& x, int epi, const RowsPlan* pl, hipStream_t st);
 
+// Q4 weights in one launch (gemm_bf3.hip): M >= 16 rows at 16-byte alignment,
+// where that is the faster of the two; up to 3 segments, no prologue
+bool rows_bf3_ok(const rina_linear_seg* segs, int nseg, int qt, const float* x, int M, int K, int epi);
+int rows_bf3(const rina_linear_seg* segs, int nseg, int qt, const float* x, int M, int K, int epi, hipStream_t st);
+
 // fp32 weights: rows and weights 16-byte aligned, K % 4 == 0; M >= 2, up to 3 segments
 bool rows_f32_ok(const rina_linear_seg* segs, int nseg, const float* x, int K);
 int rows_f32(const rina_linear_seg* segs, int nseg, const float* x, int M, int K, int epi, hipStream_t st);

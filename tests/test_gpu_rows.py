@@ -1,4 +1,4 @@
-"""Products over several activation rows (gemm.hip) against float64 products
+"""Products over several activation rows (gemm.hip, gemm_bf3.hip) against float64 products
 of the dequantized weights, at the edges of their tiles: 16 / 32 / 64-row
 tiles and one row past each, K of one block up to steps and windows with
 remainders, column counts off the tile, unaligned rows, rows of very
@@ -39,10 +39,14 @@ def product(rina, w, qt, x, N, K, epi=0, w2=None, y0=None, off=0):
 
 @pytest.mark.parametrize("qt", [5, 7, 10, 6])
 @pytest.mark.parametrize("M,N,K", [(2, 16, 32), (15, 33, 96), (16, 40, 128), (17, 100, 160), (31, 17, 512), (32, 130, 544),
-                                   (33, 64, 1024), (64, 65, 640), (65, 31, 2080), (80, 300, 256), (200, 96, 1408)])
+                                   (33, 64, 1024), (64, 65, 640), (65, 31, 2080), (80, 300, 256), (200, 96, 1408),
+                                   (15, 200, 320), (16, 200, 320), (97, 130, 512), (97, 130, 544), (129, 8000, 640),
+                                   (120, 8000, 640), (130, 1100, 8192)])
 def test_rows_product_edges(rina, orc, qt, M, N, K):
     """Every row tile and its successor, K of 1 .. 65 blocks (whole and partial
-    128-value steps, Q2_K rows that start inside pages), odd column counts."""
+    128-value steps, Q2_K rows that start inside pages), odd column counts; for
+    Q4 weights both sides of the lines between one launch and two (16 rows, K
+    512, outputs against K squared) and between 32- and 64-row tiles."""
     r = rng(M * 3 + N + K + qt)
     w, W = weights(orc, qt, r, N * K)
     x = r.standard_normal((M, K)).astype(np.float32)
@@ -67,12 +71,13 @@ def test_rows_product_unaligned_and_epilogues(rina, orc, qt, M, off):
 
 
 @pytest.mark.parametrize("qt", [5, 7, 10])
-def test_rows_product_magnitudes(rina, orc, qt):
+@pytest.mark.parametrize("K", [512, 640])
+def test_rows_product_magnitudes(rina, orc, qt, K):
     """Every row is held to its own scale: rows of 1e-30 .. 1e30 (one of
-    zeros), and rows whose values span 2^40: the sums of 512 exact products
-    stay within 1e-6 of sum |w x| (chains of at most 16 blocks of 32)."""
+    zeros), and rows whose values span 2^40: the sums of exact products stay
+    within 1e-6 of sum |w x| (chains of at most 20 blocks of 32)."""
     r = rng(qt)
-    M, N, K = 24, 48, 512
+    M, N = 24, 48
     w, W = weights(orc, qt, r, N * K)
     x = r.standard_normal((M, K))
     x[:12] *= (10.0 ** np.linspace(-30, 30, 12))[:, None]
@@ -87,13 +92,13 @@ def test_rows_product_magnitudes(rina, orc, qt):
 
 
 @pytest.mark.parametrize("qt", [5, 7, 10])
-@pytest.mark.parametrize("M", [5, 24, 70])
-def test_rows_product_outlier_facing_zero_weights(rina, orc, qt, M):
+@pytest.mark.parametrize("M,K", [(5, 480), (24, 480), (24, 672), (70, 672)])
+def test_rows_product_outlier_facing_zero_weights(rina, orc, qt, M, K):
     """A value 2^12 .. 2^60 times the others whose weights are zero adds
-    nothing: the product of the others is as close as without it.  fp32 sums of
-    480 terms in chains of at most 16 blocks: below 1e-6 of sum |w x|."""
+    nothing: the product of the others is as close as without it.  fp32 sums in
+    chains of at most 21 blocks of 32: below 1e-6 of sum |w x|."""
     r = rng(qt + M)
-    N, K, at = 48, 480, 37
+    N, at = 48, 37
     w, _ = weights(orc, qt, r, N * K)
     if qt == 10:                             # scale and minimum of the group of 16 that holds it
         g = (np.arange(N) * K + at) // 16
@@ -115,7 +120,7 @@ def test_rows_product_outlier_facing_zero_weights(rina, orc, qt, M):
 
 
 @pytest.mark.parametrize("qt", [5, 7, 10])
-@pytest.mark.parametrize("M,K", [(20, 256), (20, 416), (70, 256), (70, 416)])
+@pytest.mark.parametrize("M,K", [(20, 256), (20, 416), (70, 256), (70, 416), (20, 640), (70, 672), (300, 640)])
 def test_rows_product_nonfinite(rina, orc, qt, M, K):
     """inf and NaN stay in their rows, and rows that hold them give what the
     fp32 products give: an infinity of the weight's sign, NaN where the weight
@@ -390,3 +395,24 @@ def test_rows_product_two_threads_one_stream(rina, orc, qt, M):
         assert rcs[i] == [0] * 300
         assert all(torch.equal(y, ys[i][0]) for y in ys[i])
     assert not torch.equal(ys[0][0], ys[1][0])
+
+
+@pytest.mark.parametrize("qt", [7, 10, 6])
+@pytest.mark.parametrize("M,K,pro", [(2, 2176, 1), (20, 4160, 2), (33, 8320, 1), (3, 12416, 1), (18, 12416, 2), (40, 256, 1)])
+def test_rows_product_norm_prologue(rina, orc, qt, M, K, pro):
+    """RMSNorm / LayerNorm fused into the split of rows of every register
+    count, and of rows longer than the registers hold (past 12288)."""
+    r = rng(M + K + qt)
+    N = 40
+    w, W = weights(orc, qt, r, N * K)
+    x = (r.standard_normal((M, K)) + (0.5 if pro == 2 else 0.0)).astype(np.float32)
+    nw = r.uniform(0.8, 1.2, K).astype(np.float32)
+    y = empty(M * N)
+    seg = rina.LinearSeg(dev(w).data_ptr(), None, y.data_ptr(), N)
+    ok(rina.load_hip().rina_hip_linear_fused(C.byref(seg), 1, qt, dev(x).data_ptr(), M, K, 0, pro, dev(nw).data_ptr(),
+                                             np.float32(1e-5), stream()), "product")
+    a = x.astype(np.float64)
+    if pro == 2:
+        a = a - a.mean(1, keepdims=True)
+    a = a / np.sqrt((a ** 2).mean(1, keepdims=True) + 1e-5) * nw
+    assert_close(host(y).reshape(M, N), a @ W.reshape(N, K).T, what="norm + rows")
