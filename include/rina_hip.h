@@ -335,7 +335,9 @@ int rina_hip_moe_ffn(const float* x, const void* gate_exps, const void* up_exps,
  * and ffn multiples of 32, else one expert after the other (the selection is
  * then read back to the host once: the call synchronizes the stream).  gate_sh / up_sh / down_sh may
  * be NULL with S == 0.  Any quant type rina_hip_linear_fused takes; the
- * workspace (16-byte aligned) holds rina_hip_moe_rows_workspace() bytes. */
+ * workspace (16-byte aligned) holds rina_hip_moe_rows_workspace() bytes.
+ * gate_exps / up_exps / down_exps and, with more than one expert, the strides
+ * are multiples of 4 (else RINA_ERR_ARG). */
 size_t rina_hip_moe_rows_workspace(int T, int d, int n_experts, int k, int ffn, int shared_ffn);
 int rina_hip_moe_rows(float* h, int T, const float* ln2, float eps, const void* gate_inp, int qt_inp,
                       const void* gate_sh, const void* up_sh, const void* down_sh, int shared_ffn, int qt_sh,

@@ -1542,38 +1542,60 @@ size_t up4f(size_t n) { return (n + 3) / 4 * 4; }
 }
 
 namespace {
+// Buffers of moe_grouped: sizes in bytes, each a multiple of 256
+struct GroupedMem {
+    size_t slots, tmax;
+    int rt;
+    size_t x, g, gx, plan, src, slot_of;
+    size_t total() const { return x + g + gx + plan + src + slot_of; }
+};
+GroupedMem grouped_mem(int qt, int T, int E, int k, int d, int F) {
+    GroupedMem m;
+    const size_t tk = (size_t)T * k, groups = std::min((size_t)E, tk);
+    m.slots = (tk + 15 * groups + 15) / 16 * 16;                 // every group padded to 16-row tiles
+    const size_t per = (tk + groups - 1) / groups;               // rows of an average expert
+    m.rt = per <= 16 ? 0 : per <= 32 ? 1 : 2;
+    m.tmax = tk / (16 << m.rt) + groups;
+    auto up = [](size_t n) { return (n + 255) & ~(size_t)255; };
+    m.x = up(std::max(rows_split_bytes(qt, (int)m.slots, d), m.slots * d * 4));   // split rows, later Y
+    m.g = up(m.slots * F * 4);
+    m.gx = up(rows_split_bytes(qt, (int)m.slots, F));
+    m.plan = up((2 + 3 * m.tmax) * 4);
+    m.src = up(m.slots * 4);
+    m.slot_of = up(tk * 4);
+    return m;
+}
+
 // The routed experts of a prompt's rows without leaving the device: the rows
 // grouped by expert (moe_plan_kernel), split once in that order, one grouped
 // product for every expert's gate/up (SiLU * up), its result split, one for
 // every down, and the weighted rows added to h.  Six launches instead of four
 // or more per expert and a host round trip: 512 rows, 64 experts top 6,
-// 2048 x 1408 Q2_K: the block 3.30 ms that way, 450 us grouped.
+// 2048 x 1408 Q2_K: the block 3.30 ms that way, 0.68 ms grouped.  Row tiles of
+// 64 rows where an expert has more than 32 on average: 48 rows 492 us against
+// 567 with 32-row tiles, 28 rows 373 / 370.
+// ws: the caller's buffer where it is large enough, else library scratch.
 int moe_grouped(float* h, const float* a2, const int* ids, const float* probs, const void* wg, const void* wu, const void* wd,
-                int qt, int64_t stride_gu, int64_t stride_dn, int T, int E, int k, int d, int F, hipStream_t st) {
-    const size_t tk = (size_t)T * k, groups = std::min((size_t)E, tk);
-    const size_t slots = (tk + 15 * groups + 15) / 16 * 16;      // every group padded to 16-row tiles
-    const size_t per = (tk + groups - 1) / groups;               // rows of an average expert
-    const int rt = per <= 16 ? 0 : per <= 32 ? 1 : 2;
-    const size_t tmax = tk / (16 << rt) + groups;
-    auto up = [](size_t n) { return (n + 255) & ~(size_t)255; };
-    const size_t b_x = up(std::max(rows_split_bytes(qt, (int)slots, d), slots * d * 4));   // split rows, later Y
-    const size_t b_g = up(slots * F * 4), b_gx = up(rows_split_bytes(qt, (int)slots, F));
-    const size_t b_p = up((2 + 3 * tmax) * 4), b_s = up(slots * 4), b_o = up(tk * 4);
+                int qt, int64_t stride_gu, int64_t stride_dn, int T, int E, int k, int d, int F, char* ws, size_t ws_bytes,
+                hipStream_t st) {
+    const GroupedMem m = grouped_mem(qt, T, E, k, d, F);
+    const size_t tk = (size_t)T * k, groups = std::min((size_t)E, tk), slots = m.slots;
     RinaScratch scratch;
-    char* p = (char*)scratch.get(b_x + b_g + b_gx + b_p + b_s + b_o, st, kScratchMoe);
+    char* p = (char*)(((uintptr_t)ws + 255) & ~(uintptr_t)255);
+    if (p + m.total() > ws + ws_bytes) p = (char*)scratch.get(m.total(), st, kScratchMoe);
     if (!p) return RINA_ERR_HIP;
     void* xb = p;
-    float* G = (float*)(p + b_x);
-    void* gb = p + b_x + b_g;
-    int* plan = (int*)((char*)gb + b_gx);
-    int* src = (int*)((char*)plan + b_p);
-    int* slot_of = (int*)((char*)src + b_s);
-    hipLaunchKernelGGL(moe_plan_kernel, dim3(1), dim3(1024), 0, st, ids, (int)tk, k, E, rt, plan, src, slot_of);
+    float* G = (float*)(p + m.x);
+    void* gb = p + m.x + m.g;
+    int* plan = (int*)((char*)gb + m.gx);
+    int* src = (int*)((char*)plan + m.plan);
+    int* slot_of = (int*)((char*)src + m.src);
+    hipLaunchKernelGGL(moe_plan_kernel, dim3(1), dim3(1024), 0, st, ids, (int)tk, k, E, m.rt, plan, src, slot_of);
     RINA_LAUNCH_CHECK();
     RowsX x;
     int rc = rows_split(qt, a2, src, plan + 1, (int)slots, d, RINA_PRO_NONE, nullptr, 0.f, xb, &x, st);
     if (rc) return rc;
-    RowsPlan pl{plan, stride_gu, rt, (int)tmax, (int)std::max(groups, tk / (16 << rt))};
+    RowsPlan pl{plan, stride_gu, m.rt, (int)m.tmax, (int)std::max(groups, tk / (16 << m.rt))};
     rina_linear_seg sg{wg, wu, G, F};
     if ((rc = rows_gemm(&sg, 1, qt, x, RINA_EPI_SWIGLU, &pl, st))) return rc;
     if ((rc = rows_split(qt, G, nullptr, plan + 1, (int)slots, F, RINA_PRO_NONE, nullptr, 0.f, gb, &x, st))) return rc;
@@ -1587,12 +1609,25 @@ int moe_grouped(float* h, const float* a2, const int* ids, const float* probs, c
 }
 }  // namespace
 
+// a2 | logits | probs | ids | G_shared, then the routed experts' part: X | G | Y
+// | idx | pr for one expert after the other, or the buffers of moe_grouped
+static size_t moe_rows_head(int T, int d, int E, int k, int S) {
+    const size_t t = (size_t)T;
+    return sizeof(float) * (up4f(t * d) + up4f(t * E) + 2 * up4f(t * k) + up4f(t * S));
+}
+// (what a call needs; with less than rina_hip_moe_rows_workspace the grouped
+// experts take library scratch)
+static size_t moe_rows_least(int T, int d, int E, int k, int F, int S) {
+    const size_t tk = (size_t)T * k;
+    return moe_rows_head(T, d, E, k, S) + sizeof(float) * (up4f(tk * d) + up4f(tk * F) + up4f(tk * d) + 2 * up4f(tk));
+}
+
 extern "C" size_t rina_hip_moe_rows_workspace(int T, int d, int E, int k, int F, int S) {
     if (T < 1 || d < 1 || E < 1 || k < 1 || F < 1 || S < 0) return 0;
-    const size_t t = (size_t)T, tk = t * k;
-    // a2 | logits | probs | ids | G_shared | X | G | Y | idx | pr
-    return sizeof(float) * (up4f(t * d) + up4f(t * E) + 2 * up4f(tk) + up4f(t * S) + up4f(tk * d) + up4f(tk * F) +
-                            up4f(tk * d) + 2 * up4f(tk));
+    const size_t least = moe_rows_least(T, d, E, k, F, S);
+    if (!rows_gemm_ok(RINA_QT_GGML_Q2_K, d) || !rows_gemm_ok(RINA_QT_GGML_Q2_K, F)) return least;
+    // Q2_K: the largest of the formats
+    return std::max(least, moe_rows_head(T, d, E, k, S) + 256 + grouped_mem(RINA_QT_GGML_Q2_K, T, E, k, d, F).total());
 }
 
 extern "C" int rina_hip_moe_rows(float* h, int T, const float* ln2, float eps, const void* gate_inp, int qt_inp,
@@ -1607,8 +1642,7 @@ extern "C" int rina_hip_moe_rows(float* h, int T, const float* ln2, float eps, c
     if (((uintptr_t)gate_exps | (uintptr_t)up_exps | (uintptr_t)down_exps) % 4 ||
         (E > 1 && (stride_gu % 4 || stride_dn % 4)))
         return RINA_ERR_ARG;
-    const size_t need = rina_hip_moe_rows_workspace(T, d, E, k, F, S);
-    if (!workspace || ws_bytes < need || (uintptr_t)workspace % 16) return RINA_ERR_WORKSPACE;
+    if (!workspace || ws_bytes < moe_rows_least(T, d, E, k, F, S) || (uintptr_t)workspace % 16) return RINA_ERR_WORKSPACE;
     hipStream_t st = as_stream(stream);
     const size_t t = (size_t)T, tk = t * k;
     float* a2 = (float*)workspace;
@@ -1637,7 +1671,8 @@ extern "C" int rina_hip_moe_rows(float* h, int T, const float* ln2, float eps, c
             return rc;
     }
     if (rows_gemm_ok(qt_exps, d) && rows_gemm_ok(qt_exps, F))
-        return moe_grouped(h, a2, ids, probs, gate_exps, up_exps, down_exps, qt_exps, stride_gu, stride_dn, T, E, k, d, F, st);
+        return moe_grouped(h, a2, ids, probs, gate_exps, up_exps, down_exps, qt_exps, stride_gu, stride_dn, T, E, k, d, F, (char*)X,
+                           ws_bytes - moe_rows_head(T, d, E, k, S), st);
     // the selection on the host: rows grouped by expert, ascending
     std::vector<int> hid(tk);
     std::vector<float> hpr(tk);

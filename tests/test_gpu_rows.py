@@ -416,3 +416,34 @@ def test_rows_product_norm_prologue(rina, orc, qt, M, K, pro):
         a = a - a.mean(1, keepdims=True)
     a = a / np.sqrt((a ** 2).mean(1, keepdims=True) + 1e-5) * nw
     assert_close(host(y).reshape(M, N), a @ W.reshape(N, K).T, what="norm + rows")
+
+
+@pytest.mark.parametrize("qt", [7, 10])
+def test_moe_rows_workspace_or_scratch(rina, orc, qt):
+    """A workspace that only holds the one-expert-at-a-time form (T k (2 d + F)
+    floats and the head) is taken as before, the grouped rows then in library
+    scratch: the same bits as with rina_hip_moe_rows_workspace() bytes, of which
+    nothing past the end is written; a little less is refused."""
+    hip, T, E, k, d, F = rina.load_hip(), 45, 8, 3, 128, 96
+    r = rng(qt)
+    w = [dev(weights(orc, qt, r, E * F * d)[0]) for _ in range(3)]
+    wr, ln2 = dev((r.standard_normal((E, d)) * 0.3).astype(np.float32)), dev(np.ones(d, np.float32))
+    h0 = r.standard_normal((T, d)).astype(np.float32)
+    sb = w[0].numel() * w[0].element_size() // E
+    up = lambda n: (n + 3) // 4 * 4
+    least = 4 * (up(T * d) + up(T * E) + 4 * up(T * k) + 2 * up(T * k * d) + up(T * k * F))
+    full = hip.rina_hip_moe_rows_workspace(T, d, E, k, F, 0)
+    assert full >= least
+
+    def call(nbytes):
+        ws, h = dev(np.full(nbytes + 4096, 0xA5, np.uint8)), dev(h0)
+        rc = hip.rina_hip_moe_rows(h.data_ptr(), T, ln2.data_ptr(), np.float32(1e-5), wr.data_ptr(), 6, None, None, None, 0, qt,
+                                   w[0].data_ptr(), w[1].data_ptr(), w[2].data_ptr(), qt, sb, sb, E, k, d, F, ws.data_ptr(),
+                                   nbytes, stream())
+        assert (host(ws)[nbytes:] == 0xA5).all()
+        return rc, host(h)
+
+    rc0, a = call(full)
+    rc1, b = call(least)
+    assert rc0 == rc1 == 0 and np.array_equal(a, b) and not np.array_equal(a.reshape(T, d), h0)
+    assert call(least - 4)[0] == -6          # RINA_ERR_WORKSPACE
