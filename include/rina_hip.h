@@ -188,8 +188,10 @@ int rina_hip_rope_append(float* q, float* k, const float* v,
  * Replaces the composition of gqa_layer.cu:192-270 (cache dequant,
  * build_qkv_fp32.cu:8-33, flash_fp32.cu:12-111, row extraction).
  * pre_rope: cached keys are rotated with rope_k tables on read
- * (gqa_layer.cu:236-238).  `workspace` holds split-sequence partials;
- * rina_hip_gqa_attention_workspace() gives its size. */
+ * (gqa_layer.cu:236-238).  A row's result holds no key or value past its
+ * position, also where those are inf or NaN.  `workspace` holds split-sequence
+ * partials of T == 1; rina_hip_gqa_attention_workspace() gives its size (T > 1:
+ * not used, partials in library scratch). */
 size_t rina_hip_gqa_attention_workspace(int T, int H, int dh, int max_pos);
 /* The position count up to which rina_hip_gqa_decode_attention over an fp32
  * cache with dh == 64 is one launch (1024; beyond it, or with a packed
