@@ -332,7 +332,9 @@ struct RelaxedCapture {
 static void* alloc_scratch(size_t bytes) {
     RelaxedCapture rc;
     void* p = nullptr;
-    return hipMalloc(&p, bytes) == hipSuccess ? p : nullptr;
+    if (hipMalloc(&p, bytes) == hipSuccess) return p;
+    (void)hipGetLastError();                       // reported by the caller, not by the next launch check
+    return nullptr;
 }
 
 // a graph is gone (called by the runtime: no HIP call, no lock that is held around one)
@@ -372,7 +374,11 @@ static void scratch_reap(ScratchState& g) {
         }
     }
     RelaxedCapture rc;
-    for (void* p : gone) (void)hipFree(p);
+    for (void* p : gone)
+        if (hipFree(p) != hipSuccess) {            // not now: the next call tries again
+            (void)hipGetLastError();
+            scratch_graph_done(p);
+        }
 }
 
 void* RinaScratch::get(size_t bytes, hipStream_t st, int use) {
