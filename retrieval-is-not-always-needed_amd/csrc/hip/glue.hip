@@ -250,7 +250,6 @@ struct DevState {
     int cus = 0;
 };
 DevState g_dev[64];
-std::mutex g_mu;
 
 // Library scratch: a buffer per (device, stream, use), and within a stream
 // capture a buffer of that capture: a graph may be replayed on any stream, also

@@ -18,7 +18,7 @@ pytestmark = pytest.mark.gpu
 # contexts stay below 700, where its own error is under the tolerance
 @pytest.mark.parametrize("mode", [0, 1, 2, 3, 4, 5])
 @pytest.mark.parametrize("P,T,H,Hkv", [(1, 2, 32, 8), (63, 17, 8, 8), (64, 16, 8, 4), (65, 33, 6, 2), (600, 3, 4, 1),
-                                       (200, 65, 16, 8), (0, 70, 10, 5)])
+                                       (200, 65, 16, 8), (0, 70, 10, 5), (0, 12, 16, 8), (0, 13, 10, 5)])
 def test_rows_continue_a_cache(rina, orc, mode, P, T, H, Hkv):
     got, ref = attention_case(rina, orc, mode, P, T, H=H, Hkv=Hkv)
     assert_close_elem(got, ref, what="mode %d P %d T %d H %d/%d" % (mode, P, T, H, Hkv))
@@ -37,7 +37,8 @@ def test_rows_device_position(rina, orc, mode, P, T):
 
 
 @pytest.mark.parametrize("T,start,H,Hkv,da,db,mode", [(63, 1, 10, 5, 64, 32, 0), (2, 63, 10, 5, 64, 16, 5), (17, 400, 3, 3, 80, 34, 0), (5, 700, 6, 2, 64, 10, 5),
-                                                      (65, 63, 10, 5, 64, 64, 5), (33, 1, 8, 2, 48, 22, 0)])
+                                                      (65, 63, 10, 5, 64, 64, 5), (33, 1, 8, 2, 48, 22, 0),
+                                                      (2, 254, 10, 5, 64, 32, 5), (2, 255, 10, 5, 64, 32, 0)])
 def test_dq_rows_other_widths(rina, T, start, H, Hkv, da, db, mode):
     dq_rows_case(rina, T, start, H, Hkv, da, db, mode)
 

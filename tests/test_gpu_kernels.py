@@ -375,9 +375,8 @@ def test_attention_multi_row(rina, orc, mode, P, T):
                                      (129, 10, 5), (64, 8, 8)])
 def test_attention_prompt_from_zero(rina, orc, T, H, Hkv):
     """Prompt rows from position 0: several 64-position blocks, ragged row
-    groups, causal against the oracle.  H / Hkv a multiple of 4 takes the
-    matrix-core kernel (config 2's 512 x 32 / 8 among them), the others the
-    one-wave block kernel."""
+    groups, causal against the oracle (config 2's 512 x 32 / 8 among them),
+    with 4, 2 or 1 query heads per wave set of the row tiles."""
     got, ref = attention_case(rina, orc, 0, 0, T, H=H, Hkv=Hkv)
     assert_close_elem(got, ref, what="prompt T %d H %d/%d" % (T, H, Hkv))
 
